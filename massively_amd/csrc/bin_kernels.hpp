@@ -1,0 +1,592 @@
+// Binned gather and scatter for gfx950: random indices into a table far larger
+// than an XCD's 4 MiB L2.
+//
+// A direct random access moves a whole line for one element (48 G/s at 2^28
+// u32). Both binned forms begin with bin_tiles_kernel, which sorts every tile
+// of consecutive positions by table window in LDS; the order and the windows'
+// starts stay tile-local, so there is no scan or look-back over tiles, and
+// every later pass reads and writes runs of consecutive elements.
+//  * gather: gather_window_kernel walks the table window by window while it
+//    stays in one L2, and unbin_tiles_kernel undoes the sort through LDS with
+//    the 16-bit source positions the sort kept (2^28 u32: 0.63 + 2.07 + 0.47
+//    ms, from 5.58 directly; the L2s serve about 130 G random reads/s).
+//  * scatter: an L2 takes random 4-byte stores at about the same rate and lets
+//    them go as partial lines, so it ends in LDS instead. bin_leaves_kernel
+//    takes a window's runs from a group of tiles (a chunk of at most kBinChunk
+//    elements) and sorts them by leaf (64 KiB of the table), chunk-local;
+//    leaf_scatter_kernel collects a leaf in LDS and writes whole lines (2^28
+//    u32: 0.88 + 0.86 + 0.53 ms, from 6.10 with one look-back partition into
+//    256 windows and random stores from L2).
+// Each tile decides for itself: indices that stay near each other (sorted,
+// reversed, strided, clustered) are gathered or scattered directly in step 1,
+// and a chunk that would overflow (indices far from uniform) in step 2.
+#pragma once
+
+#include "device_common.hpp"
+
+namespace msv {
+
+constexpr int kBinBlock = 1024;
+constexpr uint32_t kBinMost = 512;           // most windows, and most leaves per window
+constexpr uint32_t kLeafBytes = 64u << 10;
+constexpr uint32_t kBinChunk = 16384;        // elements of a chunk, at most
+constexpr int kChunkIpt = kBinChunk / kBinBlock;
+constexpr uint32_t kNoPlace = 0xffffffffu;   // an element a scatter drops
+constexpr uint32_t kXcds = 8;
+
+// How a table is cut: leaf = index >> leaf_shift; window = leaf >> sub_shift.
+// A row of starts holds one entry per bin and the end, padded.
+struct BinPlan {
+  uint32_t leaf_shift, sub_shift;
+  uint32_t windows, subs;      // subs = 1 << sub_shift
+  uint32_t tile_row, chunk_row;
+  uint32_t tiles, group, groups;  // full tiles; tiles per chunk; chunks per window
+};
+
+// Exclusive scan of s_cnt[0, kBinMost) into s_start, by the first kBinMost
+// threads; s_start[kBinMost] is the total, *s_most (zero before) the largest.
+__device__ inline void bin_scan(const uint32_t* s_cnt, uint32_t* s_start, uint32_t* s_wsum,
+                                uint32_t* s_most = nullptr) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
+  uint32_t cnt = 0, incl = 0;
+  if (tid < kBinMost) {
+    cnt = s_cnt[tid];
+    incl = wave_inclusive_scan<uint32_t, OP_ADD>(cnt);
+    if (lane == 63) s_wsum[wid] = incl;
+    if (s_most) {
+      const uint32_t most = wave_reduce<uint32_t, OP_MAX>(cnt);
+      if (lane == 0) atomicMax(s_most, most);
+    }
+  }
+  __syncthreads();
+  if (tid < kBinMost) {
+    uint32_t off = 0;
+    for (uint32_t w = 0; w < wid; ++w) off += s_wsum[w];
+    s_start[tid] = off + incl - cnt;
+    if (tid == kBinMost - 1) s_start[kBinMost] = off + incl;
+  }
+  __syncthreads();
+}
+
+template <typename T>
+__device__ inline void store4(T* p, const T (&v)[4]) {
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<uint4*>(p) = make_uint4(bit_cast<uint32_t>(v[0]), bit_cast<uint32_t>(v[1]),
+                                              bit_cast<uint32_t>(v[2]), bit_cast<uint32_t>(v[3]));
+  } else {
+    reinterpret_cast<ulonglong2*>(p)[0] = make_ulonglong2(bit_cast<uint64_t>(v[0]), bit_cast<uint64_t>(v[1]));
+    reinterpret_cast<ulonglong2*>(p)[1] = make_ulonglong2(bit_cast<uint64_t>(v[2]), bit_cast<uint64_t>(v[3]));
+  }
+}
+
+// Copies cnt elements of LDS (16-byte aligned) to global memory (16-byte
+// aligned) as 16-byte stores; the last store may write past cnt (the
+// destination is padded).
+template <typename E>
+__device__ inline void copy_out16(const E* s, E* g, uint32_t cnt) {
+  constexpr uint32_t V = 16 / sizeof(E);
+  for (uint32_t i = threadIdx.x * V; i < cnt; i += kBinBlock * V)
+    *reinterpret_cast<uint4*>(g + i) = *reinterpret_cast<const uint4*>(s + i);
+}
+
+// How many of the first `count` indices of every thread lie outside the table
+// window of their wave's first one, summed over the block (all threads call).
+template <int COUNT, int N>
+__device__ inline uint32_t count_far(const uint32_t (&ix)[N], uint32_t shift, uint32_t* s_far) {
+  const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ix[0] >> shift));
+  uint32_t far = 0;
+#pragma unroll
+  for (int j = 0; j < COUNT; ++j) far += (uint32_t)__builtin_popcountll(ballot((ix[j] >> shift) != w0));
+  if ((threadIdx.x & 63u) == 0) atomicAdd(s_far, far);
+  __syncthreads();
+  return *s_far;
+}
+
+// Gather, step 1: one block to kNearTile positions. When at least half of its
+// first quarter's indices leave their wave's first window, the block is put
+// off (far[block] = 1); else it gathers directly. Blocks from `full` on
+// (a partial tile of the next step) always gather directly. A look at the
+// first quarter keeps the indices from being read twice, and small blocks keep
+// the direct gather as fast as without the look (step 2's big tiles took
+// 0.61 against 0.55 ms for 2^28 reversed indices).
+constexpr int kNearBlock = 256;
+constexpr uint32_t kNearTile = 4096;
+
+template <typename T>
+__global__ __launch_bounds__(kNearBlock) void gather_near_kernel(
+    const T* __restrict__ table, uint32_t tlen, const uint32_t* __restrict__ idx,
+    T* __restrict__ out, uint32_t n, uint32_t shift, uint32_t full, bool aligned,
+    uint8_t* __restrict__ far) {
+  constexpr int ROWS = (int)(kNearTile / kNearBlock / 4);
+  __shared__ uint32_t s_far;
+  const uint32_t tid = threadIdx.x;
+  const size_t base = (size_t)blockIdx.x * kNearTile;
+  const bool whole = base + kNearTile <= n;
+  uint32_t ix[ROWS * 4];
+  auto load_row = [&](int r) {
+    const size_t i = base + ((size_t)r * kNearBlock + tid) * 4;
+    uint32_t x[4];
+    load4<uint32_t>(idx, i, n, whole && aligned, x);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ix[4 * r + k] = whole || i + k < n ? x[k] : 0xffffffffu;
+  };
+  load_row(0);
+  if (blockIdx.x < full) {
+    if (tid == 0) s_far = 0;
+    __syncthreads();
+    const bool put_off = count_far<4>(ix, shift, &s_far) * 2 >= kNearBlock * 4;
+    if (tid == 0) far[blockIdx.x] = put_off ? 1 : 0;
+    if (put_off) return;
+  }
+#pragma unroll
+  for (int r = 1; r < ROWS; ++r) load_row(r);
+  T v[ROWS][4];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[r][k] = ix[4 * r + k] < tlen ? table[ix[4 * r + k]] : (T)0;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const size_t o = base + ((size_t)r * kNearBlock + tid) * 4;
+    if (whole && aligned) {
+      store4(out + o, v[r]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (o + k < n) out[o + k] = v[r][k];
+    }
+  }
+}
+
+// The sort of one tile by window. table: the gather's values or the scatter's
+// output, of tlen elements; io: the gather's output or the scatter's values,
+// by position. pidx: the tile's indices in window order; ppos (gather): their
+// in-tile positions; pval (scatter): their values. A row of zeros in `starts`:
+// the tile was done directly. The gather takes the tiles that
+// gather_near_kernel put off (`far`, a byte to kNearTile positions), the
+// scatter every tile (the last, partial one directly). A block that binned a
+// tile says so in the launch's status word, for the later steps (looking at it
+// first: 65536 stores to one word took 2.3 ms).
+template <typename T, int IPT, bool SCATTER>
+__global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 8 : 4) void bin_tiles_kernel(
+    T* __restrict__ table, uint32_t tlen, const uint32_t* __restrict__ idx, T* __restrict__ io,
+    uint32_t n, BinPlan p, bool aligned, const uint8_t* __restrict__ far,
+    uint32_t* __restrict__ pidx, uint16_t* __restrict__ ppos, T* __restrict__ pval,
+    uint16_t* __restrict__ starts, uint64_t* __restrict__ status, uint32_t gen) {
+  constexpr uint32_t TILE = (uint32_t)kBinBlock * IPT;
+  constexpr int ROWS = IPT / 4;
+  constexpr uint32_t W = SCATTER ? sizeof(T) : 4;
+  static_assert(TILE <= 32768 && IPT % 8 == 0 && kBinBlock * 4 == kNearTile, "tile");
+  __shared__ __align__(16) unsigned char s_mem[TILE * W];
+  __shared__ uint32_t s_cnt[kBinMost], s_start[kBinMost + 1];
+  __shared__ uint32_t s_far, s_out, s_most, s_wsum[kBinMost / kWave];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t shift = p.leaf_shift + p.sub_shift;
+  uint32_t tile = blockIdx.x;
+  if constexpr (!SCATTER) {
+    // All of the block's tiles at once, so that a launch without work ends at once.
+    const uint32_t mine = (p.tiles - tile + gridDim.x - 1) / gridDim.x;
+    bool any = false;
+    for (uint32_t i = tid; i < mine * ROWS; i += kBinBlock)
+      any = any || far[(size_t)(tile + i / ROWS * gridDim.x) * ROWS + i % ROWS];
+    if (!__syncthreads_or(any)) {
+      for (; tile < p.tiles; tile += gridDim.x)
+        if (tid <= p.windows) starts[(size_t)tile * p.tile_row + tid] = 0;
+      return;
+    }
+  }
+  do {
+    const size_t base = (size_t)tile * TILE;
+    const bool full = base + TILE <= n;
+    uint16_t* row = starts + (size_t)tile * p.tile_row;
+    // The rows (of kNearTile positions) to do here.
+    uint32_t rows = 0;
+    if constexpr (!SCATTER) {
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) rows |= (far[(size_t)tile * ROWS + r] ? 1u : 0u) << r;
+    }
+    bool spread = SCATTER ? full : rows == (1u << ROWS) - 1;
+    __syncthreads();
+    if (tid < kBinMost) s_cnt[tid] = 0;
+    if (tid == 0) s_far = s_out = s_most = 0;
+    __syncthreads();
+
+    // Element 4 r + k of a thread is position (r * kBinBlock + tid) * 4 + k.
+    uint32_t ix[IPT];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const size_t i = base + ((size_t)r * kBinBlock + tid) * 4;
+      if (full && aligned) {
+        const uint4 q = load16_nt(idx + i);
+        ix[4 * r] = q.x; ix[4 * r + 1] = q.y; ix[4 * r + 2] = q.z; ix[4 * r + 3] = q.w;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) ix[4 * r + k] = i + k < n ? idx[i + k] : 0xffffffffu;
+      }
+    }
+    if constexpr (SCATTER) {
+      // Counted in registers first: the counts below would serialise on one
+      // LDS word for a tile that stays in a window or two.
+      spread = spread && count_far<IPT>(ix, shift, &s_far) * 2 >= TILE;
+    } else {
+      bool out = false;
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) out = out || ix[j] >= tlen;
+      if (ballot(out)) s_out = 1;
+      __syncthreads();
+      spread = spread && s_out == 0;
+    }
+    uint32_t at[IPT];
+    if (spread) {
+      // A scatter drops an index past the table; a gather reads 0 there, and
+      // its tile is done directly.
+#pragma unroll
+      for (int j = 0; j < IPT; ++j)
+        at[j] = !SCATTER || ix[j] < tlen ? atomicAdd(&s_cnt[ix[j] >> shift], 1u) : kNoPlace;
+      __syncthreads();
+      bin_scan(s_cnt, s_start, s_wsum, &s_most);
+      spread = s_most * p.windows <= 4 * TILE;
+    }
+    if (!spread) {
+      if (full && tid <= p.windows) row[tid] = 0;
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const size_t o = base + ((size_t)r * kBinBlock + tid) * 4;
+        T x[4];
+        if constexpr (SCATTER) {
+          load4<T, true>(io, o, n, full && aligned, x);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (ix[4 * r + k] < tlen) table[ix[4 * r + k]] = x[k];
+        } else if (rows >> r & 1u) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) x[k] = ix[4 * r + k] < tlen ? table[ix[4 * r + k]] : (T)0;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) io[o + k] = x[k];
+        }
+      }
+      if (SCATTER) return;
+      continue;
+    }
+
+    // Recompute the windows below instead of keeping them in registers.
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) asm volatile("" : "+v"(ix[j]));
+    const uint32_t total = s_start[kBinMost];
+    if (tid == 0 && status_flag(ld_agent(status), gen) == 0)
+      st_agent(status, pack_status(gen, kFlagInc, 0, 0));
+    if (tid < p.windows) row[tid] = (uint16_t)s_start[tid];
+    if (tid == kBinMost) row[p.windows] = (uint16_t)total;
+    uint32_t* s_idx = reinterpret_cast<uint32_t*>(s_mem);
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      if (!SCATTER || at[j] != kNoPlace) {
+        at[j] += s_start[ix[j] >> shift];
+        s_idx[at[j]] = ix[j];
+      }
+    }
+    __syncthreads();
+    copy_out16(s_idx, pidx + base, total);
+    __syncthreads();
+    if constexpr (SCATTER) {
+      T* s_val = reinterpret_cast<T*>(s_mem);
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        T x[4];
+        load4<T, true>(io, base + ((size_t)r * kBinBlock + tid) * 4, n, aligned, x);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (at[4 * r + k] != kNoPlace) s_val[at[4 * r + k]] = x[k];
+      }
+      __syncthreads();
+      copy_out16(s_val, pval + base, total);
+    } else {
+      uint16_t* s_pos = reinterpret_cast<uint16_t*>(s_mem);
+#pragma unroll
+      for (int j = 0; j < IPT; ++j)
+        s_pos[at[j]] = (uint16_t)(((uint32_t)(j / 4) * kBinBlock + tid) * 4 + (j & 3));
+      __syncthreads();
+      copy_out16(s_pos, ppos + base, total);
+    }
+  } while (!SCATTER && (tile += gridDim.x) < p.tiles);
+}
+
+// Gather, step 2: replaces the indices of the binned tiles by their values,
+// window by window (pval may be pidx). Block b works on the windows w with
+// w % 8 == b % 8, which the round-robin of workgroups keeps on one XCD, in
+// order, so one or two windows are live in each L2. A group of 16 lanes reads
+// the run of one tile, U elements a lane in flight. One block of four waves a
+// CU and 2 MiB windows: 2.07 ms at 2^28 u32 (130 G reads/s); two blocks
+// 2.35, eight 4.0 (more windows at once than an L2 holds), 4 MiB windows 2.5.
+template <typename T, uint32_t TILE, int U>
+__global__ __launch_bounds__(256) void gather_window_kernel(
+    const T* __restrict__ table, uint32_t tlen, BinPlan p, const uint32_t* pidx, T* pval,
+    const uint16_t* __restrict__ starts, const uint64_t* __restrict__ status, uint32_t gen) {
+  if (status_flag(ld_agent(status), gen) == 0) return;
+  constexpr uint32_t kTilesPerWave = 16, kTilesPerBlock = 4 * kTilesPerWave;
+  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t g = blockIdx.x % kXcds;
+  const uint32_t mine = p.windows > g ? (p.windows - g + kXcds - 1) / kXcds : 0u;
+  const uint32_t chunks = (p.tiles + kTilesPerBlock - 1) / kTilesPerBlock;
+  for (uint32_t q = blockIdx.x / kXcds; q < mine * chunks; q += gridDim.x / kXcds) {
+    const uint32_t w = g + kXcds * (q / chunks);
+    const uint32_t t0 = (q % chunks) * kTilesPerBlock + wid * kTilesPerWave;
+    uint32_t s = 0, e = 0;
+    if (lane < kTilesPerWave && t0 + lane < p.tiles) {
+      const uint16_t* row = starts + (size_t)(t0 + lane) * p.tile_row + w;
+      s = row[0];
+      e = row[1];
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kTilesPerWave / 4; ++r) {
+      const uint32_t t = r * 4 + (lane >> 4);
+      const uint32_t len = (uint32_t)__shfl((int)(e - s), (int)t);
+      const size_t at = (size_t)(t0 + t) * TILE + (uint32_t)__shfl((int)s, (int)t);
+      for (uint32_t k0 = lane & 15u; k0 < len; k0 += 16 * U) {
+        uint32_t ix[U];
+        T v[U];
+        // The runs are read and written once: non-temporal, so the window stays.
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+          ix[k] = k0 + 16 * k < len ? __builtin_nontemporal_load(pidx + at + k0 + 16 * k) : tlen;
+#pragma unroll
+        for (int k = 0; k < U; ++k) v[k] = ix[k] < tlen ? table[ix[k]] : (T)0;
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+          if (k0 + 16 * k < len) __builtin_nontemporal_store(v[k], pval + at + k0 + 16 * k);
+      }
+    }
+  }
+}
+
+// Copies runs of E (s_src: their first elements, s_off: their places) to LDS,
+// 32 lanes a run, four loads of a lane in flight.
+template <typename E>
+__device__ inline void load_runs(const E* __restrict__ from, const uint32_t* s_src,
+                                 const uint32_t* s_off, uint32_t runs, E* s_to) {
+  constexpr int U = 4;
+  for (uint32_t r = threadIdx.x / 32; r < runs; r += kBinBlock / 32) {
+    const uint32_t o = s_off[r], len = s_off[r + 1] - o;
+    const E* src = from + s_src[r];
+    for (uint32_t k0 = threadIdx.x & 31u; k0 < len; k0 += 32 * U) {
+      E d[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k0 + 32 * k < len) d[k] = src[k0 + 32 * k];
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (k0 + 32 * k < len) s_to[o + k0 + 32 * k] = d[k];
+    }
+  }
+}
+
+// Scatter, step 2: one chunk a block at a time. cidx: the elements' places in
+// their leaf, in leaf order; cval: their values. A chunk that does not fit is
+// scattered directly and leaves a row of zeros. Concurrent blocks take the
+// windows of one group of tiles, so the runs they read are neighbours (a
+// window at a time over all tiles was 8% slower: 1 KiB pieces of 1 GiB).
+// 64 registers and 64 KiB of LDS: two blocks a CU (1.12 -> 0.86 ms at 2^28 u32).
+template <typename T, uint32_t TILE>
+__global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_kernel(
+    T* __restrict__ table, BinPlan p, const uint32_t* __restrict__ pidx,
+    const T* __restrict__ pval, const uint16_t* __restrict__ starts, uint16_t* __restrict__ cidx,
+    T* __restrict__ cval, uint16_t* __restrict__ rows, const uint64_t* __restrict__ status,
+    uint32_t gen) {
+  if (status_flag(ld_agent(status), gen) == 0) return;
+  __shared__ __align__(16) T s_val[kBinChunk];
+  __shared__ uint32_t s_cnt[kBinMost], s_off[kBinMost + 1], s_src[kBinMost];
+  __shared__ uint32_t s_wsum[kBinMost / kWave];
+  const uint32_t tid = threadIdx.x, lane = tid & 31u, grp = tid >> 5;
+  uint32_t* s_idx = reinterpret_cast<uint32_t*>(s_val);
+  uint16_t* s_16 = reinterpret_cast<uint16_t*>(s_val);
+  for (uint32_t q = blockIdx.x; q < p.windows * p.groups; q += gridDim.x) {
+    const uint32_t w = q % p.windows, g = q / p.windows, c = w * p.groups + g;
+    // The window's runs in the group's tiles: where each begins, and its place
+    // in the chunk.
+    const uint32_t t0 = g * p.group, runs = min(p.group, p.tiles - t0);
+    if (tid < kBinMost) {
+      uint32_t s = 0, e = 0;
+      if (tid < runs) {
+        const uint16_t* r = starts + (size_t)(t0 + tid) * p.tile_row + w;
+        s = r[0];
+        e = r[1];
+        s_src[tid] = (t0 + tid) * TILE + s;
+      }
+      s_cnt[tid] = e - s;
+    }
+    __syncthreads();
+    bin_scan(s_cnt, s_off, s_wsum);
+    const uint32_t cnt = s_off[kBinMost];
+    uint16_t* row = rows + (size_t)c * p.chunk_row;
+    if (cnt > kBinChunk) {
+      if (tid <= p.subs) row[tid] = 0;
+      for (uint32_t r = grp; r < runs; r += kBinBlock / 32)
+        for (uint32_t k = lane; k < s_off[r + 1] - s_off[r]; k += 32)
+          table[pidx[s_src[r] + k]] = pval[s_src[r] + k];
+      __syncthreads();
+      continue;
+    }
+    load_runs(pidx, s_src, s_off, runs, s_idx);
+    if (tid < kBinMost) s_cnt[tid] = 0;
+    __syncthreads();
+    uint32_t ix[kChunkIpt], at[kChunkIpt];
+#pragma unroll
+    for (int j = 0; j < kChunkIpt; ++j) {
+      const uint32_t i = tid + (uint32_t)j * kBinBlock;
+      ix[j] = s_idx[i];
+      at[j] = i < cnt ? atomicAdd(&s_cnt[(ix[j] >> p.leaf_shift) & (p.subs - 1)], 1u) : kNoPlace;
+    }
+    // Recompute the leaf numbers below instead of keeping them in registers.
+#pragma unroll
+    for (int j = 0; j < kChunkIpt; ++j) asm volatile("" : "+v"(ix[j]));
+    __syncthreads();
+    // The leaves' starts (over their counts: s_off still holds the runs' places).
+    uint32_t n_leaf = 0, incl = 0;
+    if (tid < kBinMost) {
+      n_leaf = s_cnt[tid];
+      incl = wave_inclusive_scan<uint32_t, OP_ADD>(n_leaf);
+      if ((tid & 63u) == 63u) s_wsum[tid >> 6] = incl;
+    }
+    __syncthreads();
+    if (tid < kBinMost) {
+      uint32_t start = incl - n_leaf;
+      for (uint32_t v = 0; v < (tid >> 6); ++v) start += s_wsum[v];
+      s_cnt[tid] = start;
+      if (tid < p.subs) row[tid] = (uint16_t)start;
+    }
+    if (tid == kBinMost) row[p.subs] = (uint16_t)cnt;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kChunkIpt; ++j) {
+      if (at[j] != kNoPlace) {
+        at[j] += s_cnt[(ix[j] >> p.leaf_shift) & (p.subs - 1)];
+        s_16[at[j]] = (uint16_t)(ix[j] & ((1u << p.leaf_shift) - 1));
+      }
+    }
+    __syncthreads();
+    copy_out16(s_16, cidx + (size_t)c * kBinChunk, cnt);
+    __syncthreads();
+    // The values the same way: runs into LDS, then from chunk to leaf order.
+    load_runs(pval, s_src, s_off, runs, s_val);
+    __syncthreads();
+    T v[kChunkIpt];
+#pragma unroll
+    for (int j = 0; j < kChunkIpt; ++j) v[j] = s_val[tid + (uint32_t)j * kBinBlock];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kChunkIpt; ++j)
+      if (at[j] != kNoPlace) s_val[at[j]] = v[j];
+    __syncthreads();
+    copy_out16(s_val, cval + (size_t)c * kBinChunk, cnt);
+    __syncthreads();
+  }
+}
+
+// Scatter, step 3: one leaf a block at a time. The leaf's elements meet in LDS and leave as whole lines;
+// a bitmap keeps what no index names unwritten.
+template <typename T>
+__global__ __launch_bounds__(kBinBlock) void leaf_scatter_kernel(
+    T* __restrict__ table, uint32_t tlen, BinPlan p, bool aligned,
+    const uint16_t* __restrict__ cidx, const T* __restrict__ cval,
+    const uint16_t* __restrict__ rows, const uint64_t* __restrict__ status, uint32_t gen) {
+  if (status_flag(ld_agent(status), gen) == 0) return;
+  constexpr uint32_t LEAF = kLeafBytes / sizeof(T);
+  constexpr int U = 4;
+  __shared__ __align__(16) T s_leaf[LEAF];
+  __shared__ uint32_t s_set[LEAF / 32];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
+  const uint32_t leaves = (tlen + LEAF - 1) / LEAF;
+  for (uint32_t leaf = blockIdx.x; leaf < leaves; leaf += gridDim.x) {
+    const uint32_t w = leaf >> p.sub_shift, sub = leaf & (p.subs - 1);
+    const size_t l0 = (size_t)leaf * LEAF;
+    for (uint32_t i = tid; i < LEAF / 32; i += kBinBlock) s_set[i] = 0;
+    __syncthreads();
+    for (uint32_t g0 = wid; g0 < p.groups; g0 += 16 * kWave) {
+      uint32_t s = 0, e = 0;
+      const uint32_t mine = g0 + 16 * lane;
+      if (mine < p.groups) {
+        const uint16_t* row = rows + ((size_t)w * p.groups + mine) * p.chunk_row + sub;
+        s = row[0];
+        e = row[1];
+      }
+      const uint32_t many = min((uint32_t)kWave, (p.groups - g0 + 15) / 16);
+      for (uint32_t k = 0; k < many; ++k) {
+        const uint32_t a = readlane(s, (int)k), b = readlane(e, (int)k);
+        const size_t c = ((size_t)w * p.groups + g0 + 16 * k) * kBinChunk;
+        for (uint32_t i0 = a + lane; i0 < b; i0 += kWave * U) {
+          uint32_t d[U];
+          T v[U];
+#pragma unroll
+          for (int q = 0; q < U; ++q)
+            if (i0 + kWave * q < b) {
+              d[q] = cidx[c + i0 + kWave * q];
+              v[q] = cval[c + i0 + kWave * q];
+            }
+#pragma unroll
+          for (int q = 0; q < U; ++q)
+            if (i0 + kWave * q < b) {
+              s_leaf[d[q]] = v[q];
+              atomicOr(&s_set[d[q] >> 5], 1u << (d[q] & 31u));
+            }
+        }
+      }
+    }
+    __syncthreads();
+    for (uint32_t i = tid * 4; i < LEAF; i += kBinBlock * 4) {
+      const uint32_t m = (s_set[i >> 5] >> (i & 31u)) & 15u;
+      if (m == 15u && aligned) {
+        const T x[4] = {s_leaf[i], s_leaf[i + 1], s_leaf[i + 2], s_leaf[i + 3]};
+        store4(table + l0 + i, x);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (m >> k & 1u) table[l0 + i + k] = s_leaf[i + k];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Gather, step 3: a tile's values from window order back to positions.
+template <typename T, int IPT>
+__global__ __launch_bounds__(kBinBlock, IPT * sizeof(T) == 64 ? 8 : 4) void unbin_tiles_kernel(
+    BinPlan p, const T* __restrict__ pval, const uint16_t* __restrict__ ppos,
+    const uint16_t* __restrict__ starts, T* __restrict__ out, bool aligned,
+    const uint64_t* __restrict__ status, uint32_t gen) {
+  if (status_flag(ld_agent(status), gen) == 0) return;
+  constexpr uint32_t TILE = (uint32_t)kBinBlock * IPT;
+  constexpr int V = 16 / sizeof(T);
+  __shared__ __align__(16) T s_val[TILE];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t tile = blockIdx.x; tile < p.tiles; tile += gridDim.x) {
+    if (starts[(size_t)tile * p.tile_row + p.windows] == 0) continue;
+    const size_t base = (size_t)tile * TILE;
+#pragma unroll
+    for (int r = 0; r < IPT / 8; ++r) {
+      const uint32_t i = ((uint32_t)r * kBinBlock + tid) * 8;
+      const uint4 q = load16_nt(ppos + base + i);
+      const uint32_t pw[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int h = 0; h < 8; h += 4) {
+        T x[4];
+        load4<T, true>(pval + base, i + h, 0, true, x);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s_val[(pw[(h + k) / 2] >> (16 * (k & 1))) & 0xffffu] = x[k];
+      }
+    }
+    __syncthreads();
+    if (aligned) {
+#pragma unroll
+      for (int r = 0; r < IPT / V; ++r) {
+        const uint32_t i = ((uint32_t)r * kBinBlock + tid) * V;
+        *reinterpret_cast<uint4*>(out + base + i) = *reinterpret_cast<const uint4*>(s_val + i);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < IPT; ++r) out[base + (uint32_t)r * kBinBlock + tid] = s_val[r * kBinBlock + tid];
+    }
+    __syncthreads();
+  }
+}
+
+}  // namespace msv

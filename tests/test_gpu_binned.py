@@ -1,0 +1,104 @@
+"""GPU: the binned forms of scatter and gather (large tables), bit-exact vs
+numpy indexing: ragged lengths, unaligned slices, tiles that go the direct way
+beside binned ones, chunks that overflow, dropped and out-of-range indices."""
+import numpy as np
+import pytest
+
+import massively_amd as m
+
+pytestmark = pytest.mark.gpu
+
+N = 1 << 23  # the smallest binned scatter
+
+
+def _order(kind, n, size, rng):
+    """n distinct indices below size in the given order."""
+    if kind == "random":
+        return rng.permutation(size)[:n].astype(np.uint32)
+    if kind == "half":  # twice the mean in half of the windows
+        return rng.permutation(size // 2)[:n].astype(np.uint32)
+    if kind == "reversed":
+        return np.arange(size - 1, size - 1 - n, -1, dtype=np.uint32)
+    idx = rng.permutation(size)[:n].astype(np.uint32)  # "mixed": sorted and random stretches
+    for lo in range(0, n, 100_000):
+        if (lo // 100_000) % 2:
+            idx[lo:lo + 100_000] = np.sort(idx[lo:lo + 100_000])
+    return idx
+
+
+@pytest.mark.parametrize("dtype,kind,n,size,offset", [
+    (np.uint32, "random", N, N, 0),
+    (np.uint32, "random", N + 12345, 2 * N + 7, 1),
+    (np.uint32, "half", N, 2 * N + 4, 0),
+    (np.uint32, "mixed", N + 1, N + 16385, 3),
+    (np.uint32, "reversed", N + 16383, 3 * N, 0),
+    (np.uint32, "random", 4 * N - 1, 4 * N, 0),
+    (np.uint64, "random", N + 4095, N + 8193, 0),
+    (np.uint64, "half", N, 2 * N, 1),
+    (np.uint64, "mixed", 2 * N + 3, 2 * N + 5, 0),
+])
+def test_binned_scatter(exec_, dtype, kind, n, size, offset):
+    rng = np.random.default_rng(n + size)
+    idx = _order(kind, n, size, rng)
+    idx[rng.integers(0, n, 1000)] = size + rng.integers(0, 2**20, 1000).astype(np.uint32)  # dropped
+    v = rng.integers(0, 2**32, n).astype(dtype)
+    before = rng.integers(0, 2**32, size).astype(dtype)
+    pad = np.zeros(offset, dtype)
+    di = exec_.to_device(np.concatenate([pad.astype(np.uint32), idx])).slice(offset, offset + n)
+    dv = exec_.to_device(np.concatenate([pad, v])).slice(offset, offset + n)
+    whole = exec_.to_device(np.concatenate([pad, before, pad]))
+    m.vector.scatter(exec_, dv, di, whole.slice(offset, offset + size))
+    kept = idx < size
+    before[idx[kept]] = v[kept]
+    assert np.array_equal(exec_.to_host(whole), np.concatenate([pad, before, pad]))
+
+
+def test_binned_scatter_duplicates(exec_):
+    """One of the values aimed at a place ends up there."""
+    rng = np.random.default_rng(3)
+    idx = rng.integers(0, N, N).astype(np.uint32)
+    out = exec_.to_device(np.full(N, 0xFFFFFFFF, np.uint32))
+    m.vector.scatter(exec_, exec_.to_device(np.arange(N, dtype=np.uint32)), exec_.to_device(idx), out)
+    got = exec_.to_host(out)
+    hit = np.zeros(N, bool)
+    hit[idx] = True
+    assert np.array_equal(got != 0xFFFFFFFF, hit)
+    assert np.array_equal(idx[got[hit]], np.flatnonzero(hit))
+
+
+def test_binned_scatter_replays(exec_):
+    rng = np.random.default_rng(5)
+    v = exec_.to_device(np.arange(N, dtype=np.uint32))
+    idx, out = exec_.to_device(rng.permutation(N).astype(np.uint32)), exec_.alloc(np.uint32, N)
+    with exec_.capture() as cap:
+        m.vector.scatter(exec_, v, idx, out)
+    for _ in range(3):
+        p = rng.permutation(N).astype(np.uint32)
+        m.vector.scatter(exec_, exec_.to_device(p), v, idx)  # idx <- p (v is the identity)
+        m.vector.scatter(exec_, exec_.to_device(np.zeros(N, np.uint32)), v, out)
+        exec_.sync()
+        cap.graph.launch()
+        exec_.sync()
+        got = exec_.to_host(out)
+        assert np.array_equal(got[p], np.arange(N, dtype=np.uint32))
+
+
+@pytest.mark.parametrize("kind,offset,outside", [("random", 0, 0), ("mixed", 1, 500)])
+def test_binned_gather(exec_, kind, offset, outside):
+    n, size = (1 << 27) + 40_000, (1 << 27) - 7
+    rng = np.random.default_rng(offset)
+    idx = np.empty(n + offset, np.uint32)
+    step = 1 << 24
+    for lo in range(0, n + offset, step):  # (a permutation of 2^27 costs the test 10 s)
+        k = min(step, n + offset - lo)
+        idx[lo:lo + k] = rng.integers(0, size, k, dtype=np.uint32)
+    if kind == "mixed":
+        for lo in range(0, n - 50_000, 1 << 20):
+            idx[lo:lo + 50_000] = np.arange(lo % size, lo % size + 50_000) % size
+        idx[rng.integers(0, n, outside)] = size + 3
+    v = rng.integers(0, 2**32, size, dtype=np.uint32)
+    di = exec_.to_device(idx).slice(offset, offset + n)
+    got = exec_.to_host(m.vector.gather(exec_, exec_.to_device(v), di))
+    j = idx[offset:]
+    inside = j < size
+    assert np.array_equal(got, np.where(inside, v[np.where(inside, j, 0)], 0))
