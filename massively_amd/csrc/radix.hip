@@ -24,12 +24,10 @@
 //    earlier tiles (4 status words per step); elements of 12 or 16 bytes go
 //    through LDS as keys and then values, and stay in separate key and value
 //    arrays between passes; every pass runs 1024-thread tiles at 8 waves
-//    per SIMD (2^27 u64 keys + u32 values: uniform 10.28 ms, Zipf 1.1
-//    10.10 ms, constant top byte 9.01 ms);
-//  * reduce-then-scan (11.86 / 10.84 / 10.43 ms there, 8.22 ms against 7.80
-//    for 2^28 u32 + u32; kept behind the option): pass 0's upsweep also records per
-//    tile the OR and AND of the order words (the skip test), and per digit an
-//    upsweep counts the digits of every tile into a digit-major matrix, the
+//    per SIMD (2^28 u32 + u32: 5.63 ms, 2^27 u64 + u32: 7.22 ms);
+//  * reduce-then-scan (8.22 and 11.86 ms there; kept behind the option): pass
+//    0's upsweep also records per tile the OR and AND of the order words (the
+//    skip test), and per digit an upsweep counts the digits of every tile into a digit-major matrix, the
 //    library's scan turns it into run starts, and a downsweep ranks and writes;
 //    no tile waits on another.
 // MSV_OPT_RADIX_ONESWEEP selects either.
@@ -48,21 +46,18 @@ template <int EW>
 constexpr int radix_block() { return 512; }
 template <int EW>
 constexpr int radix_ipt() { return EW <= 2 ? 16 : 8; }
-// Onesweep passes run 1024-thread blocks: 1024 x 8 for 4-byte elements,
-// 1024 x 6 for 8-byte and 1024 x 5 for 12- and 16-byte elements. Each shape
-// fits two blocks' LDS per CU (52-68 KB each) at 54-63 VGPRs, so 8 waves per
-// SIMD, where the 512-thread tiles (512 x 16, and 512 x 8 at 78 VGPRs for 12
-// bytes) held 4-6. Measured against those: 2^28 u32 keys 6.53 -> 5.58 ms,
-// 2^28 u32 + u32 7.80 -> 7.35 ms, 2^27 u64 keys 7.61 -> 6.96 ms, 2^27 u64 +
-// u32 10.18 -> 9.33 ms, 2^27 u64 + u64 12.46 -> 10.53 ms. Slower: any shape
-// above 64 VGPRs (one block per CU: 1024 x 10 or 12 for 4-byte, 1024 x 7 for
-// 8-byte elements), smaller tiles at the same occupancy (1024 x 4 for 8-byte
-// elements: 9.05 ms for u32 + u32; 1024 x 4 for 12-byte: 10.18 ms), and
-// 512 x 4 / 512 x 6 for 12-byte elements.
+// Onesweep passes run 1024-thread blocks, two per CU at 64 VGPRs (8 waves per
+// SIMD): 10 keys per thread for 4-byte elements, 8 for wider ones, the most
+// that fit those registers and LDS (63-78 KB a block). From 8, 6, 5 and 5 keys
+// (radix_onesweep_kernel says how they fit): 2^28 u32 keys 5.58 -> 4.27 ms,
+// 2^28 u32 + u32 7.31 -> 5.62, 2^27 u64 keys 6.96 -> 5.32, u64 + u32 9.35 ->
+// 7.22, u64 + u64 10.53 -> 9.22. Slower: shapes that spill (12 or 14 for
+// 4-byte elements: 4.47, 4.67 ms; 16: 51 ms) and shapes of one block per CU
+// (9 for u64 + u32: 8.2 ms).
 template <int EW>
 constexpr int radix_onesweep_block() { return 1024; }
 template <int EW>
-constexpr int radix_onesweep_ipt() { return EW >= 3 ? 5 : (EW == 2 ? 6 : 8); }
+constexpr int radix_onesweep_ipt() { return EW == 1 ? 10 : 8; }
 
 template <typename K, int MODE, int VS>
 static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, uint32_t n,

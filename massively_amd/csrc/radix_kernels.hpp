@@ -233,38 +233,6 @@ __device__ inline void store_elem(const RadixPass& rp, size_t i, const Elem<EW>&
   for (int v = 0; v < EW - KW; ++v) ((uint32_t*)rp.dst_v)[i * (EW - KW) + v] = e.w[KW + v];
 }
 
-// The key or the value part of element i of the pass's destination.
-template <typename K, int EW>
-__device__ inline void store_key_part(const RadixPass& rp, size_t i, K k) {
-  if (rp.out_aos) {
-    uint32_t* w = ((Elem<EW>*)rp.dst_k)[i].w;
-    if constexpr (sizeof(K) == 4) {
-      w[0] = bit_cast<uint32_t>(k);
-    } else {
-      const uint64_t u = bit_cast<uint64_t>(k);
-      w[0] = (uint32_t)u;
-      w[1] = (uint32_t)(u >> 32);
-    }
-    return;
-  }
-  ((K*)rp.dst_k)[i] = k;
-}
-template <typename K, int EW, typename V>
-__device__ inline void store_val_part(const RadixPass& rp, size_t i, V v) {
-  constexpr int KW = sizeof(K) / 4;
-  if (rp.out_aos) {
-    uint32_t* w = ((Elem<EW>*)rp.dst_k)[i].w;
-    if constexpr (sizeof(V) == 4) {
-      w[KW] = v;
-    } else {
-      w[KW] = (uint32_t)v;
-      w[KW + 1] = (uint32_t)(v >> 32);
-    }
-    return;
-  }
-  ((V*)rp.dst_v)[i] = v;
-}
-
 // 3. Per-pass reduce-then-scan over tiles of BLOCK * IPT keys.
 //  3a. upsweep: digit counts of every tile, digit-major
 //      (counts[d * ntiles + tile]), so that one exclusive scan of `counts`
@@ -622,24 +590,35 @@ constexpr bool radix_split(int EW) { return EW >= 3; }
 //    inclusive prefix and places the digit's run at
 //    global start + prefix. A tile publishes its aggregate before it waits on
 //    anything, so every walk ends.
-//    Elements of 12 or 16 bytes are reordered through LDS in two phases, the
-//    keys and then the values (the same LDS), so LDS holds one of them per
-//    tile instead of the whole element: 6 waves per SIMD instead of 4 for
-//    u64 keys with u32 values (11.33 -> 10.52 ms at 2^27). Narrower elements
-//    gain no waves that way (registers bound them) and keep one phase.
+//    What bounds it: the status rows that the look-back reads (2 KB per
+//    predecessor, through the Infinity Cache), the partial lines at the ends of
+//    the runs, and how far two blocks' phases overlap per CU. All shrink with
+//    the tile, so a key takes as few as it can of the 64 registers per lane
+//    that two 1024-thread blocks leave: the digit is taken from the key again
+//    wherever it is used (held per key it cost a third of the tile), the
+//    per-wave counts are 16-bit in LDS, and elements of 12 or 16 bytes hold
+//    only their keys while they are ranked: they are reordered through LDS in
+//    two phases, the keys and then the values, which are loaded in between.
+//    Per pass, before -> now: 2^28 u32 + u32 1.75 (6144-key tiles) -> 1.32 ms
+//    (8192), 2^27 u64 + u32 1.13 (5120) -> 0.86 ms (8192). Counting after the
+//    ranking instead of by one LDS atomic per key before it: 1.38 and 0.91
+//    (predecessors' counts come too late); 2, 6 or 8 predecessors a step: 1.36,
+//    1.45, 2.44; keys and values of 8-byte elements in two phases (10240-key
+//    tiles): 1.35.
 template <typename K, int MODE, int EW, int BLOCK, int IPT = kRadixIpt>
-__global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
+__global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
     const RadixPass* __restrict__ table, int pass, const uint32_t* __restrict__ gbase,
     uint32_t* __restrict__ tile_counters, uint64_t* __restrict__ status, uint32_t gen,
     uint32_t n) {
   constexpr int NW = BLOCK / kWave;
   constexpr uint32_t TILE = (uint32_t)BLOCK * IPT;
   constexpr int KW = (int)sizeof(K) / 4, VW = EW - KW;
+  static_assert(TILE <= 65535, "16-bit counts");
   using V = typename std::conditional<VW == 2, uint64_t, uint32_t>::type;
   constexpr bool kSplit = radix_split(EW);
   constexpr int MW = kSplit ? (KW > VW ? KW : VW) : EW;  // LDS words per element
   __shared__ __align__(16) uint32_t s_part[TILE * MW];
-  __shared__ uint32_t s_hist[NW][kRadixBins];     // per-wave counts, then wave offsets
+  __shared__ uint16_t s_hist[NW][kRadixBins];     // per-wave counts, then wave offsets
   __shared__ uint32_t s_tile_start[kRadixBins];   // in-tile start of each digit
   __shared__ uint32_t s_goff[kRadixBins];         // global position - in-tile position
   __shared__ uint32_t s_wsum[kRadixBins / kWave];
@@ -651,7 +630,8 @@ __global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid / 64u;
   const bool digit_thread = tid < (uint32_t)kRadixBins;
-  for (uint32_t i = tid; i < NW * kRadixBins; i += BLOCK) (&s_hist[0][0])[i] = 0;
+  for (uint32_t i = tid; i < NW * kRadixBins / 2; i += BLOCK)
+    reinterpret_cast<uint32_t*>(&s_hist[0][0])[i] = 0;
   if (digit_thread) s_cnt[tid] = 0;
   if (tid == 0) s_tile = atomicAdd(tile_counters + pass, 1u);
   __syncthreads();
@@ -659,18 +639,23 @@ __global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
   const size_t base = (size_t)tile * TILE + (size_t)wid * (kWave * IPT);
   const uint32_t shift = rp.shift;
 
-  Elem<EW> el[IPT];
-  uint32_t dig[IPT];
+  // The wave's keys are [base, base + left); key j of a lane is the lane's of
+  // row j.
+  const uint32_t left = base < n ? (uint32_t)min((size_t)n - base, (size_t)kWave * IPT) : 0u;
+  auto valid = [&](int j) { return (uint32_t)j * kWave + lane < left; };
+  auto digit = [&](const auto& e) {
+    return (uint32_t)(order_bits<K, MODE>(elem_key<K, sizeof(e) / 4>(e)) >> shift) & 0xffu;
+  };
+  // Two phases: the keys only.
+  constexpr int HW = kSplit ? KW : EW;
+  Elem<HW> el[IPT];
   uint32_t rank[IPT];
+  const K* src_k = (const K*)rp.src_k + base + lane;
 #pragma unroll
   for (int j = 0; j < IPT; ++j) {
-    const size_t i = base + (size_t)j * kWave + lane;
-    if (i < n) {
-      el[j] = load_elem<K, EW>(rp, i);
-      dig[j] = (uint32_t)(order_bits<K, MODE>(elem_key<K, EW>(el[j])) >> shift) & 0xffu;
-    } else {
-      dig[j] = 0x100u;
-    }
+    if (!valid(j)) continue;
+    if constexpr (kSplit) el[j] = bit_cast<Elem<HW>>(src_k[j * kWave]);
+    else el[j] = load_elem<K, EW>(rp, base + (size_t)j * kWave + lane);
   }
   uint32_t gstart = 0;
   if (digit_thread) gstart = gbase[pass * kRadixBins + tid];
@@ -680,7 +665,7 @@ __global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
   // for this tile's ranking.
 #pragma unroll
   for (int j = 0; j < IPT; ++j)
-    if (dig[j] < 0x100u) atomicAdd(&s_cnt[dig[j]], 1u);
+    if (valid(j)) atomicAdd(&s_cnt[digit(el[j])], 1u);
   __syncthreads();
   uint64_t* my_status = status + (size_t)tile * kRadixBins + tid;
   uint32_t cnt = 0;
@@ -689,17 +674,19 @@ __global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
     st_agent(my_status, pack_status(gen, tile == 0 ? kFlagInc : kFlagAgg, 0, cnt));
   }
 
-  // Wave-level multi-split, as in the downsweep.
+  // Wave-level multi-split, as in the downsweep. (The empty asm makes the
+  // compiler form the digit again instead of keeping all of them.)
   const uint64_t lt = lanemask_lt();
 #pragma unroll
   for (int j = 0; j < IPT; ++j) {
-    const uint32_t d = dig[j];
-    const bool valid = d < 0x100u;
-    const uint64_t peers = match_digit<8>(d, valid);
+    asm volatile("" : "+v"(el[j].w[0]));
+    const uint32_t d = digit(el[j]);
+    const uint64_t peers = match_digit<8>(d, valid(j));
     uint32_t before = 0;
-    if (valid) before = s_hist[wid][d];
+    if (valid(j)) before = s_hist[wid][d];
     const uint32_t below = (uint32_t)__builtin_popcountll(peers & lt);
-    if (valid && below == 0) s_hist[wid][d] = before + (uint32_t)__builtin_popcountll(peers);
+    if (valid(j) && below == 0)
+      s_hist[wid][d] = (uint16_t)(before + (uint32_t)__builtin_popcountll(peers));
     rank[j] = before + below;
   }
   __syncthreads();
@@ -710,7 +697,7 @@ __global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const uint32_t c = s_hist[w][tid];
-      s_hist[w][tid] = acc;
+      s_hist[w][tid] = (uint16_t)acc;
       acc += c;
     }
   }
@@ -758,64 +745,68 @@ __global__ __launch_bounds__(BLOCK) void radix_onesweep_kernel(
   }
   __syncthreads();
 
-  // Reorder into digit-sorted runs in LDS, then write the runs out (split:
-  // the keys first, each output position's digit kept for the values, then
-  // the values).
+  // Reorder into digit-sorted runs in LDS, then write the runs out (two
+  // phases: the keys first, each output position's digit kept for the values,
+  // then the values).
 #pragma unroll
-  for (int j = 0; j < IPT; ++j)
-    if (dig[j] < 0x100u) rank[j] += s_tile_start[dig[j]] + s_hist[wid][dig[j]];
+  for (int j = 0; j < IPT; ++j) {
+    if (!valid(j)) continue;
+    asm volatile("" : "+v"(el[j].w[0]));
+    const uint32_t d = digit(el[j]);
+    rank[j] += s_tile_start[d] + s_hist[wid][d];
+  }
   const uint32_t tile_n = (uint32_t)min((size_t)TILE, (size_t)n - (size_t)tile * TILE);
   if constexpr (!kSplit) {
     Elem<EW>* s_el = reinterpret_cast<Elem<EW>*>(s_part);
 #pragma unroll
     for (int j = 0; j < IPT; ++j)
-      if (dig[j] < 0x100u) s_el[rank[j]] = el[j];
+      if (valid(j)) s_el[rank[j]] = el[j];
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < IPT; ++q) {
       const uint32_t i = tid + (uint32_t)q * BLOCK;
       if (i < tile_n) {
         const Elem<EW> e = s_el[i];
-        const uint32_t d = (uint32_t)(order_bits<K, MODE>(elem_key<K, EW>(e)) >> shift) & 0xffu;
-        store_elem<K, EW>(rp, (size_t)s_goff[d] + i, e);
+        store_elem<K, EW>(rp, (size_t)s_goff[digit(e)] + i, e);
       }
     }
     return;
   }
-  K* s_key = reinterpret_cast<K*>(s_part);
+  Elem<KW>* s_key = reinterpret_cast<Elem<KW>*>(s_part);
 #pragma unroll
   for (int j = 0; j < IPT; ++j)
-    if (dig[j] < 0x100u) s_key[rank[j]] = elem_key<K, EW>(el[j]);
+    if (valid(j)) s_key[rank[j]] = bit_cast<Elem<KW>>(elem_key<K, HW>(el[j]));
+  V val[IPT];
+  const V* src_v = (const V*)rp.src_v + base + lane;
+  if constexpr (VW > 0) {
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+      if (valid(j)) val[j] = src_v[j * kWave];
+  }
   __syncthreads();
-  uint32_t dq[IPT];
+  uint32_t dq[(IPT + 3) / 4] = {};  // four digits each
 #pragma unroll
   for (int q = 0; q < IPT; ++q) {
     const uint32_t i = tid + (uint32_t)q * BLOCK;
-    dq[q] = 0;
     if (i < tile_n) {
-      const K k = s_key[i];
-      dq[q] = (uint32_t)(order_bits<K, MODE>(k) >> shift) & 0xffu;
-      store_key_part<K, EW>(rp, (size_t)s_goff[dq[q]] + i, k);
+      const Elem<KW> k = s_key[i];
+      const uint32_t d = digit(k);
+      dq[q / 4] |= d << (8 * (q & 3));
+      ((K*)rp.dst_k)[(size_t)s_goff[d] + i] = bit_cast<K>(k);
     }
   }
-  if constexpr (VW > 0) {
-    __syncthreads();  // every key read out before the values overwrite them
-    V* s_val = reinterpret_cast<V*>(s_part);
+  if constexpr (VW == 0) return;
+  __syncthreads();  // every key read out before the values overwrite them
+  V* s_val = reinterpret_cast<V*>(s_part);
 #pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      if (dig[j] < 0x100u) {
-        V v;
-        if constexpr (VW == 1) v = el[j].w[KW];
-        else v = ((uint64_t)el[j].w[KW + 1] << 32) | el[j].w[KW];
-        s_val[rank[j]] = v;
-      }
-    }
-    __syncthreads();
+  for (int j = 0; j < IPT; ++j)
+    if (valid(j)) s_val[rank[j]] = val[j];
+  __syncthreads();
 #pragma unroll
-    for (int q = 0; q < IPT; ++q) {
-      const uint32_t i = tid + (uint32_t)q * BLOCK;
-      if (i < tile_n) store_val_part<K, EW, V>(rp, (size_t)s_goff[dq[q]] + i, s_val[i]);
-    }
+  for (int q = 0; q < IPT; ++q) {
+    const uint32_t i = tid + (uint32_t)q * BLOCK;
+    if (i < tile_n)
+      ((V*)rp.dst_v)[(size_t)s_goff[(dq[q / 4] >> (8 * (q & 3))) & 0xffu] + i] = s_val[i];
   }
 }
 
