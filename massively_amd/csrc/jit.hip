@@ -347,9 +347,7 @@ static msv_status user_reduce_api(msv_executor* ex, const msv_slice* input,
     m = tiles;
     aligned = true;
   }
-  MSV_HIP(hipMemcpyAsync(out_host, d_result, es, hipMemcpyDeviceToHost, c.stream()));
-  MSV_HIP(hipStreamSynchronize(c.stream()));
-  return MSV_OK;
+  return read_back(ex, d_result, es, out_host);
 }
 
 // The built-in predicate's kernel argument (Pred<S>) for the op's dtype.

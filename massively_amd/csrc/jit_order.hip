@@ -642,12 +642,7 @@ msv_status msv_seg_unique_user(msv_executor* ex, msv_slice values, const msv_seg
   }
   uint32_t kept = 0;
   if (s == MSV_OK) {
-    hipError_t e = hipMemcpyAsync(&kept, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost, ex->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ex->stream);
-    if (e != hipSuccess) {
-      set_error(MSV_ERR_LAUNCH, 0, 0, "seg unique failed: %s", hipGetErrorString(e));
-      s = MSV_ERR_LAUNCH;
-    }
+    s = read_back(ex, d_count, sizeof(uint32_t), &kept);
   }
   if (s != MSV_OK) {
     if (vals) msv_vec_release(vals);

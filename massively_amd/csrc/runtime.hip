@@ -103,6 +103,7 @@ void executor_release(msv_executor* ex) {
   (void)hipStreamSynchronize(ex->stream);
   if (ex->d_status) (void)hipFree(ex->d_status);
   if (ex->d_counter) (void)hipFree(ex->d_counter);
+  if (ex->h_words) (void)hipHostFree(ex->h_words);
   ex->allocator.trim();
   if (ex->aux_stream) {
     (void)hipStreamSynchronize(ex->aux_stream);
@@ -121,6 +122,20 @@ msv_status no_capture(msv_executor* ex, const char* what) {
     return MSV_ERR_UNSUPPORTED;
   }
   return MSV_OK;
+}
+
+// ---- scalars to the host ------------------------------------------------------
+static __global__ void read_back_kernel(const uint32_t* __restrict__ src, uint32_t* dst, uint32_t words) {
+  if (threadIdx.x < words) dst[threadIdx.x] = src[threadIdx.x];
+}
+
+msv_status read_back(msv_executor* ex, const void* src, size_t bytes, void* host) {
+  return read_back_from(ex, bytes, host, [&](void* words) {
+    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3((unsigned)(kReadBackBytes / 4)), 0, ex->stream,
+                       (const uint32_t*)src, (uint32_t*)words, (uint32_t)(bytes / 4));
+    MSV_HIP(hipGetLastError());
+    return MSV_OK;
+  });
 }
 
 // ---- views ------------------------------------------------------------------
@@ -143,9 +158,7 @@ msv_status resolve(msv_executor* ex, const msv_slice& s, View* out) {
   if (v->d_len && s.len == MSV_WHOLE) {
     MSV_TRY(no_capture(ex, "a whole-length slice of a vector with a device-resident length"));
     MSV_HIP(hipSetDevice(ex->device));
-    MSV_HIP(hipMemcpyAsync(&logical, v->d_len, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                           ex->stream));
-    MSV_HIP(hipStreamSynchronize(ex->stream));
+    MSV_TRY(read_back(ex, v->d_len, sizeof(uint32_t), &logical));
     if (logical > v->capacity) logical = v->capacity;
   }
   if (s.offset > logical && s.len == MSV_WHOLE) {
@@ -372,6 +385,7 @@ msv_status msv_executor_create(int32_t device, msv_executor** out) {
   hipError_t e = hipStreamCreateWithFlags(&ex->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void**)&ex->d_counter, 8);
   if (e == hipSuccess) e = hipMemsetAsync(ex->d_counter, 0, 8, ex->stream);
+  if (e == hipSuccess) e = hipHostMalloc(&ex->h_words, kReadBackBytes);
   if (e != hipSuccess) {
     set_error(MSV_ERR_LAUNCH, 0, 0, "executor creation failed: %s", hipGetErrorString(e));
     delete ex;
@@ -382,6 +396,7 @@ msv_status msv_executor_create(int32_t device, msv_executor** out) {
   if (ns != MSV_OK) {
     (void)hipStreamDestroy(ex->stream);
     (void)hipFree(ex->d_counter);
+    (void)hipHostFree(ex->h_words);
     delete ex;
     return ns;
   }
@@ -598,8 +613,8 @@ msv_status msv_to_host(msv_executor* ex, msv_slice src, void* host, uint32_t hos
   if (src.vec->d_len && src.len != MSV_WHOLE) {
     // Explicit ranges are clipped to the device-resident length as well.
     uint32_t logical = 0;
-    MSV_HIP(hipMemcpyAsync(&logical, src.vec->d_len, 4, hipMemcpyDeviceToHost, ex->stream));
-    MSV_HIP(hipStreamSynchronize(ex->stream));
+    MSV_HIP(hipSetDevice(ex->device));
+    MSV_TRY(read_back(ex, src.vec->d_len, sizeof(uint32_t), &logical));
     if (src.offset >= logical) len = 0;
     else if ((uint64_t)src.offset + len > logical) len = logical - src.offset;
   }

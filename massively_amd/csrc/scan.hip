@@ -123,12 +123,9 @@ static msv_status reduce_typed(Ctx& c, const void* in, uint32_t n, const void* i
   MSV_TRY(no_capture(c.ex(), "reduce (host result)"));
   T init;
   memcpy(&init, init_host, sizeof(T));
-  T* d_result = (T*)c.scratch(sizeof(T));
-  if (!d_result) return MSV_ERR_OUT_OF_MEMORY;
-  MSV_TRY((reduce_impl<T, OP>(c, (const T*)in, n, init, d_result)));
-  MSV_HIP(hipMemcpyAsync(out_host, d_result, sizeof(T), hipMemcpyDeviceToHost, c.stream()));
-  MSV_HIP(hipStreamSynchronize(c.stream()));
-  return MSV_OK;
+  return read_back_from(c.ex(), sizeof(T), out_host, [&](void* words) {
+    return reduce_impl<T, OP>(c, (const T*)in, n, init, (T*)words);
+  });
 }
 
 #define MSV_DISPATCH_OP(T, FN, ...)                                     \

@@ -392,12 +392,7 @@ static msv_status seg_compact_api(msv_executor* ex, msv_slice values, const msv_
   }
   uint32_t kept = 0;
   if (s == MSV_OK) {
-    hipError_t e = hipMemcpyAsync(&kept, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost, ex->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ex->stream);
-    if (e != hipSuccess) {
-      set_error(MSV_ERR_LAUNCH, 0, 0, "segment compaction failed: %s", hipGetErrorString(e));
-      s = MSV_ERR_LAUNCH;
-    }
+    s = read_back(ex, d_count, sizeof(uint32_t), &kept);
   }
   if (s != MSV_OK) {
     if (vals) msv_vec_release(vals);

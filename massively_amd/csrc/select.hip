@@ -254,12 +254,7 @@ extern "C" msv_status msv_partition(msv_executor* ex, msv_slice input, const msv
     }
   }
   if (s == MSV_OK) {
-    hipError_t e = hipMemcpyAsync(boundary, d_total, sizeof(uint32_t), hipMemcpyDeviceToHost, ex->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ex->stream);
-    if (e != hipSuccess) {
-      set_error(MSV_ERR_LAUNCH, 0, 0, "partition failed: %s", hipGetErrorString(e));
-      s = MSV_ERR_LAUNCH;
-    }
+    s = read_back(ex, d_total, sizeof(uint32_t), boundary);
   }
   if (s != MSV_OK) {
     msv_vec_release(*out);
