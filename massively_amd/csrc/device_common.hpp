@@ -404,6 +404,12 @@ __device__ inline uint64_t add_agent(uint64_t* p, uint64_t v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Tells the host that the stores before it (to pinned memory, by this thread)
+// are there.
+__device__ inline void read_back_done(uint32_t* flag, uint32_t seq) {
+  __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------------------
 // Decoupled lookback.
 //

@@ -101,9 +101,10 @@ struct msv_executor {
   uint64_t* d_status;
   size_t status_words;
   uint32_t lookback_gen;
-  // Pinned host words that scalar results are written to (see read_back); one
-  // reader at a time.
-  void* h_words = nullptr;
+  // Pinned host words that scalar results are written to and the number of the
+  // last one (see read_back); one reader at a time.
+  uint32_t* h_words = nullptr;
+  uint32_t read_seq = 0;
   std::mutex read_mutex;
   // Tuning options (msv_executor_set_option).
   int64_t opt_seg_launch = MSV_SEG_LAUNCH_PERSISTENT;
@@ -163,25 +164,30 @@ msv_status no_capture(msv_executor* ex, const char* what);
 // MSV_WHOLE slice of a vector whose length is device-resident).
 msv_status resolve(msv_executor* ex, const msv_slice& s, View* out);
 
-// A scalar result on its way to the host: a kernel writes it to the executor's
-// pinned words (at most kReadBackBytes) and the stream is waited for. A copy to
-// pageable memory and the wait for it had cost a reduce of 5000 values 28 us;
-// so it takes 15.
-constexpr size_t kReadBackBytes = 64;
-// Copies `bytes` (a multiple of 4) from device memory to `host` after the work
-// enqueued so far.
-msv_status read_back(msv_executor* ex, const void* src, size_t bytes, void* host);
-// The same around a producer that is enqueued by `enqueue(words)` and writes
-// the pinned words itself.
+// A scalar result (4 or 8 bytes) on its way to the host: a kernel writes it to
+// the executor's pinned words and then `seq` to the word `flag` (read_back_done
+// in device code), which the host polls; after kReadBackPollUs it waits for the
+// stream instead, which also reports an error of the work before. A reduce of
+// 5000 values: 28 us with a copy to pageable memory, 19 with a wait for the
+// stream, 14 polled.
+struct ReadBack {
+  void* value;
+  uint32_t* flag;
+  uint32_t seq;
+};
+constexpr int kReadBackPollUs = 200;
+// Waits for the result of one ReadBack and copies it to `host`.
+msv_status read_back_wait(msv_executor* ex, const ReadBack& rb, size_t bytes, void* host);
+// `enqueue(rb)` enqueues the kernel that writes the result.
 template <typename F>
 msv_status read_back_from(msv_executor* ex, size_t bytes, void* host, F enqueue) {
   std::lock_guard<std::mutex> lk(ex->read_mutex);
-  const msv_status s = enqueue(ex->h_words);
-  if (s != MSV_OK) return s;
-  MSV_HIP(hipStreamSynchronize(ex->stream));
-  memcpy(host, ex->h_words, bytes);
-  return MSV_OK;
+  const ReadBack rb = {ex->h_words, ex->h_words + 15, ++ex->read_seq};
+  const msv_status s = enqueue(rb);
+  return s == MSV_OK ? read_back_wait(ex, rb, bytes, host) : s;
 }
+// Copies 4 or 8 bytes from device memory to `host` after the work enqueued so far.
+msv_status read_back(msv_executor* ex, const void* src, size_t bytes, void* host);
 
 // Creates a new owned output vector.
 msv_status new_vec(msv_executor* ex, msv_dtype dtype, uint32_t capacity, bool device_len,

@@ -1,7 +1,9 @@
 // Executor, DeviceVec and DeviceSlice of the C ABI
 // (massively/src/core/runtime.rs:21-545, core/extent.rs, core/error.rs).
+#include <chrono>
 #include <cstring>
 
+#include "device_common.hpp"
 #include "msv_internal.hpp"
 
 namespace msv {
@@ -125,14 +127,28 @@ msv_status no_capture(msv_executor* ex, const char* what) {
 }
 
 // ---- scalars to the host ------------------------------------------------------
-static __global__ void read_back_kernel(const uint32_t* __restrict__ src, uint32_t* dst, uint32_t words) {
-  if (threadIdx.x < words) dst[threadIdx.x] = src[threadIdx.x];
+static __global__ void read_back_kernel(const uint32_t* __restrict__ src, uint32_t words,
+                                        uint32_t* dst, uint32_t* flag, uint32_t seq) {
+  for (uint32_t i = 0; i < words; ++i) dst[i] = src[i];
+  read_back_done(flag, seq);
+}
+
+msv_status read_back_wait(msv_executor* ex, const ReadBack& rb, size_t bytes, void* host) {
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kReadBackPollUs);
+  bool seen = false;
+  for (uint32_t polls = 1; !seen; ++polls) {
+    seen = __atomic_load_n(rb.flag, __ATOMIC_ACQUIRE) == rb.seq;
+    if (!seen && polls % 64 == 0 && std::chrono::steady_clock::now() > until) break;
+  }
+  if (!seen) MSV_HIP(hipStreamSynchronize(ex->stream));
+  memcpy(host, rb.value, bytes);
+  return MSV_OK;
 }
 
 msv_status read_back(msv_executor* ex, const void* src, size_t bytes, void* host) {
-  return read_back_from(ex, bytes, host, [&](void* words) {
-    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3((unsigned)(kReadBackBytes / 4)), 0, ex->stream,
-                       (const uint32_t*)src, (uint32_t*)words, (uint32_t)(bytes / 4));
+  return read_back_from(ex, bytes, host, [&](const ReadBack& rb) {
+    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(1), 0, ex->stream, (const uint32_t*)src,
+                       (uint32_t)(bytes / 4), (uint32_t*)rb.value, rb.flag, rb.seq);
     MSV_HIP(hipGetLastError());
     return MSV_OK;
   });
@@ -385,7 +401,8 @@ msv_status msv_executor_create(int32_t device, msv_executor** out) {
   hipError_t e = hipStreamCreateWithFlags(&ex->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void**)&ex->d_counter, 8);
   if (e == hipSuccess) e = hipMemsetAsync(ex->d_counter, 0, 8, ex->stream);
-  if (e == hipSuccess) e = hipHostMalloc(&ex->h_words, kReadBackBytes);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&ex->h_words, 64);
+  if (e == hipSuccess) memset(ex->h_words, 0, 64);
   if (e != hipSuccess) {
     set_error(MSV_ERR_LAUNCH, 0, 0, "executor creation failed: %s", hipGetErrorString(e));
     delete ex;

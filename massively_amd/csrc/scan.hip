@@ -35,7 +35,8 @@ static bool is_aligned16(const void* p) {
 }
 
 template <typename T, int OP>
-static msv_status reduce_impl(Ctx& c, const T* in, uint32_t n, T init, T* d_result) {
+static msv_status reduce_impl(Ctx& c, const T* in, uint32_t n, T init, T* d_result,
+                              uint32_t* flag = nullptr, uint32_t seq = 0) {
   constexpr uint32_t TILE = (uint32_t)kReduceBlock * kReduceRows * (16 / sizeof(T));
   const T* src = in;
   uint32_t m = n;
@@ -46,7 +47,8 @@ static msv_status reduce_impl(Ctx& c, const T* in, uint32_t n, T init, T* d_resu
     T* dst = last ? d_result : (T*)c.scratch((size_t)tiles * sizeof(T));
     if (!dst) return MSV_ERR_OUT_OF_MEMORY;
     hipLaunchKernelGGL((reduce_tile_kernel<T, OP, kReduceBlock, kReduceRows, true>), dim3(tiles),
-                       dim3(kReduceBlock), 0, c.stream(), src, m, aligned, dst, last, init);
+                       dim3(kReduceBlock), 0, c.stream(), src, m, aligned, dst, last, init,
+                       last ? flag : nullptr, seq);
     MSV_HIP(hipGetLastError());
     if (last) return MSV_OK;
     src = dst;
@@ -68,7 +70,7 @@ static msv_status float_scan_impl(Ctx& c, const T* in, T* out, uint32_t n, T ini
     if (!partials || !pre) return MSV_ERR_OUT_OF_MEMORY;
     hipLaunchKernelGGL((reduce_tile_kernel<T, OP, kScanBlock, kScanRows>), dim3(ntiles),
                        dim3(kScanBlock), 0, c.stream(), in, n, aligned, partials, false,
-                       Combine<T, OP>::identity());
+                       Combine<T, OP>::identity(), (uint32_t*)nullptr, 0u);
     MSV_HIP(hipGetLastError());
     MSV_TRY((float_scan_impl<T, OP, true>(c, partials, pre, ntiles, Combine<T, OP>::identity())));
     prefixes = pre;
@@ -123,8 +125,8 @@ static msv_status reduce_typed(Ctx& c, const void* in, uint32_t n, const void* i
   MSV_TRY(no_capture(c.ex(), "reduce (host result)"));
   T init;
   memcpy(&init, init_host, sizeof(T));
-  return read_back_from(c.ex(), sizeof(T), out_host, [&](void* words) {
-    return reduce_impl<T, OP>(c, (const T*)in, n, init, (T*)words);
+  return read_back_from(c.ex(), sizeof(T), out_host, [&](const ReadBack& rb) {
+    return reduce_impl<T, OP>(c, (const T*)in, n, init, (T*)rb.value, rb.flag, rb.seq);
   });
 }
 

@@ -235,13 +235,15 @@ __device__ inline T tree_fold(T (&v)[N]) {
 // Reduces one tile of BLOCK*ROWS vectors per block into partials[blockIdx.x]
 // with a fixed tree: thread (pairwise over ROWS*V) -> wave (DPP) -> block
 // (pairwise over waves). With `apply_init`, block 0 writes op(init, total)
-// (used when one block covers the whole input). NT: non-temporal loads, for
+// (used when one block covers the whole input) and, with `flag`, tells the host
+// that polls for it. NT: non-temporal loads, for
 // an input read once (reduce); the float scans' partials pass keeps ordinary
 // loads, since their prefixed pass reads the same input again right after.
 template <typename T, int OP, int BLOCK, int ROWS, bool NT = false>
 __global__ __launch_bounds__(BLOCK) void reduce_tile_kernel(const T* __restrict__ in, uint32_t n,
                                                             bool aligned, T* __restrict__ partials,
-                                                            bool apply_init, T init) {
+                                                            bool apply_init, T init,
+                                                            uint32_t* flag, uint32_t seq) {
   using C = Combine<T, OP>;
   constexpr int V = 16 / sizeof(T);
   constexpr int NW = BLOCK / kWave;
@@ -267,6 +269,7 @@ __global__ __launch_bounds__(BLOCK) void reduce_tile_kernel(const T* __restrict_
     for (int i = 0; i < NW; ++i) w[i] = s_wave[i];
     T total = tree_fold<T, OP, NW>(w);
     partials[blockIdx.x] = apply_init ? C::apply(init, total) : total;
+    if (flag) read_back_done(flag, seq);
   }
 }
 
