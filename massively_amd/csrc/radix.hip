@@ -59,6 +59,25 @@ constexpr int radix_onesweep_block() { return 1024; }
 template <int EW>
 constexpr int radix_onesweep_ipt() { return EW == 1 ? 10 : 8; }
 
+// Sorts of up to this many keys run tiles of 2, or of 6 keys per thread: they are
+// bound by a pass's latency, which grows with the rows a wave ranks, and then by
+// how many tiles the CUs get (us a pass of u32 + u32 with 2, 6 and 8 keys: 2^16
+// 7.7, 9.8, 11.6; 2^18 11.2, 11.7, 13.3; 2^20 22.9, 17.5, 17.8; 1.5 million 6:
+// 19.2, 8: 20.7; 2 million 22.8, 21.7).
+constexpr uint32_t kRadixSmall = 1u << 18, kRadixMiddle = 7u << 18;
+
+// The local sort's elements per thread (two blocks' LDS per CU), and the sorts
+// that try one pass and local sorts: where the average run fills at most 7/8 of
+// a block. Whole sorts with a u32 payload, before -> now (us): 2000 u32 38.6 ->
+// 15.4, u64 70 -> 16.7; 8000 u32 47.6 -> 31.5, u64 91 -> 46;
+// 65536 u32 52.8 -> 31.5, u64 102 -> 44.4; 2^20 u32 88.8 -> 56.5, u64 179
+// -> 72.5. Keys whose highest byte has too few values keep all their passes (f32
+// normal, 2^20: 90.6 -> 88.8; the launch that finds nothing costs them 2 us).
+template <int EW>
+constexpr int radix_local_ipt() { return EW <= 2 ? 8 : (EW == 3 ? 5 : 4); }
+template <int EW>
+constexpr uint32_t radix_local_tile() { return 1024u * radix_local_ipt<EW>(); }
+
 template <typename K, int MODE, int VS>
 static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, uint32_t n,
                                   void* out_k, void* out_v) {
@@ -68,6 +87,19 @@ static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, ui
   constexpr int IPT = radix_ipt<EW>();
   constexpr uint32_t TILE = (uint32_t)BLOCK * IPT;
   if (n == 0) return MSV_OK;
+  // Schedule: onesweep unless the executor option forces reduce-then-scan.
+  const int64_t sched = c.ex()->opt_radix_onesweep;
+  constexpr int LIPT = radix_local_ipt<EW>();
+  constexpr uint32_t LTILE = radix_local_tile<EW>();
+  if (sched != 0 && n <= LTILE) {
+    const RadixPass only = {1u, 0u, 0u, 0u, keys, vals, out_k, out_v};
+    // Eight-byte keys are sorted by three digits and a repair.
+    constexpr int DIGITS = P == 8 ? 3 : P;
+    hipLaunchKernelGGL((radix_local_kernel<K, MODE, EW, 1024, LIPT, DIGITS>), dim3(1), dim3(1024), 0,
+                       c.stream(), (const RadixLocal*)nullptr, (const uint32_t*)nullptr, only, n);
+    MSV_HIP(hipGetLastError());
+    return MSV_OK;
+  }
   const uint32_t ntiles = div_up(n, TILE);
   const size_t elem_bytes = (size_t)n * EW * 4;
   // Two-phase onesweep passes keep keys and values apart between passes: the
@@ -77,34 +109,51 @@ static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, ui
   void* aos1 = c.scratch(elem_bytes + 256);
   RadixPass* table = (RadixPass*)c.scratch(sizeof(RadixPass) * P);
   if (!aos0 || !aos1 || !table) return MSV_ERR_OUT_OF_MEMORY;
-  // Schedule: onesweep unless the executor option forces reduce-then-scan.
-  const int64_t sched = c.ex()->opt_radix_onesweep;
   if (sched != 0) {
     // Onesweep: histograms of every digit position in one read of the keys,
     // then one look-back pass per digit position that needs one.
+    RadixPlan q = {};
     uint32_t* hist = (uint32_t*)c.scratch(sizeof(uint32_t) * (kRadixBins * P + P));
-    uint32_t* gbase = (uint32_t*)c.scratch(sizeof(uint32_t) * kRadixBins * P);
-    if (!hist || !gbase) return MSV_ERR_OUT_OF_MEMORY;
-    uint32_t* tile_counters = hist + kRadixBins * P;
+    q.gbase = (uint32_t*)c.scratch(sizeof(uint32_t) * kRadixBins * P);
+    q.local = (RadixLocal*)c.scratch(sizeof(RadixLocal));
+    if (!hist || !q.gbase || !q.local) return MSV_ERR_OUT_OF_MEMORY;
+    q.hist = hist;
+    q.tile_counters = hist + kRadixBins * P;
+    q.table = table;
+    q.local_max = n <= LTILE / 8 * 7 * kRadixBins ? LTILE : 0u;
+    q.in_k = keys;
+    q.in_v = vals;
+    q.out_k = out_k;
+    q.out_v = out_v;
+    q.aos0 = aos0;
+    q.aos1 = aos1;
+    q.vofs = vofs;
     hipLaunchKernelGGL(fill_u32_kernel, dim3(div_up(kRadixBins * P, 256)), dim3(256), 0,
                        c.stream(), hist, (uint32_t)(kRadixBins * P), 0u);
     const uint32_t hist_blocks = min(div_up(n, 256u * 16u), (uint32_t)c.num_cus() * 8u);
     hipLaunchKernelGGL((radix_hist_kernel<K, MODE, 256>), dim3(hist_blocks), dim3(256), 0,
                        c.stream(), (const K*)keys, n, hist);
-    hipLaunchKernelGGL((radix_onesweep_plan_kernel<P>), dim3(1), dim3(kRadixBins), 0, c.stream(),
-                       hist, n, table, gbase, tile_counters, keys, vals, out_k, out_v, aos0, aos1,
-                       vofs);
+    hipLaunchKernelGGL((radix_onesweep_plan_kernel<P>), dim3(1), dim3(kRadixBins), 0, c.stream(), q, n);
     MSV_HIP(hipGetLastError());
     constexpr int OBLOCK = radix_onesweep_block<EW>();
     constexpr int OIPT = radix_onesweep_ipt<EW>();
-    const uint32_t otiles = div_up(n, (uint32_t)OBLOCK * OIPT);
+    const int ipt = n <= kRadixSmall ? 2 : (n <= kRadixMiddle ? 6 : OIPT);
+    const uint32_t otiles = div_up(n, (uint32_t)OBLOCK * ipt);
+    // Slot p runs the p-th pass of the plan; passes it leaves out end at once.
     for (int p = 0; p < P; ++p) {
       uint64_t *counter, *status;
       uint32_t gen;
       MSV_TRY(c.lookback((size_t)otiles * kRadixBins, &counter, &status, &gen));
-      hipLaunchKernelGGL((radix_onesweep_kernel<K, MODE, EW, OBLOCK, OIPT>), dim3(otiles),
-                         dim3(OBLOCK), 0, c.stream(), table, p, gbase, tile_counters, status, gen,
-                         n);
+      auto pass = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(otiles), dim3(OBLOCK), 0, c.stream(), table, p, q.gbase,
+                           q.tile_counters, status, gen, n);
+      };
+      if (ipt == 2) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 2>);
+      else if (ipt == 6) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 6>);
+      else pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, OIPT>);
+      if (p == 0 && q.local_max)
+        hipLaunchKernelGGL((radix_local_kernel<K, MODE, EW, 1024, LIPT, 2>), dim3(kRadixBins),
+                           dim3(1024), 0, c.stream(), q.local, q.gbase, RadixPass{}, n);
       MSV_HIP(hipGetLastError());
     }
     return MSV_OK;

@@ -27,7 +27,7 @@ __device__ inline K elem_key(const Elem<EW>& e) {
 
 struct RadixPass {
   uint32_t active;
-  uint32_t shift;
+  uint32_t shift;  // a multiple of 8
   uint32_t in_aos;   // source is an element array (else separate keys/values)
   uint32_t out_aos;  // destination is an element array
   const void* src_k;
@@ -420,6 +420,7 @@ __global__ __launch_bounds__(BLOCK) void radix_downsweep_kernel(
 //    common: small keys, a constant top byte) is counted by one add; the other
 //    positions take one LDS add per key and no per-key test (per key and
 //    position, a uniformity test had cost more instructions than the add).
+//    (Its last block making the plan, to save that launch, gained 0-2 us.)
 template <typename K, int MODE, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__ keys, uint32_t n,
                                                           uint32_t* __restrict__ hist) {
@@ -517,65 +518,94 @@ __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__
   }
 }
 
+// What the local sort (8) does after the first pass: sorts every run of equal
+// digits `top` by the digits below it.
+struct RadixLocal {
+  uint32_t on;
+  uint32_t top;
+  RadixPass pass;  // its source and destination
+};
+
 // 6. Onesweep plan (one block of 256 threads): the exclusive scan of every
 //    digit position's histogram (the global start of each digit in that
 //    pass), which positions need a pass (a position whose histogram puts all
-//    n keys in one bin is skipped), the pass table (as the reduce-then-scan
-//    plan) and zeroed tile counters.
+//    n keys in one bin is skipped), the pass table (the passes to run first;
+//    sources and destinations as in the reduce-then-scan plan) and zeroed tile
+//    counters.
+//    local_max > 0: when at least three positions need a pass and no digit of
+//    the highest holds more than local_max keys, only that position gets a
+//    pass, and `local` the rest.
 //    vofs = 0: the intermediate buffers hold interleaved elements; else each
 //    holds the keys and, vofs bytes in, the values (the two-phase passes).
+struct RadixPlan {
+  const uint32_t* hist;     // [P][256]
+  RadixPass* table;         // [P]
+  uint32_t* gbase;          // [P][256]
+  uint32_t* tile_counters;  // [P]
+  RadixLocal* local;
+  uint32_t local_max;
+  const void *in_k, *in_v;
+  void *out_k, *out_v, *aos0, *aos1;
+  size_t vofs;
+};
+
 template <int P>
-__global__ __launch_bounds__(kRadixBins) void radix_onesweep_plan_kernel(
-    const uint32_t* __restrict__ hist, uint32_t n, RadixPass* __restrict__ table,
-    uint32_t* __restrict__ gbase, uint32_t* __restrict__ tile_counters, const void* in_k,
-    const void* in_v, void* out_k, void* out_v, void* aos0, void* aos1, size_t vofs) {
-  __shared__ uint32_t s_trivial[P];
+__global__ __launch_bounds__(kRadixBins) void radix_onesweep_plan_kernel(RadixPlan q, uint32_t n) {
+  __shared__ uint32_t s_trivial[P], s_most[P];
   __shared__ uint32_t s_wsum[kRadixBins / kWave];
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
   if (t < (uint32_t)P) {
-    s_trivial[t] = 0;
-    tile_counters[t] = 0;
+    s_trivial[t] = s_most[t] = 0;
+    q.tile_counters[t] = 0;
   }
   __syncthreads();
   for (int p = 0; p < P; ++p) {
-    const uint32_t c = hist[p * kRadixBins + t];
+    const uint32_t c = q.hist[p * kRadixBins + t];
     if (c == n) s_trivial[p] = 1;
+    const uint32_t most = wave_reduce<uint32_t, OP_MAX>(c);
+    if (lane == 0) atomicMax(&s_most[p], most);
     const uint32_t incl = wave_inclusive_scan<uint32_t, OP_ADD>(c);
     if (lane == 63) s_wsum[wid] = incl;
     __syncthreads();
     uint32_t woff = 0;
     for (uint32_t k = 0; k < wid; ++k) woff += s_wsum[k];
-    gbase[p * kRadixBins + t] = woff + incl - c;
+    q.gbase[p * kRadixBins + t] = woff + incl - c;
     __syncthreads();
   }
-  if (t == 0) {
-    int active = 0;
-    for (int p = 0; p < P; ++p) active += s_trivial[p] ? 0 : 1;
-    // All digits constant (all keys equal): one pass still moves the data.
-    const bool force_last = active == 0;
-    if (force_last) active = 1;
-    int j = 0;
-    for (int p = 0; p < P; ++p) {
-      RadixPass rp;
-      rp.shift = 8u * (uint32_t)p;
-      rp.active = (!s_trivial[p] || (force_last && p == P - 1)) ? 1u : 0u;
-      rp.in_aos = rp.out_aos = 0;
-      rp.src_k = rp.src_v = nullptr;
-      rp.dst_k = rp.dst_v = nullptr;
-      if (rp.active) {
-        char* src = (char*)(((j - 1) & 1) ? aos1 : aos0);
-        char* dst = (char*)((j & 1) ? aos1 : aos0);
-        rp.in_aos = j > 0 && vofs == 0;
-        rp.out_aos = j < active - 1 && vofs == 0;
-        rp.src_k = j == 0 ? in_k : src;
-        rp.src_v = j == 0 ? in_v : (vofs ? src + vofs : nullptr);
-        rp.dst_k = j == active - 1 ? out_k : dst;
-        rp.dst_v = j == active - 1 ? out_v : (vofs ? dst + vofs : nullptr);
-        ++j;
-      }
-      table[p] = rp;
-    }
+  if (t != 0) return;
+  int active = 0, top = 0;
+  for (int p = 0; p < P; ++p) {
+    if (s_trivial[p]) continue;
+    ++active;
+    top = p;
   }
+  const bool split = q.vofs != 0;
+  const bool use_local = q.local_max > 0 && active >= 3 && s_most[top] <= q.local_max;
+  q.local->on = use_local ? 1u : 0u;
+  q.local->top = (uint32_t)top;
+  q.local->pass = RadixPass{1u, 0u, split ? 0u : 1u, 0u,
+                            q.aos0, split ? (char*)q.aos0 + q.vofs : nullptr, q.out_k, q.out_v};
+  // All digits constant (all keys equal): one pass still moves the data.
+  const bool force_last = active == 0;
+  const int passes = use_local || force_last ? 1 : active;
+  int j = 0;
+  for (int p = 0; p < P; ++p) {
+    if (use_local ? p != top : (force_last ? p != P - 1 : s_trivial[p] != 0)) continue;
+    const bool to_out = j == passes - 1 && !use_local;
+    char* src = (char*)(((j - 1) & 1) ? q.aos1 : q.aos0);
+    char* dst = (char*)((j & 1) ? q.aos1 : q.aos0);
+    RadixPass rp;
+    rp.active = 1;
+    rp.shift = 8u * (uint32_t)p;
+    rp.in_aos = j > 0 && !split;
+    rp.out_aos = !to_out && !split;
+    rp.src_k = j == 0 ? q.in_k : src;
+    rp.src_v = j == 0 ? q.in_v : (split ? src + q.vofs : nullptr);
+    rp.dst_k = to_out ? q.out_k : dst;
+    rp.dst_v = to_out ? q.out_v : (split ? dst + q.vofs : nullptr);
+    q.table[j++] = rp;
+  }
+  for (; j < P; ++j) q.table[j].active = 0;
 }
 
 // Whether a onesweep pass over EW-word elements reorders keys and values in
@@ -658,7 +688,7 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
     else el[j] = load_elem<K, EW>(rp, base + (size_t)j * kWave + lane);
   }
   uint32_t gstart = 0;
-  if (digit_thread) gstart = gbase[pass * kRadixBins + tid];
+  if (digit_thread) gstart = gbase[shift / 8 * kRadixBins + tid];
 
   // The tile's digit counts first (LDS atomics), published at once as its
   // aggregate: successors walking back meet an aggregate instead of waiting
@@ -808,6 +838,194 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
     if (i < tile_n)
       ((V*)rp.dst_v)[(size_t)s_goff[(dq[q / 4] >> (8 * (q & 3))) & 0xffu] + i] = s_val[i];
   }
+}
+
+// 8. Local sort: one block sorts up to TILE elements stably in LDS, by the
+//    digits [0, top) of which some vary. Each digit is ranked as a pass ranks
+//    it (no counts before, no look-back); elements stay in registers between
+//    digits and go through LDS whole. A digit costs about 7 us (its chain of
+//    ranks, barriers and LDS round trips), so only the highest DIGITS varying
+//    ones are sorted by, and runs that these leave equal are put in order by
+//    insertion, one thread a run. Runs longer than kLocalRun that are out of
+//    order (keys far from uniform) send the block through all its digits.
+//    Two uses: a sort of at most TILE elements is one launch of one block
+//    (src/dst in `only`), and after the first pass of a short sort block g
+//    sorts the run of digit g (`local`, gbase: where the runs start).
+constexpr uint32_t kLocalRun = 16;
+
+template <typename K, int MODE, int EW, int BLOCK, int IPT, int DIGITS>
+__global__ __launch_bounds__(BLOCK, 8) void radix_local_kernel(
+    const RadixLocal* __restrict__ local, const uint32_t* __restrict__ gbase, RadixPass only,
+    uint32_t n) {
+  constexpr int NW = BLOCK / kWave;
+  constexpr uint32_t TILE = (uint32_t)BLOCK * IPT;
+  constexpr int P = (int)sizeof(K);
+  __shared__ __align__(16) uint32_t s_part[TILE * EW];
+  __shared__ uint16_t s_hist[NW][kRadixBins];
+  __shared__ uint32_t s_start[kRadixBins];
+  __shared__ uint32_t s_wsum[kRadixBins / kWave];
+  __shared__ uint32_t s_diff[2];
+  uint32_t start = 0, cnt = n, top = P;
+  RadixPass rp = only;
+  if (local) {
+    if (!local->on) return;
+    rp = local->pass;
+    top = local->top;
+    const uint32_t* runs = gbase + top * kRadixBins;
+    start = runs[blockIdx.x];
+    cnt = (blockIdx.x + 1 < (uint32_t)kRadixBins ? runs[blockIdx.x + 1] : n) - start;
+  }
+  if (cnt == 0) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid / 64u;
+  const bool digit_thread = tid < (uint32_t)kRadixBins;
+  // Rows the elements need, and this wave's: [base, base + left).
+  const uint32_t rows = (cnt + BLOCK - 1) / BLOCK;
+  const uint32_t base = wid * kWave * rows;
+  const uint32_t left = base < cnt ? min(cnt - base, kWave * rows) : 0u;
+  auto valid = [&](int j) { return (uint32_t)j * kWave + lane < left; };
+  auto word = [&](const Elem<EW>& e) { return order_bits<K, MODE>(elem_key<K, EW>(e)); };
+  Elem<EW>* s_el = reinterpret_cast<Elem<EW>*>(s_part);
+  Elem<EW> el[IPT];
+  if (tid < 2) s_diff[tid] = 0;
+  __syncthreads();
+  const auto first = order_bits<K, MODE>(load_key<K, EW>(rp, start));
+  uint32_t xlo = 0, xhi = 0;
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    if (!valid(j)) continue;
+    el[j] = load_elem<K, EW>(rp, (size_t)start + base + (uint32_t)j * kWave + lane);
+    const auto x = word(el[j]) ^ first;
+    xlo |= (uint32_t)x;
+    if constexpr (sizeof(K) == 8) xhi |= (uint32_t)(x >> 32);
+  }
+  if (xlo) atomicOr(&s_diff[0], xlo);
+  if (xhi) atomicOr(&s_diff[1], xhi);
+  __syncthreads();
+  const uint32_t diff[2] = {s_diff[0], s_diff[1]};
+  auto varies = [&](uint32_t p) { return ((diff[p / 4] >> (8 * (p & 3))) & 0xffu) != 0; };
+  // The lowest of the DIGITS highest varying digits, and whether any below varies.
+  uint32_t low = top;
+  bool below_varies = false;
+  for (uint32_t p = top, left_out = DIGITS; p-- > 0;) {
+    if (!varies(p)) continue;
+    if (left_out == 0) {
+      below_varies = true;
+      break;
+    }
+    --left_out;
+    low = p;
+  }
+  const uint64_t lt = lanemask_lt();
+  bool in_lds = false;
+  for (uint32_t from = low;;) {
+    for (uint32_t p = from; p < top; ++p) {
+      if (!varies(p)) continue;
+      if (in_lds) {
+#pragma unroll
+        for (int j = 0; j < IPT; ++j)
+          if (valid(j)) el[j] = s_el[base + (uint32_t)j * kWave + lane];
+      }
+      for (uint32_t i = tid; i < NW * kRadixBins / 2; i += BLOCK)
+        reinterpret_cast<uint32_t*>(&s_hist[0][0])[i] = 0;
+      __syncthreads();
+      uint32_t rank[IPT];
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) {
+        if ((uint32_t)j >= rows) break;
+        asm volatile("" : "+v"(el[j].w[0]));
+        const uint32_t d = (uint32_t)(word(el[j]) >> (8 * p)) & 0xffu;
+        const uint64_t peers = match_digit<8>(d, valid(j));
+        uint32_t before = 0;
+        if (valid(j)) before = s_hist[wid][d];
+        const uint32_t below = (uint32_t)__builtin_popcountll(peers & lt);
+        if (valid(j) && below == 0)
+          s_hist[wid][d] = (uint16_t)(before + (uint32_t)__builtin_popcountll(peers));
+        rank[j] = before + below;
+      }
+      __syncthreads();
+      uint32_t sum = 0, incl = 0;
+      if (digit_thread) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          const uint32_t c = s_hist[w][tid];
+          s_hist[w][tid] = (uint16_t)sum;
+          sum += c;
+        }
+        incl = wave_inclusive_scan<uint32_t, OP_ADD>(sum);
+        if (lane == 63) s_wsum[wid] = incl;
+      }
+      __syncthreads();
+      if (digit_thread) {
+        uint32_t woff = 0;
+        for (uint32_t k = 0; k < wid; ++k) woff += s_wsum[k];
+        s_start[tid] = woff + incl - sum;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) {
+        if (!valid(j)) continue;
+        asm volatile("" : "+v"(el[j].w[0]));
+        const uint32_t d = (uint32_t)(word(el[j]) >> (8 * p)) & 0xffu;
+        s_el[s_start[d] + s_hist[wid][d] + rank[j]] = el[j];
+      }
+      in_lds = true;
+      __syncthreads();
+    }
+    if (from == 0 || !below_varies) break;
+    // Repair: thread t looks at positions t + q * BLOCK. An element below its
+    // predecessor is in one run with it; the first such one of a run speaks
+    // for the run. (Prefixes do not change while runs are put in order.)
+    const uint32_t shift = 8 * low;
+    auto at = [&](uint32_t i) { return word(s_el[i]); };
+    if (tid == 0) s_diff[0] = 0;
+    uint32_t mine = 0;
+#pragma unroll 1
+    for (uint32_t i = tid, q = 0; i < cnt; i += BLOCK, ++q)
+      if (i > 0 && at(i - 1) > at(i)) mine |= 1u << q;
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t left_out = mine; left_out; left_out &= left_out - 1) {
+      const uint32_t q = (uint32_t)__builtin_ctz(left_out), i = tid + q * BLOCK;
+      const auto prefix = at(i) >> shift;
+      uint32_t b = i - 1, e = i + 1;
+      bool first = true;
+      while (b > 0 && i - b < kLocalRun && at(b - 1) >> shift == prefix) {
+        if (at(b - 1) > at(b)) first = false;
+        --b;
+      }
+      while (e < cnt && e - b <= kLocalRun && at(e) >> shift == prefix) ++e;
+      if (i - b >= kLocalRun || e - b > kLocalRun) s_diff[0] = 1;
+      if (!first) mine &= ~(1u << q);
+    }
+    __syncthreads();
+    if (s_diff[0]) {
+      from = 0;
+      continue;
+    }
+#pragma unroll 1
+    for (; mine; mine &= mine - 1) {
+      const uint32_t i = tid + (uint32_t)__builtin_ctz(mine) * BLOCK;
+      const auto prefix = at(i) >> shift;
+      uint32_t b = i - 1, e = i + 1;
+      while (b > 0 && at(b - 1) >> shift == prefix) --b;
+      while (e < cnt && at(e) >> shift == prefix) ++e;
+      for (uint32_t k = b + 1; k < e; ++k) {
+        const Elem<EW> x = s_el[k];
+        uint32_t h = k;
+        for (; h > b && at(h - 1) > word(x); --h) s_el[h] = s_el[h - 1];
+        s_el[h] = x;
+      }
+    }
+    __syncthreads();
+    break;
+  }
+  if (!in_lds) {
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+      if (valid(j)) store_elem<K, EW>(rp, (size_t)start + base + (uint32_t)j * kWave + lane, el[j]);
+    return;
+  }
+  for (uint32_t i = tid; i < cnt; i += BLOCK) store_elem<K, EW>(rp, (size_t)start + i, s_el[i]);
 }
 
 }  // namespace msv

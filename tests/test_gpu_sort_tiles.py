@@ -1,5 +1,6 @@
-"""GPU: sorts at the edges of the radix passes' tiles, every element width, bit-exact
-and stable vs numpy's stable sort (integer keys) and the oracle (floats)."""
+"""GPU: sorts at the edges of the radix passes' tiles and of the local sort's range,
+every element width, bit-exact and stable vs numpy's stable sort (integer keys)
+and the oracle (floats)."""
 import numpy as np
 import pytest
 
@@ -8,7 +9,8 @@ import oracle
 
 pytestmark = pytest.mark.gpu
 
-EDGES = [8191, 8192, 8193, 10239, 10240, 10241, 3 * 8192 + 5, 41 * 10240 - 1]
+EDGES = [1, 1024, 1025, 4096, 4097, 5120, 5121, 8191, 8192, 8193, 10239, 10240, 10241, 3 * 8192 + 5,
+         (1 << 18) + 1, 41 * 10240 - 1]
 
 
 def _keys(dtype, n, rng, few):
@@ -36,3 +38,30 @@ def test_sort_tile_edges(exec_, dtype, value):
             v, s = m.vector.radix_sort_by_key(exec_, dk, exec_.to_device(np.arange(n, dtype=value)), return_keys=True)
             assert np.array_equal(exec_.to_host(v), order.astype(value)), (n, few)
             assert np.array_equal(exec_.to_host(s), k[order]), (n, few)
+
+
+@pytest.mark.parametrize("dtype,value", [(np.uint32, np.uint32), (np.uint64, np.uint32), (np.uint64, np.uint64),
+                                         (np.uint32, None)])
+@pytest.mark.parametrize("spread", ["uniform", "top constant", "one digit full", "two digits"])
+def test_sort_local_range(exec_, dtype, value, spread):
+    """One pass and local sorts, and inputs whose highest varying digit rules them out."""
+    rng = np.random.default_rng(23)
+    bits = 8 * np.dtype(dtype).itemsize
+    for n in (9000, 100_003, 900_001, 1_500_000):
+        k = rng.integers(0, 2**bits, n, dtype=np.uint64)
+        if spread == "top constant":
+            k &= np.uint64(2 ** (bits - 8) - 1)
+        elif spread == "one digit full":  # a run too long for a block
+            k[rng.random(n) < 0.5] &= np.uint64(2 ** (bits - 8) - 1)
+        elif spread == "two digits":
+            k &= np.uint64(0xFF | 0xFF << (bits - 8))
+        k = k.astype(dtype)
+        order = np.argsort(k, kind="stable")
+        dk = exec_.to_device(k)
+        if value is None:
+            assert np.array_equal(exec_.to_host(m.vector.sort(exec_, dk, m.op.Less)), k[order]), n
+            assert np.array_equal(exec_.to_host(m.vector.sort(exec_, dk, m.op.Greater)), k[order][::-1]), n
+            continue
+        v, s = m.vector.radix_sort_by_key(exec_, dk, exec_.to_device(np.arange(n, dtype=value)), return_keys=True)
+        assert np.array_equal(exec_.to_host(v), order.astype(value)), n
+        assert np.array_equal(exec_.to_host(s), k[order]), n
