@@ -725,9 +725,11 @@ msv_status run_jobs(Ctx& c, const msv_job* jobs, uint32_t count) {
     if (job_is_small(jobs[i])) small.push_back(jobs[i]);
     else large.push_back(i);
   }
+  std::vector<char> host;
+  bool forked = false;
   if (!small.empty()) {
     const uint32_t cap = (uint32_t)small.size();
-    std::vector<char> host(batch_table_bytes(cap));
+    host.resize(batch_table_bytes(cap));
     uint32_t mask = 0;
     MSV_TRY(batch_table_fill(c, small.data(), cap, nullptr, 0, cap, host.data(), &mask));
     char* dev = (char*)c.scratch(host.size());
@@ -740,13 +742,49 @@ msv_status run_jobs(Ctx& c, const msv_job* jobs, uint32_t count) {
     if (!src) return MSV_ERR_OUT_OF_MEMORY;
     MSV_HIP(hipMemcpyAsync(dev, src, host.size(), hipMemcpyHostToDevice, c.stream()));
     const BatchHeader* hh = (const BatchHeader*)host.data();
-    MSV_TRY(launch_families(c.stream(), dev, mask, [&](int f) {
+    auto grid = [&](int f) {
       const uint32_t n = hh->start[f + 1] - hh->start[f];
       return std::min<uint32_t>(n, family_grid(ex, f, family_choice(ex, host.data(), f)));
-    }));
+    };
+    // A family's launch lasts as long as its longest job in one block (a sort
+    // of 2^15 u64 keys 600 us, u32 170 us) and leaves most of the chip idle, so
+    // the longest sorts run beside the rest: on the second stream, those of
+    // 8-byte keys, or of 4-byte keys when there are none. 96 jobs of every
+    // kind and type, 2^10..2^17 elements: 1049 -> 622 us. The fork and the join
+    // cost the host some 50 us, so shorter sorts (see kAsideMin) stay in line
+    // (128 jobs of at most 2^13 elements: 480 us in line, 535 forked).
+    constexpr uint32_t kWide = 0x70, kNarrow = 0x0e;
+    constexpr uint32_t kAsideMin = 1u << 14;  // 4-byte keys; half as many of 8 bytes
+    const uint32_t families = (mask & kWide) ? (mask & kWide) : (mask & kNarrow);
+    uint32_t longest = 0;
+    for (const msv_job& j : small)
+      if (j.kind == MSV_JOB_SORT_BY_KEY && (families >> (1 + sort_class(j)) & 1u))
+        longest = std::max(longest, j.n);
+    const uint32_t aside = longest >= (families & kWide ? kAsideMin / 2 : kAsideMin) ? families : 0u;
+    if (aside && (aside != mask || !large.empty())) {
+      hipStream_t aux = c.fork();
+      if (!aux) return MSV_ERR_LAUNCH;
+      forked = true;
+      const msv_status s = launch_families(aux, dev, aside, grid);
+      if (s != MSV_OK) {
+        (void)c.join();
+        return s;
+      }
+      mask &= ~aside;
+    }
+    const msv_status s = launch_families(c.stream(), dev, mask, grid);
+    if (s != MSV_OK) {
+      if (forked) (void)c.join();
+      return s;
+    }
   }
-  for (uint32_t i : large) MSV_TRY(large_job(c, jobs[i]));
-  return MSV_OK;
+  msv_status s = MSV_OK;
+  for (size_t k = 0; k < large.size() && s == MSV_OK; ++k) s = large_job(c, jobs[large[k]]);
+  if (forked) {
+    const msv_status joined = c.join();
+    if (s == MSV_OK) s = joined;
+  }
+  return s;
 }
 
 msv_status run_jobs_plain(Ctx& c, const msv_job* jobs, uint32_t count) {
