@@ -133,28 +133,68 @@ static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, ui
     const uint32_t hist_blocks = min(div_up(n, 256u * 16u), (uint32_t)c.num_cus() * 8u);
     hipLaunchKernelGGL((radix_hist_kernel<K, MODE, 256>), dim3(hist_blocks), dim3(256), 0,
                        c.stream(), (const K*)keys, n, hist);
-    hipLaunchKernelGGL((radix_onesweep_plan_kernel<P>), dim3(1), dim3(kRadixBins), 0, c.stream(), q, n);
-    MSV_HIP(hipGetLastError());
+    // Long sorts of 8-byte keys stop at a digit that a sample chooses, repair
+    // what that left, and start over with every digit when that was too much.
+    const bool repair = P == 8 && n > kRepairMin && q.local_max == 0;
+    RadixRepair* rep = nullptr;
+    if constexpr (P == 8) {
+      if (repair) {
+        rep = (RadixRepair*)c.scratch(sizeof(RadixRepair));
+        if (!rep) return MSV_ERR_OUT_OF_MEMORY;
+        q.rep = rep;
+        hipLaunchKernelGGL((radix_sample_kernel<K, MODE>), dim3(1), dim3(1024), 0, c.stream(),
+                           (const K*)keys, n, hist, rep);
+      }
+    }
     constexpr int OBLOCK = radix_onesweep_block<EW>();
     constexpr int OIPT = radix_onesweep_ipt<EW>();
     const int ipt = n <= kRadixSmall ? 2 : (n <= kRadixMiddle ? 6 : OIPT);
     const uint32_t otiles = div_up(n, (uint32_t)OBLOCK * ipt);
     // Slot p runs the p-th pass of the plan; passes it leaves out end at once.
-    for (int p = 0; p < P; ++p) {
-      uint64_t *counter, *status;
-      uint32_t gen;
-      MSV_TRY(c.lookback((size_t)otiles * kRadixBins, &counter, &status, &gen));
-      auto pass = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(otiles), dim3(OBLOCK), 0, c.stream(), table, p, q.gbase,
-                           q.tile_counters, status, gen, n);
-      };
-      if (ipt == 2) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 2>);
-      else if (ipt == 6) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 6>);
-      else pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, OIPT>);
-      if (p == 0 && q.local_max)
-        hipLaunchKernelGGL((radix_local_kernel<K, MODE, EW, 1024, LIPT, 2>), dim3(kRadixBins),
-                           dim3(1024), 0, c.stream(), q.local, q.gbase, RadixPass{}, n);
+    auto passes = [&]() -> msv_status {
+      hipLaunchKernelGGL((radix_onesweep_plan_kernel<P>), dim3(1), dim3(kRadixBins), 0, c.stream(), q, n);
       MSV_HIP(hipGetLastError());
+      for (int p = 0; p < P; ++p) {
+        uint64_t *counter, *status;
+        uint32_t gen;
+        MSV_TRY(c.lookback((size_t)otiles * kRadixBins, &counter, &status, &gen));
+        auto pass = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, dim3(otiles), dim3(OBLOCK), 0, c.stream(), table, p, q.gbase,
+                             q.tile_counters, status, gen, n);
+        };
+        if (ipt == 2) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 2>);
+        else if (ipt == 6) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 6>);
+        else pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, OIPT>);
+        if (p == 0 && q.local_max)
+          hipLaunchKernelGGL((radix_local_kernel<K, MODE, EW, 1024, LIPT, 2>), dim3(kRadixBins),
+                             dim3(1024), 0, c.stream(), q.local, q.gbase, RadixPass{}, n);
+        MSV_HIP(hipGetLastError());
+      }
+      return MSV_OK;
+    };
+    MSV_TRY(passes());
+    if constexpr (P == 8) {
+      if (repair) {
+        // The element buffers are free by now. The first holds the listed runs,
+        // their counts and a mark per element (less than n words in all), the second the
+        // places that long runs move through.
+        const uint32_t chunk = div_up(div_up(n, 8u * (uint32_t)c.num_cus()), 2048u) * 2048u;
+        const uint32_t blocks = div_up(n, chunk), words = div_up(n, 32u);
+        uint32_t* const list = (uint32_t*)aos0;
+        uint32_t* const counts = list + (size_t)blocks * (chunk / 2 + 1);
+        uint32_t* const marks = counts + blocks;
+        K* const out = (K*)out_k;
+        hipLaunchKernelGGL(radix_repair_clear_kernel, dim3(c.num_cus()), dim3(256), 0, c.stream(), rep,
+                           marks, words);
+        hipLaunchKernelGGL((radix_repair_find_kernel<K, MODE>), dim3(blocks), dim3(256), 0, c.stream(),
+                           (const K*)out, n, chunk, ((uintptr_t)out & 15u) == 0, rep, marks, list, counts);
+        hipLaunchKernelGGL((radix_repair_kernel<K, MODE, VS / 4>), dim3(blocks), dim3(1024), 0, c.stream(),
+                           out, (uint32_t*)out_v, (K*)aos1, (uint32_t*)((char*)aos1 + (size_t)n * sizeof(K)),
+                           n, chunk, rep, list, counts);
+        MSV_HIP(hipGetLastError());
+        q.redo = true;
+        return passes();
+      }
     }
     return MSV_OK;
   }

@@ -526,6 +526,12 @@ struct RadixLocal {
   RadixPass pass;  // its source and destination
 };
 
+// How a long sort of 8-byte keys goes (9).
+struct RadixRepair {
+  uint32_t low;   // passes run from this digit; 0: all of them do
+  uint32_t redo;  // the repair gave up: every digit's pass runs
+};
+
 // 6. Onesweep plan (one block of 256 threads): the exclusive scan of every
 //    digit position's histogram (the global start of each digit in that
 //    pass), which positions need a pass (a position whose histogram puts all
@@ -544,6 +550,8 @@ struct RadixPlan {
   uint32_t* tile_counters;  // [P]
   RadixLocal* local;
   uint32_t local_max;
+  const RadixRepair* rep;   // where the passes start (null: at digit 0)
+  bool redo;                // the second plan, after a repair
   const void *in_k, *in_v;
   void *out_k, *out_v, *aos0, *aos1;
   size_t vofs;
@@ -574,7 +582,12 @@ __global__ __launch_bounds__(kRadixBins) void radix_onesweep_plan_kernel(RadixPl
   }
   if (t != 0) return;
   int active = 0, top = 0;
-  for (int p = 0; p < P; ++p) {
+  const int low = q.rep && !q.redo ? (int)q.rep->low : 0;
+  if (q.redo && q.rep->redo == 0) {
+    for (int p = 0; p < P; ++p) q.table[p].active = 0;
+    return;
+  }
+  for (int p = low; p < P; ++p) {
     if (s_trivial[p]) continue;
     ++active;
     top = p;
@@ -590,7 +603,7 @@ __global__ __launch_bounds__(kRadixBins) void radix_onesweep_plan_kernel(RadixPl
   const int passes = use_local || force_last ? 1 : active;
   int j = 0;
   for (int p = 0; p < P; ++p) {
-    if (use_local ? p != top : (force_last ? p != P - 1 : s_trivial[p] != 0)) continue;
+    if (use_local ? p != top : (force_last ? p != P - 1 : p < low || s_trivial[p] != 0)) continue;
     const bool to_out = j == passes - 1 && !use_local;
     char* src = (char*)(((j - 1) & 1) ? q.aos1 : q.aos0);
     char* dst = (char*)((j & 1) ? q.aos1 : q.aos0);
@@ -1026,6 +1039,363 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_local_kernel(
     return;
   }
   for (uint32_t i = tid; i < cnt; i += BLOCK) store_elem<K, EW>(rp, (size_t)start + i, s_el[i]);
+}
+
+// 9. Long sorts of 8-byte keys by their highest digits only. n keys that are
+//    spread at all differ from most others in not many more than log2(n) of
+//    their highest varying bits, so the passes stop at digit `low` and a repair
+//    orders what they left equal: a pass moves every element once (24 bytes of
+//    traffic for u64 + u32), the look of the repair reads 8 of them.
+//     * radix_sample_kernel (one block) chooses low: at least log2(n) + 4 bits
+//       of varying digits (then n / 32 pairs of random keys agree above it, half
+//       of them in the wrong order), one digit more when some key may hold over
+//       1/64 of the input (its run would be long to repair), and lower while
+//       two different keys of a sample of kSample agree above it.
+//     * radix_repair_find_kernel lists the runs of equal digits that have an
+//       element below its predecessor, radix_repair_kernel orders them.
+//     * When that is too much (many runs, or long ones: a run that holds a good
+//       part of the input and few keys that differ), the passes start over with
+//       every digit. Any input is sorted; the choice only decides how soon.
+//    2^27 u64 + u32, eight passes -> now: uniform 7.0 -> 4.42 ms (four passes),
+//    zipf with hot keys 7.2 -> 5.09 ms (five); the look 0.23 ms (4.7 TB/s; with
+//    64 consecutive bytes per thread 0.46), ordering the runs 5 us, the sample
+//    26 us, the passes left out 14 us each. 2^25 with half the keys equal and
+//    1e-5 of them off in the low digits, which starts over: 2.3 -> 3.5 ms.
+constexpr uint32_t kRepairMin = 1u << 21;   // keys: 2^21 + 1 uniform u64 + u32 214 -> 184 us, 2^23 522 -> 379
+constexpr uint32_t kRepairRun = 32;         // elements one thread orders
+constexpr uint32_t kRepairLong = 1u << 15;  // elements of a run that a block orders,
+constexpr uint32_t kRepairSum = 1u << 16;   // and of all that one block does,
+constexpr uint32_t kRepairLongs = 64;       // and how many
+constexpr uint32_t kSample = 8192;
+
+template <typename K, int MODE>
+__global__ __launch_bounds__(1024) void radix_sample_kernel(const K* __restrict__ keys, uint32_t n,
+                                                            const uint32_t* __restrict__ hist,
+                                                            RadixRepair* __restrict__ rep) {
+  constexpr int P = (int)sizeof(K);
+  constexpr uint32_t SLOTS = 2 * kSample;
+  __shared__ uint64_t s_word[kSample];
+  __shared__ uint32_t s_slot[SLOTS];
+  __shared__ uint32_t s_most[P], s_clash;
+  const uint32_t tid = threadIdx.x;
+  if (tid < (uint32_t)P) s_most[tid] = 0;
+  __syncthreads();
+  for (uint32_t i = tid; i < (uint32_t)P * kRadixBins; i += 1024) atomicMax(&s_most[i / kRadixBins], hist[i]);
+  // Positions spread by an odd multiplier.
+  for (uint32_t i = tid; i < kSample; i += 1024)
+    s_word[i] = (uint64_t)order_bits<K, MODE>(keys[(uint64_t)(i * 2654435761u) * n >> 32]);
+  __syncthreads();
+  uint32_t bits = 4, hot = n;
+  while ((1ull << (bits - 4)) < n) ++bits;
+  int want = (int)(bits + 7) / 8;
+  for (int p = 0; p < P; ++p) hot = min(hot, s_most[p]);
+  if (hot > n / 64) ++want;
+  int low = P;
+  for (int p = P; p-- > 0 && want > 0;) {
+    low = p;
+    want -= s_most[p] < n ? 1 : 0;
+  }
+  for (; low > 0; --low) {
+    if (s_most[low - 1] == n) continue;  // a constant digit needs no look
+    for (uint32_t i = tid; i < SLOTS; i += 1024) s_slot[i] = 0;
+    if (tid == 0) s_clash = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < kSample; i += 1024) {
+      const uint64_t prefix = s_word[i] >> (8 * low);
+      uint32_t h = (uint32_t)((prefix * 0x9E3779B97F4A7C15ull) >> 40) % SLOTS;
+      for (;;) {
+        const uint32_t other = atomicCAS(&s_slot[h], 0u, i + 1);
+        if (other == 0) break;
+        const uint64_t w = s_word[other - 1];
+        if (w >> (8 * low) == prefix) {
+          if (w != s_word[i]) s_clash = 1;
+          break;
+        }
+        h = (h + 1) % SLOTS;
+      }
+    }
+    __syncthreads();
+    const bool clash = s_clash != 0;
+    __syncthreads();
+    if (!clash) break;
+  }
+  if (tid == 0) {
+    bool below = false;
+    for (int p = 0; p < low; ++p) below = below || s_most[p] < n;
+    rep->low = below ? (uint32_t)low : 0u;
+    rep->redo = 0;
+  }
+}
+
+// Zeroes the marks (a bit per element).
+static __global__ void radix_repair_clear_kernel(const RadixRepair* __restrict__ rep,
+                                                 uint32_t* __restrict__ marks, uint32_t words) {
+  if (rep->low == 0) return;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) marks[i] = 0;
+}
+
+// The end of the run of equal words >> shift that i is in (the first index
+// after it), or its start.
+template <typename K, int MODE>
+__device__ inline uint32_t run_end(const K* __restrict__ keys, uint32_t n, uint32_t i, uint32_t shift) {
+  const auto prefix = order_bits<K, MODE>(keys[i]) >> shift;
+  uint64_t step = 1, in = i;
+  while (in + step < n && order_bits<K, MODE>(keys[in + step]) >> shift == prefix) {
+    in += step;
+    step *= 2;
+  }
+  uint64_t lo = in + 1, hi = min((uint64_t)n, in + step);
+  while (lo < hi) {
+    const uint64_t mid = (lo + hi) / 2;
+    if (order_bits<K, MODE>(keys[mid]) >> shift == prefix) lo = mid + 1;
+    else hi = mid;
+  }
+  return (uint32_t)lo;
+}
+template <typename K, int MODE>
+__device__ inline uint32_t run_start(const K* __restrict__ keys, uint32_t i, uint32_t shift) {
+  const auto prefix = order_bits<K, MODE>(keys[i]) >> shift;
+  int64_t step = 1, in = i;
+  while (in - step >= 0 && order_bits<K, MODE>(keys[in - step]) >> shift == prefix) {
+    in -= step;
+    step *= 2;
+  }
+  int64_t lo = in - step < 0 ? 0 : in - step, hi = in;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) / 2;
+    if (order_bits<K, MODE>(keys[mid]) >> shift == prefix) hi = mid;
+    else lo = mid + 1;
+  }
+  return (uint32_t)lo;
+}
+
+// Block b looks at elements [b * chunk, (b + 1) * chunk) and lists runs in
+// list[b * (chunk / 2 + 1)...] (each has an element below its predecessor in
+// the chunk, so there are no more), counts[b] of them. chunk is a multiple of
+// 2048.
+template <typename K, int MODE>
+__global__ __launch_bounds__(256) void radix_repair_find_kernel(const K* __restrict__ keys, uint32_t n,
+                                                                uint32_t chunk, bool aligned,
+                                                                RadixRepair* __restrict__ rep,
+                                                                uint32_t* __restrict__ marks,
+                                                                uint32_t* __restrict__ list,
+                                                                uint32_t* __restrict__ counts) {
+  static_assert(sizeof(K) == 8, "8-byte keys");
+  constexpr int ROWS = 4;  // rows of 256 threads x 2 keys
+  __shared__ uint32_t s_count;
+  if (rep->low == 0) return;
+  const uint32_t shift = 8 * rep->low, lane = threadIdx.x & 63u;
+  list += (size_t)blockIdx.x * (chunk / 2 + 1);
+  if (threadIdx.x == 0) s_count = 0;
+  __syncthreads();
+  const size_t end = min((size_t)n, (size_t)(blockIdx.x + 1) * chunk);
+  for (size_t base = (size_t)blockIdx.x * chunk; base < end; base += 256 * 2 * ROWS) {
+    uint64_t w[ROWS][2], left[ROWS];
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+      const size_t i = base + (j * 256 + threadIdx.x) * 2;
+      K x[2] = {};
+      if (aligned && i + 2 <= n) {
+        const uint4 q = *reinterpret_cast<const uint4*>(keys + i);
+        x[0] = bit_cast<K>((uint64_t)q.y << 32 | q.x);
+        x[1] = bit_cast<K>((uint64_t)q.w << 32 | q.z);
+      } else {
+        if (i < n) x[0] = keys[i];
+        if (i + 1 < n) x[1] = keys[i + 1];
+      }
+      if (lane == 0 && i < n) left[j] = order_bits<K, MODE>(keys[i > 0 ? i - 1 : 0]);
+      w[j][0] = order_bits<K, MODE>(x[0]);
+      w[j][1] = order_bits<K, MODE>(x[1]);
+    }
+#pragma unroll
+    for (int h = 0; h < 2 * ROWS; ++h) {
+      const int j = h / 2, k = h % 2;
+      const uint64_t word = w[j][k];
+      const uint64_t up = __shfl_up(w[j][1], 1);
+      const uint64_t before = k == 1 ? w[j][0] : (lane == 0 ? left[j] : up);
+      const size_t at = base + (j * 256 + threadIdx.x) * 2 + k;
+      const uint32_t i = (uint32_t)at;
+      if (at < n && before > word) {
+        // The run's first such element lists it. One that sees neither the
+        // run's start nor another before it within kRepairRun elements may be
+        // the first; the mark at the start decides.
+        const uint64_t prefix = word >> shift;
+        uint64_t cur = before;
+        uint32_t s = i - 1;
+        bool first = true;
+        while (s > 0) {
+          const uint64_t p = order_bits<K, MODE>(keys[s - 1]);
+          if (p >> shift != prefix) break;
+          if (p > cur) {
+            first = false;
+            break;
+          }
+          if (i - s >= kRepairRun) {
+            s = run_start<K, MODE>(keys, s, shift);
+            break;
+          }
+          cur = p;
+          --s;
+        }
+        if (first && !(atomicOr(&marks[s / 32], 1u << (s % 32)) >> (s % 32) & 1u)) list[atomicAdd(&s_count, 1u)] = s;
+      }
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) counts[blockIdx.x] = s_count;
+}
+
+// Block b orders the runs that block b of the find listed: a thread each run of
+// up to kRepairRun elements by insertion, the block each longer one by stable
+// LSD passes over its varying digits below low, 1024 elements at a time,
+// between the run and the same places of tmp. What is too much for that leaves
+// redo set. VW: 4-byte words of a value (0: none).
+template <typename K, int MODE, int VW>
+__global__ __launch_bounds__(1024) void radix_repair_kernel(K* keys, uint32_t* vals, K* tmp_k,
+                                                            uint32_t* tmp_v, uint32_t n, uint32_t chunk,
+                                                            RadixRepair* rep,
+                                                            const uint32_t* __restrict__ list,
+                                                            const uint32_t* __restrict__ counts) {
+  constexpr int NW = 1024 / kWave;
+  __shared__ uint32_t s_base[kRadixBins];
+  __shared__ uint16_t s_hist[NW][kRadixBins];
+  __shared__ uint32_t s_wsum[kRadixBins / kWave], s_diff[2];
+  __shared__ uint32_t s_start[kRepairLongs], s_end[kRepairLongs], s_longs, s_sum;
+  const uint32_t low = rep->low;
+  if (low == 0) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid / 64u, shift = 8 * low;
+  const uint32_t runs = counts[blockIdx.x];
+  if (runs > chunk / 8) {
+    if (tid == 0) rep->redo = 1;
+    return;
+  }
+  list += (size_t)blockIdx.x * (chunk / 2 + 1);
+  if (tid == 0) s_longs = s_sum = 0;
+  __syncthreads();
+  for (uint32_t r = tid; r < runs; r += 1024) {
+    const uint32_t s = list[r];
+    const auto prefix = order_bits<K, MODE>(keys[s]) >> shift;
+    uint32_t e = s + 1;
+    while (e < n && e - s <= kRepairRun && order_bits<K, MODE>(keys[e]) >> shift == prefix) ++e;
+    if (e - s > kRepairRun) {
+      const uint32_t j = atomicAdd(&s_longs, 1u);
+      if (j < kRepairLongs) {
+        e = run_end<K, MODE>(keys, n, s, shift);
+        s_start[j] = s;
+        s_end[j] = e;
+        atomicAdd(&s_sum, min(e - s, 2 * kRepairSum));
+        if (e - s > kRepairLong) atomicAdd(&s_sum, kRepairSum);
+      }
+      continue;
+    }
+    for (uint32_t k = s + 1; k < e; ++k) {
+      const K x = keys[k];
+      const auto w = order_bits<K, MODE>(x);
+      uint32_t h = k;
+      if (order_bits<K, MODE>(keys[h - 1]) <= w) continue;
+      uint32_t v[VW > 0 ? VW : 1];
+#pragma unroll
+      for (int c = 0; c < VW; ++c) v[c] = vals[(size_t)k * VW + c];
+      for (; h > s && order_bits<K, MODE>(keys[h - 1]) > w; --h) {
+        keys[h] = keys[h - 1];
+#pragma unroll
+        for (int c = 0; c < VW; ++c) vals[(size_t)h * VW + c] = vals[(size_t)(h - 1) * VW + c];
+      }
+      keys[h] = x;
+#pragma unroll
+      for (int c = 0; c < VW; ++c) vals[(size_t)h * VW + c] = v[c];
+    }
+  }
+  __syncthreads();
+  const uint32_t longs = s_longs;
+  if (longs > kRepairLongs || s_sum > kRepairSum) {
+    if (tid == 0) rep->redo = 1;
+    return;
+  }
+  const bool digit_thread = tid < (uint32_t)kRadixBins;
+  const uint64_t lt = lanemask_lt();
+  for (uint32_t r = 0; r < longs; ++r) {
+    const uint32_t s = s_start[r], e = s_end[r];
+    __syncthreads();
+    if (tid < 2) s_diff[tid] = 0;
+    __syncthreads();
+    const uint64_t word = order_bits<K, MODE>(keys[s]);
+    uint64_t x = 0;
+    for (uint32_t i = s + tid; i < e; i += 1024) x |= order_bits<K, MODE>(keys[i]) ^ word;
+    if (x) {
+      atomicOr(&s_diff[0], (uint32_t)x);
+      atomicOr(&s_diff[1], (uint32_t)(x >> 32));
+    }
+    __syncthreads();
+    const uint64_t diff = (uint64_t)s_diff[1] << 32 | s_diff[0];
+    K *src_k = keys, *dst_k = tmp_k;
+    uint32_t *src_v = vals, *dst_v = tmp_v;
+    for (uint32_t p = 0; p < low; ++p) {
+      if ((diff >> (8 * p) & 0xffu) == 0) continue;
+      auto digit = [&](K k) { return (uint32_t)(order_bits<K, MODE>(k) >> (8 * p)) & 0xffu; };
+      if (digit_thread) s_base[tid] = 0;
+      __syncthreads();
+      for (uint32_t i = s + tid; i < e; i += 1024) atomicAdd(&s_base[digit(src_k[i])], 1u);
+      __syncthreads();
+      uint32_t c = 0, incl = 0;
+      if (digit_thread) {
+        c = s_base[tid];
+        incl = wave_inclusive_scan<uint32_t, OP_ADD>(c);
+        if (lane == 63) s_wsum[wid] = incl;
+      }
+      __syncthreads();
+      if (digit_thread) {
+        uint32_t off = s + incl - c;
+        for (uint32_t w = 0; w < wid; ++w) off += s_wsum[w];
+        s_base[tid] = off;
+      }
+      for (uint32_t c0 = s; c0 < e; c0 += 1024) {
+        for (uint32_t i = tid; i < NW * kRadixBins / 2; i += 1024)
+          reinterpret_cast<uint32_t*>(&s_hist[0][0])[i] = 0;
+        __syncthreads();
+        const uint32_t i = c0 + tid;
+        const bool valid = i < e;
+        const K k = src_k[valid ? i : s];
+        const uint32_t d = digit(k);
+        const uint64_t peers = match_digit<8>(d, valid);
+        const uint32_t below = (uint32_t)__builtin_popcountll(peers & lt);
+        if (valid && below == 0) s_hist[wid][d] = (uint16_t)__builtin_popcountll(peers);
+        __syncthreads();
+        uint32_t total = 0;
+        if (digit_thread) {
+#pragma unroll
+          for (int w = 0; w < NW; ++w) {
+            const uint32_t h = s_hist[w][tid];
+            s_hist[w][tid] = (uint16_t)total;
+            total += h;
+          }
+        }
+        __syncthreads();
+        if (valid) {
+          const uint32_t o = s_base[d] + s_hist[wid][d] + below;
+          dst_k[o] = k;
+#pragma unroll
+          for (int q = 0; q < VW; ++q) dst_v[(size_t)o * VW + q] = src_v[(size_t)i * VW + q];
+        }
+        __syncthreads();
+        if (digit_thread) s_base[tid] += total;
+      }
+      __syncthreads();
+      K* const tk = src_k;
+      src_k = dst_k;
+      dst_k = tk;
+      uint32_t* const tv = src_v;
+      src_v = dst_v;
+      dst_v = tv;
+    }
+    if (src_k != keys) {
+      for (uint32_t i = s + tid; i < e; i += 1024) {
+        keys[i] = tmp_k[i];
+#pragma unroll
+        for (int q = 0; q < VW; ++q) vals[(size_t)i * VW + q] = tmp_v[(size_t)i * VW + q];
+      }
+    }
+  }
 }
 
 }  // namespace msv

@@ -65,3 +65,43 @@ def test_sort_local_range(exec_, dtype, value, spread):
         v, s = m.vector.radix_sort_by_key(exec_, dk, exec_.to_device(np.arange(n, dtype=value)), return_keys=True)
         assert np.array_equal(exec_.to_host(v), order.astype(value)), n
         assert np.array_equal(exec_.to_host(s), k[order]), n
+
+
+@pytest.mark.parametrize("dtype,value", [(np.uint64, np.uint32), (np.int64, None), (np.float64, np.uint64)])
+@pytest.mark.parametrize("spread", ["uniform", "sorted", "pairs", "runs", "half", "one digit"])
+def test_sort_high_digits_and_repair(exec_, dtype, value, spread):
+    """Long sorts of 8-byte keys: nothing, pairs, runs of some hundred elements and a
+    run of half the keys that differ only in the digits the first passes leave out."""
+    n = (1 << 23) + 4099
+    rng = np.random.default_rng(41)
+    few = rng.random(n) < (1e-4 if spread == "runs" else 1e-5)
+    low = rng.integers(0, 1 << 16, n, dtype=np.uint64)
+    if spread == "pairs":  # one pair of keys in three shares all but 16 bits
+        k = rng.permutation(rng.integers(0, 2**46, n, dtype=np.uint64).repeat(2)[:n]) << np.uint64(16)
+        k |= np.where(rng.random(n) < 1 / 3, low, np.uint64(0))
+    elif spread == "runs":
+        k = rng.choice(rng.integers(0, 2**46, 1 << 14, dtype=np.uint64), n) << np.uint64(16)
+        k |= np.where(few, low, np.uint64(0))
+    elif spread == "half":
+        k = rng.integers(0, 2**62, n, dtype=np.uint64)
+        hot = rng.random(n) < 0.5
+        k[hot] = np.uint64(5 << 40) | np.where(few, low, np.uint64(7))[hot]
+    elif spread == "one digit":
+        k = rng.integers(0, 256, n, dtype=np.uint64) << np.uint64(48)
+    else:
+        k = rng.integers(0, 2**62, n, dtype=np.uint64)
+    if dtype == np.float64:
+        k = (k + np.uint64(1 << 52)).view(np.float64)  # positive normal numbers: ordered as their bits
+    else:
+        k = k.astype(dtype)
+    if spread == "sorted":
+        k.sort()
+    order = np.argsort(k, kind="stable")
+    dk = exec_.to_device(k)
+    if value is None:
+        assert np.array_equal(exec_.to_host(m.vector.sort(exec_, dk, m.op.Less)), k[order])
+        assert np.array_equal(exec_.to_host(m.vector.sort(exec_, dk, m.op.Greater)), k[order][::-1])
+        return
+    v, s = m.vector.radix_sort_by_key(exec_, dk, exec_.to_device(np.arange(n, dtype=value)), return_keys=True)
+    assert np.array_equal(exec_.to_host(v), order.astype(value))
+    assert np.array_equal(exec_.to_host(s), k[order])
