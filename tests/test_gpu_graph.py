@@ -60,3 +60,27 @@ def test_graph_replays_scan_seg_sort_and_jobs(exec_):
         hk2 = oracle.uniform_u32(0, 99, 90 + rep, 3000)
         assert ex.to_host(skeys_out).tobytes() == np.sort(hk2, kind="stable").tobytes(), rep
     g.close()
+
+
+def test_graph_replays_long_sort_of_wide_keys(exec_):
+    """The digits that get a pass, and whether the passes start over, are chosen on every replay."""
+    n = (1 << 21) + 77
+    k, v = exec_.alloc(np.uint64, n), exec_.to_device(np.arange(n, dtype=np.uint32))
+    mr.uniform_u64(exec_, 0, 9, 1, k)
+    exec_.sync()
+    with exec_.capture() as cap:
+        out, srt = m.vector.radix_sort_by_key(exec_, k, v, return_keys=True)
+    rng = np.random.default_rng(3)
+    uniform = rng.integers(0, 2**63, n, dtype=np.uint64)
+    half = uniform.copy()  # one key in half of the places, a few of them off in the lowest bits
+    half[rng.random(n) < 0.5] = 5 << 40
+    half[half == 5 << 40] += (rng.random(int((half == 5 << 40).sum())) < 1e-5).astype(np.uint64)
+    for rep, h in enumerate((uniform, half, uniform & np.uint64(1023), uniform[::-1].copy(), half)):
+        m.vector.scatter(exec_, exec_.to_device(h), v, k)
+        exec_.sync()
+        cap.graph.launch()
+        exec_.sync()
+        order = np.argsort(h, kind="stable")
+        assert np.array_equal(exec_.to_host(out), order.astype(np.uint32)), rep
+        assert np.array_equal(exec_.to_host(srt), h[order]), rep
+    cap.graph.close()
