@@ -495,7 +495,7 @@ __global__ __launch_bounds__(kBinBlock) void leaf_scatter_kernel(
   __shared__ __align__(16) T s_leaf[LEAF];
   __shared__ uint32_t s_set[LEAF / 32];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
-  const uint32_t leaves = (tlen + LEAF - 1) / LEAF;
+  const uint32_t leaves = (tlen - 1) / LEAF + 1;  // (tlen + LEAF may not fit 32 bits)
   for (uint32_t leaf = blockIdx.x; leaf < leaves; leaf += gridDim.x) {
     const uint32_t w = leaf >> p.sub_shift, sub = leaf & (p.subs - 1);
     const size_t l0 = (size_t)leaf * LEAF;

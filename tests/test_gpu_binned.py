@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import massively_amd as m
+from massively_amd import random as mr
 
 pytestmark = pytest.mark.gpu
 
@@ -81,6 +82,23 @@ def test_binned_scatter_replays(exec_):
         exec_.sync()
         got = exec_.to_host(out)
         assert np.array_equal(got[p], np.arange(N, dtype=np.uint32))
+
+
+def test_binned_scatter_largest_output():
+    """An output of 2^32 - 1 elements, whose last leaf ends past 32 bits."""
+    ex = m.Executor(0)  # its 24 GB go back with it
+    n, size = 1 << 28, (1 << 32) - 1
+    idx = np.arange(n, dtype=np.uint32) * np.uint32(2654435761)  # distinct, in no order
+    v, out = ex.alloc(np.uint32, n), ex.alloc(np.uint32, size)
+    mr.iota_u32(ex, v, 1)
+    for lo in range(0, size, 1 << 31):
+        mr.uniform_u32(ex, 0, 0, 1, out.slice(lo, min(size, lo + (1 << 31))))
+    di = ex.to_device(idx)
+    m.vector.scatter(ex, v, di, out)
+    got = ex.to_host(m.vector.gather(ex, out, di))
+    kept = idx < size
+    assert np.array_equal(got[kept], np.arange(1, n + 1, dtype=np.uint32)[kept])
+    ex.close()
 
 
 @pytest.mark.parametrize("kind,offset,outside", [("random", 0, 0), ("mixed", 1, 500)])
