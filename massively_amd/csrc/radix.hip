@@ -192,6 +192,12 @@ static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, ui
                            out, (uint32_t*)out_v, (K*)aos1, (uint32_t*)((char*)aos1 + (size_t)n * sizeof(K)),
                            n, chunk, rep, list, counts);
         MSV_HIP(hipGetLastError());
+        // Starting over reads what the first passes left in the output (equal keys
+        // still in input order): the caller's arrays may have been written by
+        // then, when a job sorts its keys or its values in place. It is sound
+        // because a repair follows at least four passes, so these are five or more.
+        q.in_k = out_k;
+        q.in_v = out_v;
         q.redo = true;
         return passes();
       }

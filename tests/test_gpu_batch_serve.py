@@ -144,6 +144,25 @@ def test_run_jobs_mixed_batch(exec_):
                 assert r.tobytes() == res[i].tobytes(), (i, host[i][0])
 
 
+@pytest.mark.parametrize("in_place", ["keys", "values", "both"])
+def test_run_jobs_long_sort_in_place(exec_, in_place):
+    """A device-wide sort whose keys or values are written over its input, with
+    half the keys equal and a few of them off in the low digits (which the
+    sort's first passes leave out and then have to order after all)."""
+    n = (1 << 23) + 11
+    rng = np.random.default_rng(9)
+    k = rng.integers(0, 2**62, n, dtype=np.uint64)
+    k[rng.random(n) < 0.5] = 5 << 40 | 7
+    k[np.flatnonzero(k == (5 << 40 | 7))[777::50_000]] -= np.uint64(1)
+    order = np.argsort(k, kind="stable")
+    dk, dv = exec_.to_device(k), exec_.to_device(np.arange(n, dtype=np.uint32))
+    ok = exec_.alloc(np.uint64, n) if in_place == "values" else dk
+    ov = exec_.alloc(np.uint32, n) if in_place == "keys" else dv
+    serve.run_jobs(exec_, [serve.Job("sort_by_key", dk, ov, inp2=dv, out2=ok)])
+    assert np.array_equal(exec_.to_host(ok), k[order])
+    assert np.array_equal(exec_.to_host(ov), order.astype(np.uint32))
+
+
 def test_run_jobs_rejects_bad_jobs(exec_):
     x = exec_.to_device(np.arange(10, dtype=np.float32))
     with pytest.raises(m.Error):
