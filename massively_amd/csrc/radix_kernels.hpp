@@ -1315,27 +1315,29 @@ __global__ __launch_bounds__(1024) void radix_repair_kernel(K* keys, uint32_t* v
   const bool digit_thread = tid < (uint32_t)kRadixBins;
   const uint64_t lt = lanemask_lt();
   for (uint32_t r = 0; r < longs; ++r) {
-    const uint32_t s = s_start[r], e = s_end[r];
+    // Indices count from the run's start (beside 2^32 elements, start + index +
+    // stride does not fit 32 bits).
+    const uint32_t s = s_start[r], cnt = s_end[r] - s;
     __syncthreads();
     if (tid < 2) s_diff[tid] = 0;
     __syncthreads();
     const uint64_t word = order_bits<K, MODE>(keys[s]);
     uint64_t x = 0;
-    for (uint32_t i = s + tid; i < e; i += 1024) x |= order_bits<K, MODE>(keys[i]) ^ word;
+    for (uint32_t i = tid; i < cnt; i += 1024) x |= order_bits<K, MODE>(keys[s + i]) ^ word;
     if (x) {
       atomicOr(&s_diff[0], (uint32_t)x);
       atomicOr(&s_diff[1], (uint32_t)(x >> 32));
     }
     __syncthreads();
     const uint64_t diff = (uint64_t)s_diff[1] << 32 | s_diff[0];
-    K *src_k = keys, *dst_k = tmp_k;
-    uint32_t *src_v = vals, *dst_v = tmp_v;
+    K *src_k = keys + s, *dst_k = tmp_k + s;
+    uint32_t *src_v = vals + (size_t)s * VW, *dst_v = tmp_v + (size_t)s * VW;
     for (uint32_t p = 0; p < low; ++p) {
       if ((diff >> (8 * p) & 0xffu) == 0) continue;
       auto digit = [&](K k) { return (uint32_t)(order_bits<K, MODE>(k) >> (8 * p)) & 0xffu; };
       if (digit_thread) s_base[tid] = 0;
       __syncthreads();
-      for (uint32_t i = s + tid; i < e; i += 1024) atomicAdd(&s_base[digit(src_k[i])], 1u);
+      for (uint32_t i = tid; i < cnt; i += 1024) atomicAdd(&s_base[digit(src_k[i])], 1u);
       __syncthreads();
       uint32_t c = 0, incl = 0;
       if (digit_thread) {
@@ -1345,17 +1347,17 @@ __global__ __launch_bounds__(1024) void radix_repair_kernel(K* keys, uint32_t* v
       }
       __syncthreads();
       if (digit_thread) {
-        uint32_t off = s + incl - c;
+        uint32_t off = incl - c;
         for (uint32_t w = 0; w < wid; ++w) off += s_wsum[w];
         s_base[tid] = off;
       }
-      for (uint32_t c0 = s; c0 < e; c0 += 1024) {
+      for (uint32_t c0 = 0; c0 < cnt; c0 += 1024) {
         for (uint32_t i = tid; i < NW * kRadixBins / 2; i += 1024)
           reinterpret_cast<uint32_t*>(&s_hist[0][0])[i] = 0;
         __syncthreads();
         const uint32_t i = c0 + tid;
-        const bool valid = i < e;
-        const K k = src_k[valid ? i : s];
+        const bool valid = i < cnt;
+        const K k = src_k[valid ? i : 0];
         const uint32_t d = digit(k);
         const uint64_t peers = match_digit<8>(d, valid);
         const uint32_t below = (uint32_t)__builtin_popcountll(peers & lt);
@@ -1388,11 +1390,11 @@ __global__ __launch_bounds__(1024) void radix_repair_kernel(K* keys, uint32_t* v
       src_v = dst_v;
       dst_v = tv;
     }
-    if (src_k != keys) {
-      for (uint32_t i = s + tid; i < e; i += 1024) {
-        keys[i] = tmp_k[i];
+    if (src_k != keys + s) {
+      for (uint32_t i = tid; i < cnt; i += 1024) {
+        dst_k[i] = src_k[i];
 #pragma unroll
-        for (int q = 0; q < VW; ++q) vals[(size_t)i * VW + q] = tmp_v[(size_t)i * VW + q];
+        for (int q = 0; q < VW; ++q) dst_v[(size_t)i * VW + q] = src_v[(size_t)i * VW + q];
       }
     }
   }

@@ -6,6 +6,7 @@ import pytest
 
 import massively_amd as m
 import oracle
+from massively_amd import random as mr
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +106,24 @@ def test_sort_high_digits_and_repair(exec_, dtype, value, spread):
     v, s = m.vector.radix_sort_by_key(exec_, dk, exec_.to_device(np.arange(n, dtype=value)), return_keys=True)
     assert np.array_equal(exec_.to_host(v), order.astype(value))
     assert np.array_equal(exec_.to_host(s), k[order])
+
+
+def test_sort_most_keys_repair_at_the_end():
+    """2^32 - 1 keys of 8 bytes, the last 2000 of which differ in the lowest digits
+    only: the run to repair ends beside the largest 32-bit index."""
+    ex = m.Executor(0)  # its 140 GB go back with it
+    n, many = (1 << 32) - 1, 2000
+    rng = np.random.default_rng(5)
+    last = np.sort(np.uint64(0xFFFFFFFFFF000000) | rng.integers(0, 1 << 24, many, dtype=np.uint64))
+    keys = ex.alloc(np.uint64, n)
+    for lo in range(0, n, 1 << 31):
+        hi = min(n, lo + (1 << 31))
+        mr.uniform_u64(ex, 0, 2**63 - 1, lo + 1, keys.slice(lo, hi))
+    places = rng.choice(n, many, replace=False).astype(np.uint32)
+    m.vector.scatter(ex, ex.to_device(last[::-1].copy()), ex.to_device(np.sort(places)), keys)
+    out = m.vector.sort(ex, keys, m.op.Less)
+    assert np.array_equal(ex.to_host(out.slice(n - many, n)), last)
+    for lo in (0, n // 3, n - (1 << 20)):
+        part = ex.to_host(out.slice(lo, lo + (1 << 20)))
+        assert np.all(part[:-1] <= part[1:])
+    ex.close()
