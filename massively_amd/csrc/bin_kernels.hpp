@@ -6,10 +6,11 @@
 // of consecutive positions by table window in LDS; the order and the windows'
 // starts stay tile-local, so there is no scan or look-back over tiles, and
 // every later pass reads and writes runs of consecutive elements.
-//  * gather: gather_window_kernel walks the table window by window while it
-//    stays in one L2, and unbin_tiles_kernel undoes the sort through LDS with
-//    the 16-bit source positions the sort kept (2^28 u32: 0.63 + 2.07 + 0.47
-//    ms, from 5.58 directly; the L2s serve about 130 G random reads/s).
+//  * gather: gather_look_kernel looks at some tiles, and the whole call goes
+//    directly or this way. gather_window_kernel walks the table window by window
+//    while it stays in one L2, and unbin_tiles_kernel undoes the sort through
+//    LDS with the 16-bit source positions the sort kept (2^28 u32: 0.58 + 2.07 +
+//    0.43 ms, from 5.56 directly; the L2s serve about 130 G random reads/s).
 //  * scatter: an L2 takes random 4-byte stores at about the same rate and lets
 //    them go as partial lines, so it ends in LDS instead. bin_leaves_kernel
 //    takes a window's runs from a group of tiles (a chunk of at most kBinChunk
@@ -17,9 +18,10 @@
 //    leaf_scatter_kernel collects a leaf in LDS and writes whole lines (2^28
 //    u32: 0.88 + 0.86 + 0.53 ms, from 6.10 with one look-back partition into
 //    256 windows and random stores from L2).
-// Each tile decides for itself: indices that stay near each other (sorted,
-// reversed, strided, clustered) are gathered or scattered directly in step 1,
-// and a chunk that would overflow (indices far from uniform) in step 2.
+// Each tile decides for itself as well: one whose indices stay near each other
+// (sorted, reversed, clustered) is gathered or scattered directly by
+// bin_tiles_kernel, and a chunk that would overflow (indices far from uniform)
+// by the scatter's step 2.
 #pragma once
 
 #include "device_common.hpp"
@@ -89,94 +91,113 @@ __device__ inline void copy_out16(const E* s, E* g, uint32_t cnt) {
     *reinterpret_cast<uint4*>(g + i) = *reinterpret_cast<const uint4*>(s + i);
 }
 
-// How many of the first `count` indices of every thread lie outside the table
-// window of their wave's first one, summed over the block (all threads call).
-template <int COUNT, int N>
+// How many indices lie outside the table window of their wave's first one,
+// summed over the block (all threads call).
+template <int N>
 __device__ inline uint32_t count_far(const uint32_t (&ix)[N], uint32_t shift, uint32_t* s_far) {
   const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ix[0] >> shift));
   uint32_t far = 0;
 #pragma unroll
-  for (int j = 0; j < COUNT; ++j) far += (uint32_t)__builtin_popcountll(ballot((ix[j] >> shift) != w0));
+  for (int j = 0; j < N; ++j) far += (uint32_t)__builtin_popcountll(ballot((ix[j] >> shift) != w0));
   if ((threadIdx.x & 63u) == 0) atomicAdd(s_far, far);
   __syncthreads();
   return *s_far;
 }
 
-// Gather, step 1: one block to kNearTile positions. When at least half of its
-// first quarter's indices leave their wave's first window, the block is put
-// off (far[block] = 1); else it gathers directly. Blocks from `full` on
-// (a partial tile of the next step) always gather directly. A look at the
-// first quarter keeps the indices from being read twice, and small blocks keep
-// the direct gather as fast as without the look (step 2's big tiles took
-// 0.61 against 0.55 ms for 2^28 reversed indices).
-constexpr int kNearBlock = 256;
-constexpr uint32_t kNearTile = 4096;
+// Gather, step 1: whether the binned form pays, from kLooks looks at kLookTile
+// indices, spread over all of them. A look votes for it when its indices touch
+// lines of the table that no other of them touches (5/8 of them; rows of a few elements, a permutation back
+// from a partition and strides along a matrix share lines, which a direct
+// gather then finds in L2), do not go on by equal steps, and meet no window
+// often (4 times the mean: indices near each other or a few hot ones, which a
+// cache holds). 3/4 of the votes decide, since a tile that should have gone
+// the other way costs more in the binned form. The look and the three launches
+// that then find nothing to do add 15 us to a direct gather. Times at 2^28 u32, direct and
+// binned (ms): random 5.56, 3.1; rows of 64 elements 0.57, 1.9; 256 interleaved
+// sorted streams 1.19, 2.7; columns of a matrix 1.84, 2.8; random within a
+// window of 2^20 that moves along 2.2, 4.7; Zipf 2.2, 2.2.
+constexpr uint32_t kLooks = 64, kLookTile = 16384;
+constexpr int kLineShift = 5;  // 4-byte elements of a 128-byte line
 
-template <typename T>
-__global__ __launch_bounds__(kNearBlock) void gather_near_kernel(
-    const T* __restrict__ table, uint32_t tlen, const uint32_t* __restrict__ idx,
-    T* __restrict__ out, uint32_t n, uint32_t shift, uint32_t full, bool aligned,
-    uint8_t* __restrict__ far) {
-  constexpr int ROWS = (int)(kNearTile / kNearBlock / 4);
-  __shared__ uint32_t s_far;
-  const uint32_t tid = threadIdx.x;
-  const size_t base = (size_t)blockIdx.x * kNearTile;
-  const bool whole = base + kNearTile <= n;
-  uint32_t ix[ROWS * 4];
-  auto load_row = [&](int r) {
-    const size_t i = base + ((size_t)r * kNearBlock + tid) * 4;
-    uint32_t x[4];
-    load4<uint32_t>(idx, i, n, whole && aligned, x);
+// The verdict of the looks (a byte each, 0 or 1).
+__device__ inline bool look_binned(const uint32_t* __restrict__ looks) {
+  uint32_t votes = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) ix[4 * r + k] = whole || i + k < n ? x[k] : 0xffffffffu;
-  };
-  load_row(0);
-  if (blockIdx.x < full) {
-    if (tid == 0) s_far = 0;
-    __syncthreads();
-    const bool put_off = count_far<4>(ix, shift, &s_far) * 2 >= kNearBlock * 4;
-    if (tid == 0) far[blockIdx.x] = put_off ? 1 : 0;
-    if (put_off) return;
-  }
-#pragma unroll
-  for (int r = 1; r < ROWS; ++r) load_row(r);
-  T v[ROWS][4];
+  for (uint32_t i = 0; i < kLooks / 4; ++i) votes += (uint32_t)__builtin_popcount(looks[i]);
+  return votes * 4 >= kLooks * 3;
+}
+
+static __global__ __launch_bounds__(kBinBlock) void gather_look_kernel(
+    const uint32_t* __restrict__ idx, uint32_t n, BinPlan p, bool aligned, uint8_t* __restrict__ looks) {
+  constexpr uint32_t TILE = kLookTile;
+  constexpr int ROWS = (int)(TILE / kBinBlock / 4);
+  constexpr uint32_t BITS = 17;  // of the lines' hash
+  __shared__ uint32_t s_lines[(1u << BITS) / 32], s_cnt[kBinMost];
+  __shared__ uint32_t s_new, s_regular, s_most;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t shift = p.leaf_shift + p.sub_shift;
+  const size_t base = (size_t)((uint64_t)blockIdx.x * (n / TILE) / kLooks) * TILE;
+  for (uint32_t i = tid; i < (1u << BITS) / 32; i += kBinBlock) s_lines[i] = 0;
+  if (tid < kBinMost) s_cnt[tid] = 0;
+  if (tid == 0) s_new = s_regular = s_most = 0;
+  uint32_t ix[ROWS][4];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[r][k] = ix[4 * r + k] < tlen ? table[ix[4 * r + k]] : (T)0;
+    load4<uint32_t>(idx, base + ((size_t)r * kBinBlock + tid) * 4, 0xffffffffu, aligned, ix[r]);
+  __syncthreads();
+  uint32_t regular = 0;
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    const size_t o = base + ((size_t)r * kNearBlock + tid) * 4;
-    if (whole && aligned) {
-      store4(out + o, v[r]);
-    } else {
+    const uint32_t step = ix[r][1] - ix[r][0];
+    regular += ix[r][2] - ix[r][1] == step && ix[r][3] - ix[r][2] == step ? 1 : 0;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (o + k < n) out[o + k] = v[r][k];
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t line = ix[r][k] >> kLineShift;
+      if (k == 0 || line != ix[r][k - 1] >> kLineShift) {
+        const uint32_t h = (line * 2654435761u) >> (32 - BITS);
+        atomicOr(&s_lines[h >> 5], 1u << (h & 31u));
+      }
+      // A wave in one window adds once (an index past the table counts for the last).
+      const uint32_t w = min(ix[r][k] >> shift, p.windows - 1);
+      const uint32_t w0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
+      if (ballot(w != w0) != 0) atomicAdd(&s_cnt[w], 1u);
+      else if (lane == 0) atomicAdd(&s_cnt[w0], (uint32_t)kWave);
     }
   }
+  regular = wave_reduce<uint32_t, OP_ADD>(regular);
+  if (lane == 0) atomicAdd(&s_regular, regular);
+  __syncthreads();
+  uint32_t lines = 0;
+  for (uint32_t i = tid; i < (1u << BITS) / 32; i += kBinBlock) lines += (uint32_t)__builtin_popcount(s_lines[i]);
+  lines = wave_reduce<uint32_t, OP_ADD>(lines);
+  const uint32_t most = wave_reduce<uint32_t, OP_MAX>(tid < p.windows ? s_cnt[tid] : 0u);
+  if (lane == 0) {
+    atomicAdd(&s_new, lines);
+    atomicMax(&s_most, most);
+  }
+  __syncthreads();
+  if (tid == 0)
+    looks[blockIdx.x] = s_new * 8 >= TILE * 5 && s_regular * 2 < TILE / 4 && s_most * p.windows <= 4 * TILE;
 }
 
 // The sort of one tile by window. table: the gather's values or the scatter's
 // output, of tlen elements; io: the gather's output or the scatter's values,
 // by position. pidx: the tile's indices in window order; ppos (gather): their
 // in-tile positions; pval (scatter): their values. A row of zeros in `starts`:
-// the tile was done directly. The gather takes the tiles that
-// gather_near_kernel put off (`far`, a byte to kNearTile positions), the
-// scatter every tile (the last, partial one directly). A block that binned a
-// tile says so in the launch's status word, for the later steps (looking at it
-// first: 65536 stores to one word took 2.3 ms).
+// the tile was done directly. The gather takes the full tiles, and none unless
+// the looks say so; the scatter takes every tile (the last, partial one
+// directly), and a block that binned one says so in the launch's status word,
+// for the later steps (looking at it first: 65536 stores to one word took 2.3 ms).
 template <typename T, int IPT, bool SCATTER>
 __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 8 : 4) void bin_tiles_kernel(
     T* __restrict__ table, uint32_t tlen, const uint32_t* __restrict__ idx, T* __restrict__ io,
-    uint32_t n, BinPlan p, bool aligned, const uint8_t* __restrict__ far,
+    uint32_t n, BinPlan p, bool aligned, const uint32_t* __restrict__ looks,
     uint32_t* __restrict__ pidx, uint16_t* __restrict__ ppos, T* __restrict__ pval,
     uint16_t* __restrict__ starts, uint64_t* __restrict__ status, uint32_t gen) {
   constexpr uint32_t TILE = (uint32_t)kBinBlock * IPT;
   constexpr int ROWS = IPT / 4;
   constexpr uint32_t W = SCATTER ? sizeof(T) : 4;
-  static_assert(TILE <= 32768 && IPT % 8 == 0 && kBinBlock * 4 == kNearTile, "tile");
+  static_assert(TILE <= 32768 && IPT % 8 == 0, "tile");
   __shared__ __align__(16) unsigned char s_mem[TILE * W];
   __shared__ uint32_t s_cnt[kBinMost], s_start[kBinMost + 1];
   __shared__ uint32_t s_far, s_out, s_most, s_wsum[kBinMost / kWave];
@@ -184,28 +205,12 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
   const uint32_t shift = p.leaf_shift + p.sub_shift;
   uint32_t tile = blockIdx.x;
   if constexpr (!SCATTER) {
-    // All of the block's tiles at once, so that a launch without work ends at once.
-    const uint32_t mine = (p.tiles - tile + gridDim.x - 1) / gridDim.x;
-    bool any = false;
-    for (uint32_t i = tid; i < mine * ROWS; i += kBinBlock)
-      any = any || far[(size_t)(tile + i / ROWS * gridDim.x) * ROWS + i % ROWS];
-    if (!__syncthreads_or(any)) {
-      for (; tile < p.tiles; tile += gridDim.x)
-        if (tid <= p.windows) starts[(size_t)tile * p.tile_row + tid] = 0;
-      return;
-    }
+    if (!look_binned(looks)) return;
   }
   do {
     const size_t base = (size_t)tile * TILE;
     const bool full = base + TILE <= n;
     uint16_t* row = starts + (size_t)tile * p.tile_row;
-    // The rows (of kNearTile positions) to do here.
-    uint32_t rows = 0;
-    if constexpr (!SCATTER) {
-#pragma unroll
-      for (int r = 0; r < ROWS; ++r) rows |= (far[(size_t)tile * ROWS + r] ? 1u : 0u) << r;
-    }
-    bool spread = SCATTER ? full : rows == (1u << ROWS) - 1;
     __syncthreads();
     if (tid < kBinMost) s_cnt[tid] = 0;
     if (tid == 0) s_far = s_out = s_most = 0;
@@ -224,11 +229,10 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
         for (int k = 0; k < 4; ++k) ix[4 * r + k] = i + k < n ? idx[i + k] : 0xffffffffu;
       }
     }
-    if constexpr (SCATTER) {
-      // Counted in registers first: the counts below would serialise on one
-      // LDS word for a tile that stays in a window or two.
-      spread = spread && count_far<IPT>(ix, shift, &s_far) * 2 >= TILE;
-    } else {
+    // Counted in registers first: the counts below would serialise on one
+    // LDS word for a tile that stays in a window or two.
+    bool spread = full && count_far(ix, shift, &s_far) * 2 >= TILE;
+    if constexpr (!SCATTER) {
       bool out = false;
 #pragma unroll
       for (int j = 0; j < IPT; ++j) out = out || ix[j] >= tlen;
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
 #pragma unroll
           for (int k = 0; k < 4; ++k)
             if (ix[4 * r + k] < tlen) table[ix[4 * r + k]] = x[k];
-        } else if (rows >> r & 1u) {
+        } else {
 #pragma unroll
           for (int k = 0; k < 4; ++k) x[k] = ix[4 * r + k] < tlen ? table[ix[4 * r + k]] : (T)0;
 #pragma unroll
@@ -273,8 +277,10 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
 #pragma unroll
     for (int j = 0; j < IPT; ++j) asm volatile("" : "+v"(ix[j]));
     const uint32_t total = s_start[kBinMost];
-    if (tid == 0 && status_flag(ld_agent(status), gen) == 0)
-      st_agent(status, pack_status(gen, kFlagInc, 0, 0));
+    if constexpr (SCATTER) {
+      if (tid == 0 && status_flag(ld_agent(status), gen) == 0)
+        st_agent(status, pack_status(gen, kFlagInc, 0, 0));
+    }
     if (tid < p.windows) row[tid] = (uint16_t)s_start[tid];
     if (tid == kBinMost) row[p.windows] = (uint16_t)total;
     uint32_t* s_idx = reinterpret_cast<uint32_t*>(s_mem);
@@ -321,8 +327,8 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
 template <typename T, uint32_t TILE, int U>
 __global__ __launch_bounds__(256) void gather_window_kernel(
     const T* __restrict__ table, uint32_t tlen, BinPlan p, const uint32_t* pidx, T* pval,
-    const uint16_t* __restrict__ starts, const uint64_t* __restrict__ status, uint32_t gen) {
-  if (status_flag(ld_agent(status), gen) == 0) return;
+    const uint16_t* __restrict__ starts, const uint32_t* __restrict__ looks) {
+  if (!look_binned(looks)) return;
   constexpr uint32_t kTilesPerWave = 16, kTilesPerBlock = 4 * kTilesPerWave;
   const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
   const uint32_t g = blockIdx.x % kXcds;
@@ -552,8 +558,8 @@ template <typename T, int IPT>
 __global__ __launch_bounds__(kBinBlock, IPT * sizeof(T) == 64 ? 8 : 4) void unbin_tiles_kernel(
     BinPlan p, const T* __restrict__ pval, const uint16_t* __restrict__ ppos,
     const uint16_t* __restrict__ starts, T* __restrict__ out, bool aligned,
-    const uint64_t* __restrict__ status, uint32_t gen) {
-  if (status_flag(ld_agent(status), gen) == 0) return;
+    const uint32_t* __restrict__ looks) {
+  if (!look_binned(looks)) return;
   constexpr uint32_t TILE = (uint32_t)kBinBlock * IPT;
   constexpr int V = 16 / sizeof(T);
   __shared__ __align__(16) T s_val[TILE];

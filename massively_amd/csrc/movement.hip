@@ -19,14 +19,19 @@ constexpr int kMoveBlock = 256;
 constexpr int kMoveRows = 4;  // 4 x uint4 of indices = 16 indices per thread
 constexpr uint32_t kMoveTile = kMoveBlock * kMoveRows * 4;
 
+// With `looks` (see gather_look_kernel), the first `binned` positions are done by
+// the binned form when the looks say so.
 template <typename T>
 __global__ __launch_bounds__(kMoveBlock) void gather_kernel(const T* __restrict__ values,
                                                             uint32_t vlen,
                                                             const uint32_t* __restrict__ idx,
                                                             T* __restrict__ out, uint32_t n,
-                                                            bool aligned) {
+                                                            bool aligned,
+                                                            const uint32_t* __restrict__ looks,
+                                                            uint32_t binned) {
   const uint32_t tid = threadIdx.x;
   const size_t base = (size_t)blockIdx.x * kMoveTile;
+  if (looks && base < binned && look_binned(looks)) return;
   const bool full = aligned && base + kMoveTile <= n;
   uint32_t ix[kMoveRows][4];
   if (full) {
@@ -116,10 +121,10 @@ __global__ void iota_u32_kernel(uint32_t* __restrict__ out, uint32_t n, uint32_t
 // ---- host ------------------------------------------------------------------
 template <typename T>
 static msv_status direct_gather(Ctx& c, const T* values, uint32_t vlen, const uint32_t* idx, T* out,
-                                uint32_t n) {
+                                uint32_t n, const uint32_t* looks = nullptr, uint32_t binned = 0) {
   const bool aligned = (((uintptr_t)idx | (uintptr_t)out) & 15u) == 0;
   hipLaunchKernelGGL(gather_kernel<T>, dim3(div_up(n, kMoveTile)), dim3(kMoveBlock), 0, c.stream(),
-                     values, vlen, idx, out, n, aligned);
+                     values, vlen, idx, out, n, aligned, looks, binned);
   MSV_HIP(hipGetLastError());
   return MSV_OK;
 }
@@ -161,27 +166,25 @@ static msv_status binned_gather(Ctx& c, const uint32_t* values, uint32_t vlen, c
   uint32_t* pidx = (uint32_t*)c.scratch(sizeof(uint32_t) * (size_t)p.tiles * TILE);
   uint16_t* ppos = (uint16_t*)c.scratch(sizeof(uint16_t) * (size_t)p.tiles * TILE);
   uint16_t* starts = (uint16_t*)c.scratch(sizeof(uint16_t) * (size_t)p.tiles * p.tile_row);
-  uint8_t* far = (uint8_t*)c.scratch((size_t)p.tiles * (TILE / kNearTile));
-  if (!pidx || !ppos || !starts || !far) {
+  uint32_t* looks = (uint32_t*)c.scratch(kLooks);
+  if (!pidx || !ppos || !starts || !looks) {
     clear_error();
     return direct_gather(c, values, vlen, idx, out, n);
   }
-  uint64_t *counter, *status;
-  uint32_t gen;
-  MSV_TRY(c.lookback(1, &counter, &status, &gen));
   const bool aligned = (((uintptr_t)idx | (uintptr_t)out) & 15u) == 0;
   const uint32_t cus = (uint32_t)c.num_cus();
-  hipLaunchKernelGGL(gather_near_kernel<uint32_t>, dim3(div_up(n, kNearTile)), dim3(kNearBlock), 0,
-                     c.stream(), values, vlen, idx, out, n, shift, p.tiles * (TILE / kNearTile),
-                     aligned, far);
+  static_assert(TILE % kMoveTile == 0, "a tile is whole direct tiles");
+  hipLaunchKernelGGL(gather_look_kernel, dim3(kLooks), dim3(kBinBlock), 0, c.stream(), idx, n, p,
+                     aligned, (uint8_t*)looks);
+  MSV_TRY(direct_gather(c, values, vlen, idx, out, n, looks, p.tiles * TILE));
   hipLaunchKernelGGL((bin_tiles_kernel<uint32_t, IPT, false>), dim3(std::min(p.tiles, cus)),
                      dim3(kBinBlock), 0, c.stream(), const_cast<uint32_t*>(values), vlen, idx, out, n,
-                     p, aligned, far, pidx, ppos, (uint32_t*)nullptr, starts, status, gen);
+                     p, aligned, looks, pidx, ppos, (uint32_t*)nullptr, starts, (uint64_t*)nullptr, 0u);
   // The values replace the indices in place.
   hipLaunchKernelGGL((gather_window_kernel<uint32_t, TILE, 8>), dim3(div_up(cus, kXcds) * kXcds),
-                     dim3(256), 0, c.stream(), values, vlen, p, pidx, pidx, starts, status, gen);
+                     dim3(256), 0, c.stream(), values, vlen, p, pidx, pidx, starts, looks);
   hipLaunchKernelGGL((unbin_tiles_kernel<uint32_t, IPT>), dim3(std::min(p.tiles, 4 * cus)),
-                     dim3(kBinBlock), 0, c.stream(), p, pidx, ppos, starts, out, aligned, status, gen);
+                     dim3(kBinBlock), 0, c.stream(), p, pidx, ppos, starts, out, aligned, looks);
   MSV_HIP(hipGetLastError());
   return MSV_OK;
 }
@@ -216,7 +219,7 @@ static msv_status binned_scatter(Ctx& c, const T* values, const uint32_t* idx, u
   const uint32_t cus = (uint32_t)c.num_cus();
   hipLaunchKernelGGL((bin_tiles_kernel<T, IPT, true>), dim3(div_up(n, TILE)), dim3(kBinBlock), 0,
                      c.stream(), out, olen, idx, const_cast<T*>(values), n, p, aligned,
-                     (const uint8_t*)nullptr, pidx, (uint16_t*)nullptr, pval, starts, status, gen);
+                     (const uint32_t*)nullptr, pidx, (uint16_t*)nullptr, pval, starts, status, gen);
   hipLaunchKernelGGL((bin_leaves_kernel<T, TILE>), dim3(std::min(p.windows * p.groups, 2 * cus)),
                      dim3(kBinBlock), 0, c.stream(), out, p, pidx, pval, starts, cidx, cval, rows,
                      status, gen);
@@ -228,9 +231,9 @@ static msv_status binned_scatter(Ctx& c, const T* values, const uint32_t* idx, u
 }
 
 // The binned gather: 4-byte elements (8-byte ones gained 16% at 2^27), at least
-// 2^27 indices (random 2.54 -> 1.57 ms; the three launches that find nothing to
-// do add 8 us to a sorted gather, 3% there) and at most 16 table elements to an
-// index, since every window is read once.
+// 2^27 indices (random 2.54 -> 1.57 ms; the look and the launches that find
+// nothing to do add 15 us to any other, 5% to a sorted gather there) and at most
+// 16 table elements to an index, since every window is read once.
 static bool gather_binned(msv_dtype dt, uint32_t n, uint32_t vlen) {
   return dtype_size(dt) == 4 && n >= (1u << 27) && vlen / 16 <= n && vlen >= (1u << 24);
 }

@@ -101,8 +101,10 @@ def test_binned_scatter_largest_output():
     ex.close()
 
 
-@pytest.mark.parametrize("kind,offset,outside", [("random", 0, 0), ("mixed", 1, 500)])
+@pytest.mark.parametrize("kind,offset,outside", [("random", 0, 0), ("mixed", 1, 500), ("rows", 3, 40),
+                                                 ("mostly random", 0, 0)])
 def test_binned_gather(exec_, kind, offset, outside):
+    """Both ways the looks decide, and tiles that go directly in the binned form."""
     n, size = (1 << 27) + 40_000, (1 << 27) - 7
     rng = np.random.default_rng(offset)
     idx = np.empty(n + offset, np.uint32)
@@ -113,7 +115,14 @@ def test_binned_gather(exec_, kind, offset, outside):
     if kind == "mixed":
         for lo in range(0, n - 50_000, 1 << 20):
             idx[lo:lo + 50_000] = np.arange(lo % size, lo % size + 50_000) % size
-        idx[rng.integers(0, n, outside)] = size + 3
+    elif kind == "rows":  # of 64 elements: a direct gather
+        rows = idx[:(n + offset) // 64] // np.uint32(64) * np.uint32(64)
+        idx[:rows.size * 64].reshape(-1, 64)[:] = rows[:, None] + np.arange(64, dtype=np.uint32)
+    elif kind == "mostly random":  # one tile in eight is sorted
+        for lo in range(0, n - 65536, 8 * 32768):
+            idx[lo:lo + 32768] = np.sort(idx[lo:lo + 32768])
+            idx[lo + 32768:lo + 65536] = np.arange(32768, dtype=np.uint32) + np.uint32(lo % (size - 32768))
+    idx[rng.integers(0, n, outside)] = size + 3
     v = rng.integers(0, 2**32, size, dtype=np.uint32)
     di = exec_.to_device(idx).slice(offset, offset + n)
     got = exec_.to_host(m.vector.gather(exec_, exec_.to_device(v), di))
