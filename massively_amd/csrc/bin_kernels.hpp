@@ -14,14 +14,13 @@
 //  * scatter: an L2 takes random 4-byte stores at about the same rate and lets
 //    them go as partial lines, so it ends in LDS instead. bin_leaves_kernel
 //    takes a window's runs from a group of tiles (a chunk of at most kBinChunk
-//    elements) and sorts them by leaf (64 KiB of the table), chunk-local;
-//    leaf_scatter_kernel collects a leaf in LDS and writes whole lines (2^28
-//    u32: 0.88 + 0.86 + 0.53 ms, from 6.10 with one look-back partition into
-//    256 windows and random stores from L2).
+//    elements; more of them where the window has more) and sorts them by leaf
+//    (64 KiB of the table), chunk-local; leaf_scatter_kernel collects a leaf in
+//    LDS and writes whole lines (2^28 u32: 0.76 + 0.94 + 0.57 ms, from 6.0 with one look-back
+//    partition into 256 windows and random stores from L2).
 // Each tile decides for itself as well: one whose indices stay near each other
-// (sorted, reversed, clustered) is gathered or scattered directly by
-// bin_tiles_kernel, and a chunk that would overflow (indices far from uniform)
-// by the scatter's step 2.
+// (sorted, reversed, clustered) is gathered or scattered
+// directly by bin_tiles_kernel.
 #pragma once
 
 #include "device_common.hpp"
@@ -42,8 +41,37 @@ struct BinPlan {
   uint32_t leaf_shift, sub_shift;
   uint32_t windows, subs;      // subs = 1 << sub_shift
   uint32_t tile_row, chunk_row;
-  uint32_t tiles, group, groups;  // full tiles; tiles per chunk; chunks per window
+  uint32_t tiles, group, groups;  // full tiles; tiles of a group; groups
+  uint32_t cap;                   // chunks a window can have
 };
+
+// What bin_leaves_kernel hands to leaf_scatter_kernel. Chunk c of window w has row
+// w * cap + c of leaf starts. Elements are placed as blocks come, in one of
+// kShards parts of the memory (one counter for all blocks cost 8 us when 512
+// blocks begin at once).
+constexpr uint32_t kShards = 8, kShardStep = 16;
+struct BinChunks {
+  uint32_t* used;    // elements / 8 of each part, kShardStep words apart
+  uint32_t* counts;  // chunks of each window
+  uint32_t* at;      // a chunk's first element / 8
+  uint32_t shard;    // elements / 8 of a part
+};
+
+// Room for cnt elements (their first / 8), in two steps: the first only asks, so
+// that the answer can come while the block does other work. A part that has run
+// out leaves less than a chunk unused, which the parts' size allows for.
+__device__ inline uint32_t ask_room(const BinChunks& c, uint32_t cnt) {
+  return atomicAdd(&c.used[blockIdx.x % kShards * kShardStep], (cnt + 7) / 8);
+}
+__device__ inline uint32_t take_room(const BinChunks& c, uint32_t cnt, uint32_t asked) {
+  const uint32_t units = (cnt + 7) / 8;
+  uint32_t s = blockIdx.x % kShards;
+  while (asked + units > c.shard) {
+    s = (s + 1) % kShards;
+    asked = atomicAdd(&c.used[s * kShardStep], units);
+  }
+  return s * c.shard + asked;
+}
 
 // Exclusive scan of s_cnt[0, kBinMost) into s_start, by the first kBinMost
 // threads; s_start[kBinMost] is the total, *s_most (zero before) the largest.
@@ -180,6 +208,34 @@ static __global__ __launch_bounds__(kBinBlock) void gather_look_kernel(
     looks[blockIdx.x] = s_new * 8 >= TILE * 5 && s_regular * 2 < TILE / 4 && s_most * p.windows <= 4 * TILE;
 }
 
+// Keeps one element of those of a tile with the same index (most of the time: not
+// where another index has the same hash) and marks the others kNoPlace. All of
+// them meet in one leaf, which one block collects: 2^24 u32 with Zipf indices
+// (7% of them one index) 1.29 ms, now 0.13; 2^28 3.8 -> 1.93. s_slot: a word to
+// an element.
+template <int IPT>
+__device__ inline void drop_repeats(uint32_t (&ix)[IPT], uint32_t tlen, uint32_t* s_slot) {
+  constexpr uint32_t SLOTS = (uint32_t)kBinBlock * IPT;
+  static_assert((SLOTS & (SLOTS - 1)) == 0 && IPT <= 32, "slots");
+  auto slot = [](uint32_t i) { return (i * 2654435761u) >> (32 - __builtin_ctz(SLOTS)); };
+  uint32_t mine = 0;  // elements whose index has its slot
+#pragma unroll
+  for (int j = 0; j < IPT; ++j)
+    if (ix[j] < tlen) s_slot[slot(ix[j])] = ix[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) mine |= (ix[j] < tlen && s_slot[slot(ix[j])] == ix[j] ? 1u : 0u) << j;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < IPT; ++j)
+    if (mine >> j & 1u) s_slot[slot(ix[j])] = threadIdx.x * IPT + j;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < IPT; ++j)
+    if ((mine >> j & 1u) && s_slot[slot(ix[j])] != threadIdx.x * IPT + j) ix[j] = kNoPlace;
+  __syncthreads();
+}
+
 // The sort of one tile by window. table: the gather's values or the scatter's
 // output, of tlen elements; io: the gather's output or the scatter's values,
 // by position. pidx: the tile's indices in window order; ppos (gather): their
@@ -193,7 +249,7 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
     T* __restrict__ table, uint32_t tlen, const uint32_t* __restrict__ idx, T* __restrict__ io,
     uint32_t n, BinPlan p, bool aligned, const uint32_t* __restrict__ looks,
     uint32_t* __restrict__ pidx, uint16_t* __restrict__ ppos, T* __restrict__ pval,
-    uint16_t* __restrict__ starts, uint64_t* __restrict__ status, uint32_t gen) {
+    uint16_t* __restrict__ starts, BinChunks chunks, uint64_t* __restrict__ status, uint32_t gen) {
   constexpr uint32_t TILE = (uint32_t)kBinBlock * IPT;
   constexpr int ROWS = IPT / 4;
   constexpr uint32_t W = SCATTER ? sizeof(T) : 4;
@@ -201,11 +257,14 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
   __shared__ __align__(16) unsigned char s_mem[TILE * W];
   __shared__ uint32_t s_cnt[kBinMost], s_start[kBinMost + 1];
   __shared__ uint32_t s_far, s_out, s_most, s_wsum[kBinMost / kWave];
-  const uint32_t tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t shift = p.leaf_shift + p.sub_shift;
   uint32_t tile = blockIdx.x;
   if constexpr (!SCATTER) {
     if (!look_binned(looks)) return;
+  } else if (tile == 0) {  // for the next step
+    if (tid < p.windows) chunks.counts[tid] = 0;
+    if (tid < kShards) chunks.used[tid * kShardStep] = 0;
   }
   do {
     const size_t base = (size_t)tile * TILE;
@@ -241,7 +300,7 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
       spread = spread && s_out == 0;
     }
     uint32_t at[IPT];
-    if (spread) {
+    auto count = [&]() {
       // A scatter drops an index past the table; a gather reads 0 there, and
       // its tile is done directly.
 #pragma unroll
@@ -250,6 +309,23 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
       __syncthreads();
       bin_scan(s_cnt, s_start, s_wsum, &s_most);
       spread = s_most * p.windows <= 4 * TILE;
+    };
+    if (spread) count();
+    if constexpr (SCATTER) {
+      // A window with far more than its share (6 standard deviations) may come
+      // from an index that is there many times (then it also follows itself):
+      // only one of its values stays.
+      const int32_t over = (int32_t)s_most - (int32_t)(TILE / p.windows);
+      bool twin = false;
+#pragma unroll
+      for (int j = 1; j < IPT; ++j) twin = twin || ((j & 3) && ix[j] == ix[j - 1] && ix[j] < tlen);
+      if (over > 0 && (uint32_t)(over * over) > 36 * (TILE / p.windows) && __syncthreads_or(twin)) {
+        drop_repeats<IPT>(ix, tlen, reinterpret_cast<uint32_t*>(s_mem));
+        if (tid < kBinMost) s_cnt[tid] = 0;
+        if (tid == 0) s_most = 0;
+        __syncthreads();
+        count();
+      }
     }
     if (!spread) {
       if (full && tid <= p.windows) row[tid] = 0;
@@ -365,50 +441,57 @@ __global__ __launch_bounds__(256) void gather_window_kernel(
   }
 }
 
-// Copies runs of E (s_src: their first elements, s_off: their places) to LDS,
-// 32 lanes a run, four loads of a lane in flight.
+// Copies the elements [lo, hi) of a sequence of runs of E (s_src: their first
+// elements, s_off: their places in the sequence) to LDS, 32 lanes a run, four
+// loads of a lane in flight.
 template <typename E>
 __device__ inline void load_runs(const E* __restrict__ from, const uint32_t* s_src,
-                                 const uint32_t* s_off, uint32_t runs, E* s_to) {
+                                 const uint32_t* s_off, uint32_t runs, uint32_t lo, uint32_t hi,
+                                 E* s_to) {
   constexpr int U = 4;
   for (uint32_t r = threadIdx.x / 32; r < runs; r += kBinBlock / 32) {
-    const uint32_t o = s_off[r], len = s_off[r + 1] - o;
+    const uint32_t o = s_off[r], e = min(s_off[r + 1], hi);
     const E* src = from + s_src[r];
-    for (uint32_t k0 = threadIdx.x & 31u; k0 < len; k0 += 32 * U) {
+    for (uint32_t k0 = max(o, lo) + (threadIdx.x & 31u); k0 < e; k0 += 32 * U) {
       E d[U];
 #pragma unroll
       for (int k = 0; k < U; ++k)
-        if (k0 + 32 * k < len) d[k] = src[k0 + 32 * k];
+        if (k0 + 32 * k < e) d[k] = src[k0 + 32 * k - o];
 #pragma unroll
       for (int k = 0; k < U; ++k)
-        if (k0 + 32 * k < len) s_to[o + k0 + 32 * k] = d[k];
+        if (k0 + 32 * k < e) s_to[k0 + 32 * k - lo] = d[k];
     }
   }
 }
 
-// Scatter, step 2: one chunk a block at a time. cidx: the elements' places in
-// their leaf, in leaf order; cval: their values. A chunk that does not fit is
-// scattered directly and leaves a row of zeros. Concurrent blocks take the
+// Scatter, step 2: the runs of one window in one group of tiles at a time, in as
+// many chunks of equal length as they fill. cidx: the elements' places in their
+// leaf, in leaf order; cval: their values. Where indices are spread evenly a
+// group fills 7/8 of a chunk; a window with up to four times its share (a tile
+// with more does not get here) takes up to four. (Chunks of fixed places, one to
+// a window and group, with what did not fit scattered directly: 2^28 u32 into
+// half of the output 9.0 ms, now 2.8.) Concurrent blocks take the
 // windows of one group of tiles, so the runs they read are neighbours (a
 // window at a time over all tiles was 8% slower: 1 KiB pieces of 1 GiB).
-// 64 registers and 64 KiB of LDS: two blocks a CU (1.12 -> 0.86 ms at 2^28 u32).
+// 64 registers and 64 KiB of LDS: two blocks a CU (one: 1.12 ms at 2^28 u32, two
+// then 0.86, and 0.94 with the chunks' places asked for).
 template <typename T, uint32_t TILE>
 __global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_kernel(
-    T* __restrict__ table, BinPlan p, const uint32_t* __restrict__ pidx,
-    const T* __restrict__ pval, const uint16_t* __restrict__ starts, uint16_t* __restrict__ cidx,
-    T* __restrict__ cval, uint16_t* __restrict__ rows, const uint64_t* __restrict__ status,
-    uint32_t gen) {
+    BinPlan p, const uint32_t* __restrict__ pidx, const T* __restrict__ pval,
+    const uint16_t* __restrict__ starts, uint16_t* __restrict__ cidx, T* __restrict__ cval,
+    uint16_t* __restrict__ rows, BinChunks chunks, const uint64_t* __restrict__ status, uint32_t gen) {
   if (status_flag(ld_agent(status), gen) == 0) return;
   __shared__ __align__(16) T s_val[kBinChunk];
   __shared__ uint32_t s_cnt[kBinMost], s_off[kBinMost + 1], s_src[kBinMost];
   __shared__ uint32_t s_wsum[kBinMost / kWave];
-  const uint32_t tid = threadIdx.x, lane = tid & 31u, grp = tid >> 5;
+  __shared__ uint32_t s_at, s_place;
+  const uint32_t tid = threadIdx.x;
   uint32_t* s_idx = reinterpret_cast<uint32_t*>(s_val);
   uint16_t* s_16 = reinterpret_cast<uint16_t*>(s_val);
   for (uint32_t q = blockIdx.x; q < p.windows * p.groups; q += gridDim.x) {
-    const uint32_t w = q % p.windows, g = q / p.windows, c = w * p.groups + g;
+    const uint32_t w = q % p.windows, g = q / p.windows;
     // The window's runs in the group's tiles: where each begins, and its place
-    // in the chunk.
+    // among them.
     const uint32_t t0 = g * p.group, runs = min(p.group, p.tiles - t0);
     if (tid < kBinMost) {
       uint32_t s = 0, e = 0;
@@ -422,69 +505,77 @@ __global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_
     }
     __syncthreads();
     bin_scan(s_cnt, s_off, s_wsum);
-    const uint32_t cnt = s_off[kBinMost];
-    uint16_t* row = rows + (size_t)c * p.chunk_row;
-    if (cnt > kBinChunk) {
-      if (tid <= p.subs) row[tid] = 0;
-      for (uint32_t r = grp; r < runs; r += kBinBlock / 32)
-        for (uint32_t k = lane; k < s_off[r + 1] - s_off[r]; k += 32)
-          table[pidx[s_src[r] + k]] = pval[s_src[r] + k];
+    const uint32_t total = s_off[kBinMost];
+    const uint32_t pieces = (total + kBinChunk - 1) / kBinChunk;
+    for (uint32_t c = 0; c < pieces; ++c) {
+      const uint32_t lo = (uint32_t)((uint64_t)total * c / pieces);
+      const uint32_t hi = (uint32_t)((uint64_t)total * (c + 1) / pieces), cnt = hi - lo;
+      load_runs(pidx, s_src, s_off, runs, lo, hi, s_idx);
+      if (tid < kBinMost) s_cnt[tid] = 0;
       __syncthreads();
-      continue;
-    }
-    load_runs(pidx, s_src, s_off, runs, s_idx);
-    if (tid < kBinMost) s_cnt[tid] = 0;
-    __syncthreads();
-    uint32_t ix[kChunkIpt], at[kChunkIpt];
-#pragma unroll
-    for (int j = 0; j < kChunkIpt; ++j) {
-      const uint32_t i = tid + (uint32_t)j * kBinBlock;
-      ix[j] = s_idx[i];
-      at[j] = i < cnt ? atomicAdd(&s_cnt[(ix[j] >> p.leaf_shift) & (p.subs - 1)], 1u) : kNoPlace;
-    }
-    // Recompute the leaf numbers below instead of keeping them in registers.
-#pragma unroll
-    for (int j = 0; j < kChunkIpt; ++j) asm volatile("" : "+v"(ix[j]));
-    __syncthreads();
-    // The leaves' starts (over their counts: s_off still holds the runs' places).
-    uint32_t n_leaf = 0, incl = 0;
-    if (tid < kBinMost) {
-      n_leaf = s_cnt[tid];
-      incl = wave_inclusive_scan<uint32_t, OP_ADD>(n_leaf);
-      if ((tid & 63u) == 63u) s_wsum[tid >> 6] = incl;
-    }
-    __syncthreads();
-    if (tid < kBinMost) {
-      uint32_t start = incl - n_leaf;
-      for (uint32_t v = 0; v < (tid >> 6); ++v) start += s_wsum[v];
-      s_cnt[tid] = start;
-      if (tid < p.subs) row[tid] = (uint16_t)start;
-    }
-    if (tid == kBinMost) row[p.subs] = (uint16_t)cnt;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kChunkIpt; ++j) {
-      if (at[j] != kNoPlace) {
-        at[j] += s_cnt[(ix[j] >> p.leaf_shift) & (p.subs - 1)];
-        s_16[at[j]] = (uint16_t)(ix[j] & ((1u << p.leaf_shift) - 1));
+      uint32_t place = 0, asked = 0;
+      if (tid == kBinBlock - 1) {
+        place = atomicAdd(&chunks.counts[w], 1u);
+        asked = ask_room(chunks, cnt);
       }
+      uint32_t ix[kChunkIpt], at[kChunkIpt];
+#pragma unroll
+      for (int j = 0; j < kChunkIpt; ++j) {
+        const uint32_t i = tid + (uint32_t)j * kBinBlock;
+        ix[j] = s_idx[i];
+        at[j] = i < cnt ? atomicAdd(&s_cnt[(ix[j] >> p.leaf_shift) & (p.subs - 1)], 1u) : kNoPlace;
+      }
+      // Recompute the leaf numbers below instead of keeping them in registers.
+#pragma unroll
+      for (int j = 0; j < kChunkIpt; ++j) asm volatile("" : "+v"(ix[j]));
+      __syncthreads();
+      // The leaves' starts (over their counts: s_off still holds the runs' places).
+      uint32_t n_leaf = 0, incl = 0;
+      if (tid < kBinMost) {
+        n_leaf = s_cnt[tid];
+        incl = wave_inclusive_scan<uint32_t, OP_ADD>(n_leaf);
+        if ((tid & 63u) == 63u) s_wsum[tid >> 6] = incl;
+      }
+      if (tid == kBinBlock - 1) {
+        s_place = w * p.cap + place;
+        s_at = take_room(chunks, cnt, asked);
+        chunks.at[s_place] = s_at;
+      }
+      __syncthreads();
+      uint16_t* row = rows + (size_t)s_place * p.chunk_row;
+      const size_t first = (size_t)s_at * 8;
+      if (tid < kBinMost) {
+        uint32_t start = incl - n_leaf;
+        for (uint32_t v = 0; v < (tid >> 6); ++v) start += s_wsum[v];
+        s_cnt[tid] = start;
+        if (tid < p.subs) row[tid] = (uint16_t)start;
+      }
+      if (tid == kBinMost) row[p.subs] = (uint16_t)cnt;
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kChunkIpt; ++j) {
+        if (at[j] != kNoPlace) {
+          at[j] += s_cnt[(ix[j] >> p.leaf_shift) & (p.subs - 1)];
+          s_16[at[j]] = (uint16_t)(ix[j] & ((1u << p.leaf_shift) - 1));
+        }
+      }
+      __syncthreads();
+      copy_out16(s_16, cidx + first, cnt);
+      __syncthreads();
+      // The values the same way: runs into LDS, then from chunk to leaf order.
+      load_runs(pval, s_src, s_off, runs, lo, hi, s_val);
+      __syncthreads();
+      T v[kChunkIpt];
+#pragma unroll
+      for (int j = 0; j < kChunkIpt; ++j) v[j] = s_val[tid + (uint32_t)j * kBinBlock];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kChunkIpt; ++j)
+        if (at[j] != kNoPlace) s_val[at[j]] = v[j];
+      __syncthreads();
+      copy_out16(s_val, cval + first, cnt);
+      __syncthreads();
     }
-    __syncthreads();
-    copy_out16(s_16, cidx + (size_t)c * kBinChunk, cnt);
-    __syncthreads();
-    // The values the same way: runs into LDS, then from chunk to leaf order.
-    load_runs(pval, s_src, s_off, runs, s_val);
-    __syncthreads();
-    T v[kChunkIpt];
-#pragma unroll
-    for (int j = 0; j < kChunkIpt; ++j) v[j] = s_val[tid + (uint32_t)j * kBinBlock];
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kChunkIpt; ++j)
-      if (at[j] != kNoPlace) s_val[at[j]] = v[j];
-    __syncthreads();
-    copy_out16(s_val, cval + (size_t)c * kBinChunk, cnt);
-    __syncthreads();
   }
 }
 
@@ -494,49 +585,75 @@ template <typename T>
 __global__ __launch_bounds__(kBinBlock) void leaf_scatter_kernel(
     T* __restrict__ table, uint32_t tlen, BinPlan p, bool aligned,
     const uint16_t* __restrict__ cidx, const T* __restrict__ cval,
-    const uint16_t* __restrict__ rows, const uint64_t* __restrict__ status, uint32_t gen) {
+    const uint16_t* __restrict__ rows, BinChunks chunks, const uint64_t* __restrict__ status, uint32_t gen) {
   if (status_flag(ld_agent(status), gen) == 0) return;
   constexpr uint32_t LEAF = kLeafBytes / sizeof(T);
   constexpr int U = 4;
+  // Rows of so many elements (indices that follow each other in this leaf, as
+  // behind a partition) are left for the whole block: 2^28 u32 in 256 streams
+  // 3.25 -> 2.82 ms.
+  constexpr uint32_t kLongRow = 1024, kLongRows = 64;
   __shared__ __align__(16) T s_leaf[LEAF];
   __shared__ uint32_t s_set[LEAF / 32];
+  __shared__ uint3 s_long[kLongRows];
+  __shared__ uint32_t s_longs;
+  // Elements [i0, b) of the chunk at c, `step` apart.
+  auto collect = [&](size_t c, uint32_t i0, uint32_t b, uint32_t step) {
+    for (; i0 < b; i0 += step * U) {
+      uint32_t d[U];
+      T v[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+        if (i0 + step * q < b) {
+          d[q] = cidx[c + i0 + step * q];
+          v[q] = cval[c + i0 + step * q];
+        }
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+        if (i0 + step * q < b) {
+          s_leaf[d[q]] = v[q];
+          atomicOr(&s_set[d[q] >> 5], 1u << (d[q] & 31u));
+        }
+    }
+  };
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
   const uint32_t leaves = (tlen - 1) / LEAF + 1;  // (tlen + LEAF may not fit 32 bits)
   for (uint32_t leaf = blockIdx.x; leaf < leaves; leaf += gridDim.x) {
     const uint32_t w = leaf >> p.sub_shift, sub = leaf & (p.subs - 1);
     const size_t l0 = (size_t)leaf * LEAF;
+    if (tid == 0) s_longs = 0;
     for (uint32_t i = tid; i < LEAF / 32; i += kBinBlock) s_set[i] = 0;
     __syncthreads();
-    for (uint32_t g0 = wid; g0 < p.groups; g0 += 16 * kWave) {
-      uint32_t s = 0, e = 0;
-      const uint32_t mine = g0 + 16 * lane;
-      if (mine < p.groups) {
-        const uint16_t* row = rows + ((size_t)w * p.groups + mine) * p.chunk_row + sub;
+    const uint32_t mine = chunks.counts[w];
+    for (uint32_t g0 = wid; g0 < mine; g0 += 16 * kWave) {
+      uint32_t s = 0, e = 0, at = 0;
+      const uint32_t g = g0 + 16 * lane;
+      if (g < mine) {
+        const uint32_t c = w * p.cap + g;
+        const uint16_t* row = rows + (size_t)c * p.chunk_row + sub;
+        at = chunks.at[c];
         s = row[0];
         e = row[1];
       }
-      const uint32_t many = min((uint32_t)kWave, (p.groups - g0 + 15) / 16);
+      const uint32_t many = min((uint32_t)kWave, (mine - g0 + 15) / 16);
       for (uint32_t k = 0; k < many; ++k) {
         const uint32_t a = readlane(s, (int)k), b = readlane(e, (int)k);
-        const size_t c = ((size_t)w * p.groups + g0 + 16 * k) * kBinChunk;
-        for (uint32_t i0 = a + lane; i0 < b; i0 += kWave * U) {
-          uint32_t d[U];
-          T v[U];
-#pragma unroll
-          for (int q = 0; q < U; ++q)
-            if (i0 + kWave * q < b) {
-              d[q] = cidx[c + i0 + kWave * q];
-              v[q] = cval[c + i0 + kWave * q];
-            }
-#pragma unroll
-          for (int q = 0; q < U; ++q)
-            if (i0 + kWave * q < b) {
-              s_leaf[d[q]] = v[q];
-              atomicOr(&s_set[d[q] >> 5], 1u << (d[q] & 31u));
-            }
+        const uint32_t c = readlane(at, (int)k);
+        if (b - a >= kLongRow) {
+          uint32_t j = 0;
+          if (lane == 0) j = atomicAdd(&s_longs, 1u);
+          j = (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
+          if (j < kLongRows) {
+            if (lane == 0) s_long[j] = make_uint3(c, a, b);
+            continue;
+          }
         }
+        collect((size_t)c * 8, a + lane, b, kWave);
       }
     }
+    __syncthreads();
+    for (uint32_t j = 0; j < min(s_longs, kLongRows); ++j)
+      collect((size_t)s_long[j].x * 8, s_long[j].y + tid, s_long[j].z, kBinBlock);
     __syncthreads();
     for (uint32_t i = tid * 4; i < LEAF; i += kBinBlock * 4) {
       const uint32_t m = (s_set[i >> 5] >> (i & 31u)) & 15u;

@@ -149,9 +149,11 @@ static BinPlan bin_plan(uint32_t tlen, uint32_t n, uint32_t tile, uint32_t leaf_
   p.tile_row = (p.windows + 8) & ~7u;
   p.chunk_row = (p.subs + 8) & ~7u;
   p.tiles = n / tile;
-  // A chunk is filled to 7/8 by indices spread evenly over the windows.
+  // A chunk is filled to 7/8 by indices spread evenly over the windows. (A tile
+  // has at most 4 times the mean in a window.)
   p.group = std::min(kBinMost, std::max(1u, (uint32_t)((uint64_t)kBinChunk * 7 / 8 * p.windows / tile)));
   p.groups = div_up(p.tiles, p.group);
+  p.cap = p.groups * div_up((uint64_t)p.group * (4 * tile / p.windows), kBinChunk);
   return p;
 }
 
@@ -179,7 +181,7 @@ static msv_status binned_gather(Ctx& c, const uint32_t* values, uint32_t vlen, c
   MSV_TRY(direct_gather(c, values, vlen, idx, out, n, looks, p.tiles * TILE));
   hipLaunchKernelGGL((bin_tiles_kernel<uint32_t, IPT, false>), dim3(std::min(p.tiles, cus)),
                      dim3(kBinBlock), 0, c.stream(), const_cast<uint32_t*>(values), vlen, idx, out, n,
-                     p, aligned, looks, pidx, ppos, (uint32_t*)nullptr, starts, (uint64_t*)nullptr, 0u);
+                     p, aligned, looks, pidx, ppos, (uint32_t*)nullptr, starts, BinChunks{}, (uint64_t*)nullptr, 0u);
   // The values replace the indices in place.
   hipLaunchKernelGGL((gather_window_kernel<uint32_t, TILE, 8>), dim3(div_up(cus, kXcds) * kXcds),
                      dim3(256), 0, c.stream(), values, vlen, p, pidx, pidx, starts, looks);
@@ -201,14 +203,23 @@ static msv_status binned_scatter(Ctx& c, const T* values, const uint32_t* idx, u
   uint32_t bits = 0;
   while ((1u << bits) < leaves) ++bits;
   const BinPlan p = bin_plan(olen, n, TILE, leaf_shift, (bits + 1) / 2);
-  const size_t slots = (size_t)p.windows * p.groups * kBinChunk;
+  // Room for the elements, for rounding each chunk to 8 of them and for less than
+  // a chunk left over in each part.
+  const size_t most = (size_t)p.tiles * TILE / kBinChunk + (size_t)p.windows * p.groups;
+  BinChunks chunks = {};
+  chunks.shard = (uint32_t)(((size_t)p.tiles * TILE / 8 + most) / kShards + 1 + kBinChunk / 8);
+  const size_t slots = (size_t)chunks.shard * 8 * kShards;
   uint32_t* pidx = (uint32_t*)c.scratch(sizeof(uint32_t) * (size_t)p.tiles * TILE);
   T* pval = (T*)c.scratch(sizeof(T) * (size_t)p.tiles * TILE);
   uint16_t* starts = (uint16_t*)c.scratch(sizeof(uint16_t) * (size_t)p.tiles * p.tile_row);
   uint16_t* cidx = (uint16_t*)c.scratch(sizeof(uint16_t) * slots);
   T* cval = (T*)c.scratch(sizeof(T) * slots);
-  uint16_t* rows = (uint16_t*)c.scratch(sizeof(uint16_t) * (size_t)p.windows * p.groups * p.chunk_row);
-  if (!pidx || !pval || !starts || !cidx || !cval || !rows) {
+  uint16_t* rows = (uint16_t*)c.scratch(sizeof(uint16_t) * (size_t)p.windows * p.cap * p.chunk_row);
+  chunks.used = (uint32_t*)c.scratch(sizeof(uint32_t) * kShards * kShardStep);
+  chunks.counts = (uint32_t*)c.scratch(sizeof(uint32_t) * p.windows);
+  chunks.at = (uint32_t*)c.scratch(sizeof(uint32_t) * (size_t)p.windows * p.cap);
+  if (!pidx || !pval || !starts || !cidx || !cval || !rows || !chunks.used || !chunks.counts ||
+      !chunks.at) {
     clear_error();
     return direct_scatter(c, values, idx, n, out, olen);
   }
@@ -219,13 +230,13 @@ static msv_status binned_scatter(Ctx& c, const T* values, const uint32_t* idx, u
   const uint32_t cus = (uint32_t)c.num_cus();
   hipLaunchKernelGGL((bin_tiles_kernel<T, IPT, true>), dim3(div_up(n, TILE)), dim3(kBinBlock), 0,
                      c.stream(), out, olen, idx, const_cast<T*>(values), n, p, aligned,
-                     (const uint32_t*)nullptr, pidx, (uint16_t*)nullptr, pval, starts, status, gen);
+                     (const uint32_t*)nullptr, pidx, (uint16_t*)nullptr, pval, starts, chunks, status, gen);
   hipLaunchKernelGGL((bin_leaves_kernel<T, TILE>), dim3(std::min(p.windows * p.groups, 2 * cus)),
-                     dim3(kBinBlock), 0, c.stream(), out, p, pidx, pval, starts, cidx, cval, rows,
+                     dim3(kBinBlock), 0, c.stream(), p, pidx, pval, starts, cidx, cval, rows, chunks,
                      status, gen);
   hipLaunchKernelGGL(leaf_scatter_kernel<T>, dim3(std::min(leaves, 2 * cus)), dim3(kBinBlock), 0,
-                     c.stream(), out, olen, p, ((uintptr_t)out & 15u) == 0, cidx, cval, rows, status,
-                     gen);
+                     c.stream(), out, olen, p, ((uintptr_t)out & 15u) == 0, cidx, cval, rows, chunks,
+                     status, gen);
   MSV_HIP(hipGetLastError());
   return MSV_OK;
 }

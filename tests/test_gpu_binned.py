@@ -18,6 +18,13 @@ def _order(kind, n, size, rng):
         return rng.permutation(size)[:n].astype(np.uint32)
     if kind == "half":  # twice the mean in half of the windows
         return rng.permutation(size // 2)[:n].astype(np.uint32)
+    if kind in ("third", "sixth"):  # four chunks of a group; more than the mean that tiles are binned with
+        return rng.permutation(size // (3 if kind == "third" else 6))[:n].astype(np.uint32)
+    if kind == "streams":  # the places of a stable partition into 256 parts: long rows of one leaf
+        part = rng.integers(0, 256, n).astype(np.uint8)
+        idx = np.empty(n, np.uint32)
+        idx[np.argsort(part, kind="stable")] = np.arange(n, dtype=np.uint32) + (size - n)
+        return idx
     if kind == "reversed":
         return np.arange(size - 1, size - 1 - n, -1, dtype=np.uint32)
     idx = rng.permutation(size)[:n].astype(np.uint32)  # "mixed": sorted and random stretches
@@ -37,6 +44,11 @@ def _order(kind, n, size, rng):
     (np.uint64, "random", N + 4095, N + 8193, 0),
     (np.uint64, "half", N, 2 * N, 1),
     (np.uint64, "mixed", 2 * N + 3, 2 * N + 5, 0),
+    (np.uint32, "third", N + 5, 3 * N + 1000, 0),
+    (np.uint32, "sixth", N, 6 * N + 9, 1),
+    (np.uint64, "third", N, 3 * N + 77, 0),
+    (np.uint32, "streams", 4 * N + 3, 4 * N + 3, 0),
+    (np.uint64, "streams", N + 1, N + 5, 1),
 ])
 def test_binned_scatter(exec_, dtype, kind, n, size, offset):
     rng = np.random.default_rng(n + size)
@@ -65,6 +77,25 @@ def test_binned_scatter_duplicates(exec_):
     hit[idx] = True
     assert np.array_equal(got != 0xFFFFFFFF, hit)
     assert np.array_equal(idx[got[hit]], np.flatnonzero(hit))
+
+
+@pytest.mark.parametrize("dtype", [np.uint32, np.uint64])
+@pytest.mark.parametrize("hot", [0.07, 0.9])
+def test_binned_scatter_hot_indices(exec_, dtype, hot):
+    """Some indices are there many times: one of their values ends up there."""
+    n, size = N + 20_000, 3 * N
+    rng = np.random.default_rng(int(hot * 100))
+    idx = rng.integers(0, size, n).astype(np.uint32)
+    few = np.array([0, 5, size - 1], np.uint32)
+    idx[rng.random(n) < hot] = few[2]
+    idx[rng.random(n) < hot / 4] = few[0]
+    out = exec_.to_device(np.full(size, 2**32 - 1, dtype))
+    m.vector.scatter(exec_, exec_.to_device(np.arange(n, dtype=dtype)), exec_.to_device(idx), out)
+    got = exec_.to_host(out)
+    hit = np.zeros(size, bool)
+    hit[idx] = True
+    assert np.array_equal(got != 2**32 - 1, hit)
+    assert np.array_equal(idx[got[hit].astype(np.int64)], np.flatnonzero(hit))
 
 
 def test_binned_scatter_replays(exec_):
