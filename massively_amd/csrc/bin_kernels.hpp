@@ -19,7 +19,7 @@
 //    LDS and writes whole lines (2^28 u32: 0.76 + 0.94 + 0.57 ms, from 6.0 with one look-back
 //    partition into 256 windows and random stores from L2).
 // Each tile decides for itself as well: one whose indices stay near each other
-// (sorted, reversed, clustered) is gathered or scattered
+// (sorted, reversed, clustered, rows of elements) is gathered or scattered
 // directly by bin_tiles_kernel.
 #pragma once
 
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
   static_assert(TILE <= 32768 && IPT % 8 == 0, "tile");
   __shared__ __align__(16) unsigned char s_mem[TILE * W];
   __shared__ uint32_t s_cnt[kBinMost], s_start[kBinMost + 1];
-  __shared__ uint32_t s_far, s_out, s_most, s_wsum[kBinMost / kWave];
+  __shared__ uint32_t s_far, s_joined, s_out, s_most, s_wsum[kBinMost / kWave];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t shift = p.leaf_shift + p.sub_shift;
   uint32_t tile = blockIdx.x;
@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
     uint16_t* row = starts + (size_t)tile * p.tile_row;
     __syncthreads();
     if (tid < kBinMost) s_cnt[tid] = 0;
-    if (tid == 0) s_far = s_out = s_most = 0;
+    if (tid == 0) s_far = s_joined = s_out = s_most = 0;
     __syncthreads();
 
     // Element 4 r + k of a thread is position (r * kBinBlock + tid) * 4 + k.
@@ -288,9 +288,23 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
         for (int k = 0; k < 4; ++k) ix[4 * r + k] = i + k < n ? idx[i + k] : 0xffffffffu;
       }
     }
+    if constexpr (SCATTER) {
+      // Lanes whose first index shares its line with the one before it.
+      constexpr int LINE = sizeof(T) == 4 ? kLineShift : kLineShift - 1;
+      uint32_t joined = 0;
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const uint32_t before = (uint32_t)__shfl_up((int)ix[4 * r + 3], 1);
+        joined += (uint32_t)__builtin_popcountll(ballot(lane > 0 && before >> LINE == ix[4 * r] >> LINE));
+      }
+      if (lane == 0) atomicAdd(&s_joined, joined);
+    }
     // Counted in registers first: the counts below would serialise on one
-    // LDS word for a tile that stays in a window or two.
+    // LDS word for a tile that stays in a window or two. Rows of some elements
+    // are written directly as well (half of the lanes go on in a line): 2^28 u32
+    // in rows of 64 3.5 -> 0.65 ms, of 16 2.7 -> 0.95; rows of 4 stay (2.6).
     bool spread = full && count_far(ix, shift, &s_far) * 2 >= TILE;
+    if constexpr (SCATTER) spread = spread && s_joined * 2 < TILE / 4;
     if constexpr (!SCATTER) {
       bool out = false;
 #pragma unroll

@@ -25,6 +25,10 @@ def _order(kind, n, size, rng):
         idx = np.empty(n, np.uint32)
         idx[np.argsort(part, kind="stable")] = np.arange(n, dtype=np.uint32) + (size - n)
         return idx
+    if kind.startswith("rows"):  # of some elements: written directly, or not
+        w = int(kind[4:])
+        return (rng.permutation(size // w)[:n // w + 1, None].astype(np.uint32) * np.uint32(w)
+                + np.arange(w, dtype=np.uint32)).reshape(-1)[:n]
     if kind == "reversed":
         return np.arange(size - 1, size - 1 - n, -1, dtype=np.uint32)
     idx = rng.permutation(size)[:n].astype(np.uint32)  # "mixed": sorted and random stretches
@@ -49,6 +53,9 @@ def _order(kind, n, size, rng):
     (np.uint64, "third", N, 3 * N + 77, 0),
     (np.uint32, "streams", 4 * N + 3, 4 * N + 3, 0),
     (np.uint64, "streams", N + 1, N + 5, 1),
+    (np.uint32, "rows16", N + 7, 2 * N, 1),
+    (np.uint32, "rows4", N, 2 * N, 0),
+    (np.uint64, "rows8", N + 9, 2 * N, 0),
 ])
 def test_binned_scatter(exec_, dtype, kind, n, size, offset):
     rng = np.random.default_rng(n + size)
