@@ -105,6 +105,22 @@ def test_binned_scatter_hot_indices(exec_, dtype, hot):
     assert np.array_equal(idx[got[hit].astype(np.int64)], np.flatnonzero(hit))
 
 
+@pytest.mark.parametrize("dtype", [np.uint32, np.uint64])
+@pytest.mark.parametrize("n,apart", [(1, 1), (63, 2), (4096, 1), (70_001, 3), (1_000_003, 64), (N + 4097, 16)])
+def test_scatter_sorted_indices(exec_, dtype, n, apart):
+    """Indices in order, some elements apart, up and down, from unaligned slices."""
+    size = n * apart + 5
+    up = np.arange(n, dtype=np.uint32) * np.uint32(apart) + np.uint32(2)
+    v = np.arange(1, n + 1, dtype=dtype)
+    for idx in (up, up[::-1].copy()):
+        di = exec_.to_device(np.concatenate([[9], idx]).astype(np.uint32)).slice(1, n + 1)
+        out = exec_.to_device(np.zeros(size, dtype))
+        m.vector.scatter(exec_, exec_.to_device(np.concatenate([[0], v]).astype(dtype)).slice(1, n + 1), di, out)
+        want = np.zeros(size, dtype)
+        want[idx] = v
+        assert np.array_equal(exec_.to_host(out), want), n
+
+
 def test_binned_scatter_replays(exec_):
     rng = np.random.default_rng(5)
     v = exec_.to_device(np.arange(N, dtype=np.uint32))
