@@ -751,17 +751,29 @@ msv_status run_jobs(Ctx& c, const msv_job* jobs, uint32_t count) {
     // the longest sorts run beside the rest: on the second stream, those of
     // 8-byte keys, or of 4-byte keys when there are none. 96 jobs of every
     // kind and type, 2^10..2^17 elements: 1049 -> 622 us. The fork and the join
-    // cost the host some 50 us, so shorter sorts (see kAsideMin) stay in line
-    // (128 jobs of at most 2^13 elements: 480 us in line, 535 forked).
+    // cost the host 20 to 50 us, so the sorts set aside take at least 100 us (see
+    // kAsideMin) and the rest, one launch after another, 60: about 1 us to 1024
+    // elements of a scan, reduce or copy_where, to 128 4-byte keys; 15 us a
+    // device-wide job, 60 a sort (u64 sort of 2^13 beside a u32 sort of 2^12: in
+    // line 150 us, forked 150; of 2^13: 183, 136; beside a scan of 2^10: 118, 136;
+    // 2^17: 244, 144; 64 such sorts beside 64 scans of 2^12: 408, 497).
     constexpr uint32_t kWide = 0x70, kNarrow = 0x0e;
     constexpr uint32_t kAsideMin = 1u << 14;  // 4-byte keys; half as many of 8 bytes
+    constexpr uint32_t kRestMin = 60;
     const uint32_t families = (mask & kWide) ? (mask & kWide) : (mask & kNarrow);
-    uint32_t longest = 0;
-    for (const msv_job& j : small)
-      if (j.kind == MSV_JOB_SORT_BY_KEY && (families >> (1 + sort_class(j)) & 1u))
-        longest = std::max(longest, j.n);
-    const uint32_t aside = longest >= (families & kWide ? kAsideMin / 2 : kAsideMin) ? families : 0u;
-    if (aside && (aside != mask || !large.empty())) {
+    uint32_t longest[kBatchFamilies] = {}, aside_longest = 0, rest = 0;
+    for (const msv_job& j : small) {
+      uint32_t& most = longest[j.kind == MSV_JOB_SORT_BY_KEY ? 1 + sort_class(j) : 0];
+      most = std::max(most, j.n);
+    }
+    for (int f = 0; f < kBatchFamilies; ++f) {
+      if (families >> f & 1u) aside_longest = std::max(aside_longest, longest[f]);
+      else rest += longest[f] / (f == 0 ? 1024u : 128u);
+    }
+    for (uint32_t i : large) rest += jobs[i].kind == MSV_JOB_SORT_BY_KEY ? 60u : 15u;
+    const uint32_t aside_min = families & kWide ? kAsideMin / 2 : kAsideMin;
+    const uint32_t aside = aside_longest >= aside_min && rest >= kRestMin ? families : 0u;
+    if (aside) {
       hipStream_t aux = c.fork();
       if (!aux) return MSV_ERR_LAUNCH;
       forked = true;

@@ -84,3 +84,34 @@ def test_graph_replays_long_sort_of_wide_keys(exec_):
         assert np.array_equal(exec_.to_host(out), order.astype(np.uint32)), rep
         assert np.array_equal(exec_.to_host(srt), h[order]), rep
     cap.graph.close()
+
+
+@pytest.mark.parametrize("beside", ["scans", "device-wide"])
+def test_graph_replays_forked_jobs(exec_, beside):
+    """A captured batch whose long sort runs on the second stream, beside scans of
+    its table and device-wide jobs."""
+    ex, n = exec_, 1 << 14
+    k, ok = ex.alloc(np.uint64, n), ex.alloc(np.uint64, n)
+    v, ov = ex.to_device(np.arange(n, dtype=np.uint32)), ex.alloc(np.uint32, n)
+    sizes = [1 << 17, 70_000, 5000] if beside == "scans" else [1 << 18, 150_000, 200_001, 140_000]
+    xs, ys = [ex.alloc(np.uint32, c) for c in sizes], [ex.alloc(np.uint32, c) for c in sizes]
+    jobs = [serve.Job("sort_by_key", k, ov, op=m.op.Less, inp2=v, out2=ok)]
+    jobs += [serve.Job("inclusive_scan", x, y, op=m.op.Add) for x, y in zip(xs, ys)]
+    serve.run_jobs(ex, jobs)  # (tunes its launches outside of the capture)
+    ex.sync()
+    with ex.capture() as cap:
+        serve.run_jobs(ex, jobs)
+    for rep in range(4):
+        mr.uniform_u64(ex, 0, 1 << 40, 7 + rep, k)
+        for x in xs:
+            mr.uniform_u32(ex, 0, 1000, 40 + rep, x)
+        ex.sync()
+        cap.graph.launch()
+        ex.sync()
+        hk = ex.to_host(k)
+        order = np.argsort(hk, kind="stable")
+        assert np.array_equal(ex.to_host(ok), hk[order]), rep
+        assert np.array_equal(ex.to_host(ov), order.astype(np.uint32)), rep
+        for x, y in zip(xs, ys):
+            assert np.array_equal(ex.to_host(y), np.cumsum(ex.to_host(x), dtype=np.uint32)), rep
+    cap.graph.close()
