@@ -858,9 +858,12 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
 //    it (no counts before, no look-back); elements stay in registers between
 //    digits and go through LDS whole. A digit costs about 7 us (its chain of
 //    ranks, barriers and LDS round trips), so only the highest DIGITS varying
-//    ones are sorted by, and runs that these leave equal are put in order by
-//    insertion, one thread a run. Runs longer than kLocalRun that are out of
-//    order (keys far from uniform) send the block through all its digits.
+//    ones are sorted by (more where these vary in too few bits to tell the
+//    elements apart: 65536 u32 keys of four digits with 10 values each, two
+//    digits and then all again 88.7 us, at once 48), and runs that these leave
+//    equal are put in order by insertion, one thread a run. Runs longer than
+//    kLocalRun that are out of order (keys far from uniform) send the block
+//    through all its digits.
 //    Two uses: a sort of at most TILE elements is one launch of one block
 //    (src/dst in `only`), and after the first pass of a short sort block g
 //    sorts the run of digit g (`local`, gbase: where the runs start).
@@ -914,19 +917,28 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_local_kernel(
   if (xlo) atomicOr(&s_diff[0], xlo);
   if (xhi) atomicOr(&s_diff[1], xhi);
   __syncthreads();
-  const uint32_t diff[2] = {s_diff[0], s_diff[1]};
+  const uint32_t diff[2] = {(uint32_t)__builtin_amdgcn_readfirstlane((int)s_diff[0]),
+                            (uint32_t)__builtin_amdgcn_readfirstlane((int)s_diff[1])};
   auto varies = [&](uint32_t p) { return ((diff[p / 4] >> (8 * (p & 3))) & 0xffu) != 0; };
-  // The lowest of the DIGITS highest varying digits, and whether any below varies.
-  uint32_t low = top;
+  // The lowest of the DIGITS highest varying digits, or of as many as have two
+  // varying bits more than the elements need, and whether any below varies.
+  uint32_t low = DIGITS >= P ? 0u : top;
   bool below_varies = false;
-  for (uint32_t p = top, left_out = DIGITS; p-- > 0;) {
-    if (!varies(p)) continue;
-    if (left_out == 0) {
-      below_varies = true;
-      break;
+  if constexpr (DIGITS < P) {
+    const int need = 32 - __builtin_clz(cnt) + 2;
+    int digits = 0, bits = 0;
+#pragma unroll
+    for (int p = P - 1; p >= 0; --p) {
+      const uint32_t varying = (diff[p / 4] >> (8 * (p & 3))) & 0xffu;
+      if (varying == 0 || (uint32_t)p >= top) continue;
+      if (digits >= DIGITS && bits >= need) {
+        below_varies = true;
+      } else {
+        ++digits;
+        bits += __builtin_popcount(varying);
+        low = (uint32_t)p;
+      }
     }
-    --left_out;
-    low = p;
   }
   const uint64_t lt = lanemask_lt();
   bool in_lds = false;

@@ -68,6 +68,31 @@ def test_sort_local_range(exec_, dtype, value, spread):
         assert np.array_equal(exec_.to_host(s), k[order]), n
 
 
+@pytest.mark.parametrize("dtype,value", [(np.uint32, np.uint32), (np.uint64, np.uint32), (np.uint64, np.uint64),
+                                         (np.uint64, None)])
+@pytest.mark.parametrize("values", [(0, 1), (0, 255), (3, 4, 7, 99)])
+def test_sort_few_values_in_high_digits(exec_, dtype, value, values):
+    """Short sorts whose highest varying digits tell few elements apart: those that
+    vary in few bits take more digits at once, those of 0 and 255 leave runs that
+    are too long to repair and start over."""
+    rng = np.random.default_rng(len(values))
+    width = np.dtype(dtype).itemsize
+    for n, top in ((17, False), (1500, False), (4096, False), (100_003, True), (300_000, True), (12_000, False)):
+        k = rng.integers(0, 256, (n, width), dtype=np.uint8)  # little endian digits
+        few = np.array(values, np.uint8)
+        for d in range(width - 3 - top, width - top):
+            k[:, d] = few[rng.integers(0, few.size, n)]
+        k = k.view(dtype).reshape(-1)
+        order = np.argsort(k, kind="stable")
+        dk = exec_.to_device(k)
+        if value is None:
+            assert np.array_equal(exec_.to_host(m.vector.sort(exec_, dk, m.op.Less)), k[order]), n
+            continue
+        v, s = m.vector.radix_sort_by_key(exec_, dk, exec_.to_device(np.arange(n, dtype=value)), return_keys=True)
+        assert np.array_equal(exec_.to_host(v), order.astype(value)), n
+        assert np.array_equal(exec_.to_host(s), k[order]), n
+
+
 @pytest.mark.parametrize("dtype,value", [(np.uint64, np.uint32), (np.int64, None), (np.float64, np.uint64)])
 @pytest.mark.parametrize("spread", ["uniform", "sorted", "pairs", "runs", "half", "one digit"])
 def test_sort_high_digits_and_repair(exec_, dtype, value, spread):
