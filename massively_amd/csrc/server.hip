@@ -91,6 +91,9 @@ struct msv_server {
   uint64_t used = 0;
   uint64_t outstanding = 0;  // submitted and not yet done
   bool stop = false;
+  // Results are copied on a stream of their own: a copy on the legacy stream fails
+  // while the worker captures a batch.
+  hipStream_t copies = nullptr;
   std::thread worker;
 };
 
@@ -444,6 +447,8 @@ msv_status msv_server_create(const msv_server_config* cfg, msv_server** out) {
   s->slots.resize(s->cfg.streams);
   for (Slot& sl : s->slots) {
     msv_status st = msv_executor_create(cfg->device, &sl.ex);
+    if (st == MSV_OK && !s->copies && hipStreamCreateWithFlags(&s->copies, hipStreamNonBlocking) != hipSuccess)
+      st = MSV_ERR_LAUNCH;
     if (st == MSV_OK && hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming) != hipSuccess)
       st = MSV_ERR_LAUNCH;
     if (st == MSV_OK && hipHostMalloc((void**)&sl.h_counts, sizeof(uint32_t) * s->cfg.max_batch) !=
@@ -467,6 +472,7 @@ msv_status msv_server_create(const msv_server_config* cfg, msv_server** out) {
         if (t.ev) hipEventDestroy(t.ev);
         if (t.ex) msv_executor_destroy(t.ex);
       }
+      if (s->copies) hipStreamDestroy(s->copies);
       delete s;
       set_error(st, 0, 0, "server resources could not be created");
       return st;
@@ -499,6 +505,7 @@ msv_status msv_server_destroy(msv_server* s) {
     hipEventDestroy(sl.ev);
     msv_executor_destroy(sl.ex);
   }
+  hipStreamDestroy(s->copies);
   delete s;
   return MSV_OK;
 }
@@ -613,8 +620,10 @@ msv_status msv_server_result(msv_server* s, uint64_t ticket, void* out, uint64_t
     ++q->readers;
   }
   hipError_t e = hipSetDevice(s->cfg.device);
-  if (e == hipSuccess && need) e = hipMemcpy(out, src, need, hipMemcpyDeviceToHost);
-  if (e == hipSuccess && out2 && src2 && need2) e = hipMemcpy(out2, src2, need2, hipMemcpyDeviceToHost);
+  if (e == hipSuccess && need) e = hipMemcpyAsync(out, src, need, hipMemcpyDeviceToHost, s->copies);
+  if (e == hipSuccess && out2 && src2 && need2)
+    e = hipMemcpyAsync(out2, src2, need2, hipMemcpyDeviceToHost, s->copies);
+  if (e == hipSuccess) e = hipStreamSynchronize(s->copies);
   {
     std::lock_guard<std::mutex> g(s->mu);
     --q->readers;
