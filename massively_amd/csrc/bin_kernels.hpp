@@ -339,10 +339,13 @@ __global__ __launch_bounds__(kBinBlock, IPT * (SCATTER ? sizeof(T) : 4) == 64 ? 
       // from an index that is there many times (then it also follows itself):
       // only one of its values stays.
       const int32_t over = (int32_t)s_most - (int32_t)(TILE / p.windows);
-      bool twin = false;
+      bool twins = false;
+      if (over > 0 && (uint32_t)(over * over) > 36 * (TILE / p.windows)) {
 #pragma unroll
-      for (int j = 1; j < IPT; ++j) twin = twin || ((j & 3) && ix[j] == ix[j - 1] && ix[j] < tlen);
-      if (over > 0 && (uint32_t)(over * over) > 36 * (TILE / p.windows) && __syncthreads_or(twin)) {
+        for (int j = 1; j < IPT; ++j) twins = twins || ((j & 3) && ix[j] == ix[j - 1] && ix[j] < tlen);
+        twins = __syncthreads_or(twins);
+      }
+      if (twins) {
         drop_repeats<IPT>(ix, tlen, reinterpret_cast<uint32_t*>(s_mem));
         if (tid < kBinMost) s_cnt[tid] = 0;
         if (tid == 0) s_most = 0;

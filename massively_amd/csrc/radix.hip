@@ -48,7 +48,8 @@ template <int EW>
 constexpr int radix_ipt() { return EW <= 2 ? 16 : 8; }
 // Onesweep passes run 1024-thread blocks, two per CU at 64 VGPRs (8 waves per
 // SIMD): 10 keys per thread for 4-byte elements, 8 for wider ones, the most
-// that fit those registers and LDS (63-78 KB a block). From 8, 6, 5 and 5 keys
+// that fit those registers and LDS (52 KB a block for 4-byte elements, 77 for
+// wider ones). From 8, 6, 5 and 5 keys
 // (radix_onesweep_kernel says how they fit): 2^28 u32 keys 5.58 -> 4.27 ms,
 // 2^28 u32 + u32 7.31 -> 5.62, 2^27 u64 keys 6.96 -> 5.32, u64 + u32 9.35 ->
 // 7.22, u64 + u64 10.53 -> 9.22. Slower: shapes that spill (12 or 14 for
@@ -68,7 +69,8 @@ constexpr uint32_t kRadixSmall = 1u << 18, kRadixMiddle = 7u << 18;
 
 // The local sort's elements per thread (two blocks' LDS per CU), and the sorts
 // that try one pass and local sorts: where the average run fills at most 7/8 of
-// a block. Whole sorts with a u32 payload, before -> now (us): 2000 u32 38.6 ->
+// a block (1.83 million elements of up to 8 bytes, 1.15 of 12, 0.92 of 16). Whole
+// sorts with a u32 payload, before -> now (us): 2000 u32 38.6 ->
 // 15.4, u64 70 -> 16.7; 8000 u32 47.6 -> 31.5, u64 91 -> 46;
 // 65536 u32 52.8 -> 31.5, u64 102 -> 44.4; 2^20 u32 88.8 -> 56.5, u64 179
 // -> 72.5. Keys whose highest byte has too few values keep all their passes (f32
@@ -107,20 +109,30 @@ static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, ui
   const size_t vofs = radix_split(EW) ? (((size_t)n * sizeof(K) + 255) & ~(size_t)255) : 0;
   void* aos0 = c.scratch(elem_bytes + 256);
   void* aos1 = c.scratch(elem_bytes + 256);
-  RadixPass* table = (RadixPass*)c.scratch(sizeof(RadixPass) * P);
+  RadixPass* table = (RadixPass*)c.scratch(sizeof(RadixPass) * 2 * P);
   if (!aos0 || !aos1 || !table) return MSV_ERR_OUT_OF_MEMORY;
   if (sched != 0) {
     // Onesweep: histograms of every digit position in one read of the keys,
     // then one look-back pass per digit position that needs one.
     RadixPlan q = {};
-    uint32_t* hist = (uint32_t*)c.scratch(sizeof(uint32_t) * (kRadixBins * P + P));
-    q.gbase = (uint32_t*)c.scratch(sizeof(uint32_t) * kRadixBins * P);
-    q.local = (RadixLocal*)c.scratch(sizeof(RadixLocal));
-    if (!hist || !q.gbase || !q.local) return MSV_ERR_OUT_OF_MEMORY;
-    q.hist = hist;
-    q.tile_counters = hist + kRadixBins * P;
-    q.table = table;
     q.local_max = n <= LTILE / 8 * 7 * kRadixBins ? LTILE : 0u;
+    // Long sorts of 8-byte keys stop at a digit that samples choose, repair what
+    // that left, and start over with every digit when that was too much.
+    const bool repair = P == 8 && n > kRepairMin && q.local_max == 0;
+    constexpr uint32_t kHist = kRadixBins * P, kRep = sizeof(RadixRepair) / 4;
+    const uint32_t marks = repair ? div_up(n, 32u) : 0u;  // a bit per element
+    uint32_t* hist = (uint32_t*)c.scratch(sizeof(uint32_t) * (kHist + kRep + (size_t)marks));
+    RadixRepair* rep = (RadixRepair*)(hist + kHist);
+    RadixSample* sample = repair ? (RadixSample*)c.scratch(sizeof(RadixSample)) : nullptr;
+    q.gbase = (uint32_t*)c.scratch(sizeof(uint32_t) * kHist);
+    q.local = (RadixLocal*)c.scratch(sizeof(RadixLocal));
+    q.tile_counters = (uint32_t*)c.scratch(sizeof(uint32_t) * 2 * P);
+    if (!hist || !q.gbase || !q.local || !q.tile_counters || (repair && !sample)) return MSV_ERR_OUT_OF_MEMORY;
+    q.launches = repair ? kFirstPasses + P : P;
+    q.hist = hist;
+    q.table = table;
+    q.sample = sample;
+    q.rep = rep;
     q.in_k = keys;
     q.in_v = vals;
     q.out_k = out_k;
@@ -128,78 +140,71 @@ static msv_status radix_sort_impl(Ctx& c, const void* keys, const void* vals, ui
     q.aos0 = aos0;
     q.aos1 = aos1;
     q.vofs = vofs;
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(div_up(kRadixBins * P, 256)), dim3(256), 0,
-                       c.stream(), hist, (uint32_t)(kRadixBins * P), 0u);
     const uint32_t hist_blocks = min(div_up(n, 256u * 16u), (uint32_t)c.num_cus() * 8u);
-    hipLaunchKernelGGL((radix_hist_kernel<K, MODE, 256>), dim3(hist_blocks), dim3(256), 0,
-                       c.stream(), (const K*)keys, n, hist);
-    // Long sorts of 8-byte keys stop at a digit that a sample chooses, repair
-    // what that left, and start over with every digit when that was too much.
-    const bool repair = P == 8 && n > kRepairMin && q.local_max == 0;
-    RadixRepair* rep = nullptr;
     if constexpr (P == 8) {
       if (repair) {
-        rep = (RadixRepair*)c.scratch(sizeof(RadixRepair));
-        if (!rep) return MSV_ERR_OUT_OF_MEMORY;
-        q.rep = rep;
-        hipLaunchKernelGGL((radix_sample_kernel<K, MODE>), dim3(1), dim3(1024), 0, c.stream(),
-                           (const K*)keys, n, hist, rep);
+        const uint32_t words = kHist + kRep + marks;
+        hipLaunchKernelGGL((radix_begin_kernel<K, MODE>), dim3(kSamples * kLows + min(div_up(words, 4096u), 256u)),
+                           dim3(1024), 0, c.stream(), (const K*)keys, n, sample, hist, words);
+        hipLaunchKernelGGL((radix_hist_kernel<K, MODE, 256, true>), dim3(hist_blocks), dim3(256), 0,
+                           c.stream(), (const K*)keys, n, hist, sample, rep);
       }
     }
+    if (!repair) {
+      hipLaunchKernelGGL(fill_u32_kernel, dim3(div_up(kHist, 256)), dim3(256), 0, c.stream(), hist, kHist, 0u);
+      hipLaunchKernelGGL((radix_hist_kernel<K, MODE, 256>), dim3(hist_blocks), dim3(256), 0, c.stream(),
+                         (const K*)keys, n, hist, (const RadixSample*)nullptr, (RadixRepair*)nullptr);
+    }
+    hipLaunchKernelGGL((radix_onesweep_plan_kernel<P>), dim3(1), dim3(kRadixBins), 0, c.stream(), q, n);
+    MSV_HIP(hipGetLastError());
     constexpr int OBLOCK = radix_onesweep_block<EW>();
     constexpr int OIPT = radix_onesweep_ipt<EW>();
     const int ipt = n <= kRadixSmall ? 2 : (n <= kRadixMiddle ? 6 : OIPT);
     const uint32_t otiles = div_up(n, (uint32_t)OBLOCK * ipt);
-    // Slot p runs the p-th pass of the plan; passes it leaves out end at once.
-    auto passes = [&]() -> msv_status {
-      hipLaunchKernelGGL((radix_onesweep_plan_kernel<P>), dim3(1), dim3(kRadixBins), 0, c.stream(), q, n);
+    // Launch l runs entry `first` of the pass table, or after a repair that gave up
+    // (rep) entry `again`; entries without a pass end at once.
+    auto pass = [&](uint32_t l, int first, int again, const RadixRepair* after) -> msv_status {
+      uint64_t *counter, *status;
+      uint32_t gen;
+      MSV_TRY(c.lookback((size_t)otiles * kRadixBins, &counter, &status, &gen));
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(otiles), dim3(OBLOCK), 0, c.stream(), table, first, again, after,
+                           q.gbase, q.tile_counters + l, status, gen, n);
+      };
+      if (ipt == 2) launch(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 2>);
+      else if (ipt == 6) launch(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 6>);
+      else launch(radix_onesweep_kernel<K, MODE, EW, OBLOCK, OIPT>);
       MSV_HIP(hipGetLastError());
-      for (int p = 0; p < P; ++p) {
-        uint64_t *counter, *status;
-        uint32_t gen;
-        MSV_TRY(c.lookback((size_t)otiles * kRadixBins, &counter, &status, &gen));
-        auto pass = [&](auto kernel) {
-          hipLaunchKernelGGL(kernel, dim3(otiles), dim3(OBLOCK), 0, c.stream(), table, p, q.gbase,
-                             q.tile_counters, status, gen, n);
-        };
-        if (ipt == 2) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 2>);
-        else if (ipt == 6) pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, 6>);
-        else pass(radix_onesweep_kernel<K, MODE, EW, OBLOCK, OIPT>);
-        if (p == 0 && q.local_max)
-          hipLaunchKernelGGL((radix_local_kernel<K, MODE, EW, 1024, LIPT, 2>), dim3(kRadixBins),
-                             dim3(1024), 0, c.stream(), q.local, q.gbase, RadixPass{}, n);
-        MSV_HIP(hipGetLastError());
-      }
       return MSV_OK;
     };
-    MSV_TRY(passes());
+    for (int p = 0; p < (repair ? kFirstPasses : P); ++p) {
+      MSV_TRY(pass((uint32_t)p, p, p, nullptr));
+      if (p == 0 && q.local_max) {
+        hipLaunchKernelGGL((radix_local_kernel<K, MODE, EW, 1024, LIPT, 2>), dim3(kRadixBins),
+                           dim3(1024), 0, c.stream(), q.local, q.gbase, RadixPass{}, n);
+        MSV_HIP(hipGetLastError());
+      }
+    }
     if constexpr (P == 8) {
       if (repair) {
-        // The element buffers are free by now. The first holds the listed runs,
-        // their counts and a mark per element (less than n words in all), the second the
-        // places that long runs move through.
+        // The element buffers are free by now, if the passes are done. The first
+        // holds the listed runs and their counts (less than n words in all), the
+        // second the places that long runs move through.
         const uint32_t chunk = div_up(div_up(n, 8u * (uint32_t)c.num_cus()), 2048u) * 2048u;
-        const uint32_t blocks = div_up(n, chunk), words = div_up(n, 32u);
+        const uint32_t blocks = div_up(n, chunk);
         uint32_t* const list = (uint32_t*)aos0;
         uint32_t* const counts = list + (size_t)blocks * (chunk / 2 + 1);
-        uint32_t* const marks = counts + blocks;
         K* const out = (K*)out_k;
-        hipLaunchKernelGGL(radix_repair_clear_kernel, dim3(c.num_cus()), dim3(256), 0, c.stream(), rep,
-                           marks, words);
         hipLaunchKernelGGL((radix_repair_find_kernel<K, MODE>), dim3(blocks), dim3(256), 0, c.stream(),
-                           (const K*)out, n, chunk, ((uintptr_t)out & 15u) == 0, rep, marks, list, counts);
+                           (const K*)out, n, chunk, ((uintptr_t)out & 15u) == 0, rep, hist + kHist + kRep,
+                           list, counts);
         hipLaunchKernelGGL((radix_repair_kernel<K, MODE, VS / 4>), dim3(blocks), dim3(1024), 0, c.stream(),
                            out, (uint32_t*)out_v, (K*)aos1, (uint32_t*)((char*)aos1 + (size_t)n * sizeof(K)),
                            n, chunk, rep, list, counts);
         MSV_HIP(hipGetLastError());
-        // Starting over reads what the first passes left in the output (equal keys
-        // still in input order): the caller's arrays may have been written by
-        // then, when a job sorts its keys or its values in place. It is sound
-        // because a repair follows at least four passes, so these are five or more.
-        q.in_k = out_k;
-        q.in_v = out_v;
-        q.redo = true;
-        return passes();
+        // The last passes where there was nothing to repair (every digit has one), or all again.
+        for (int p = 0; p < P; ++p)
+          MSV_TRY(pass((uint32_t)(kFirstPasses + p), p < P - kFirstPasses ? kFirstPasses + p : -1, P + p, rep));
       }
     }
     return MSV_OK;

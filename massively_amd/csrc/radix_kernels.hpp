@@ -410,6 +410,111 @@ __global__ __launch_bounds__(BLOCK) void radix_downsweep_kernel(
 
 
 // ---- onesweep: one histogram pass, then one pass per digit ---------------------
+// How a long sort of 8-byte keys goes (9).
+struct RadixRepair {
+  uint32_t low;   // passes run from this digit; 0: all of them do
+  uint32_t redo;  // the repair gave up: every digit's pass runs
+  uint32_t near;  // 8 - the highest digit in which a key differs from a hot key that
+                  // it shares the digits from the looked-at one on with; 0: none does
+};
+constexpr uint32_t kSample = 8192, kSamples = 16;  // keys of a sample (most), samples
+constexpr uint32_t kHots = 128;                    // most hot keys of a sample
+constexpr uint32_t kLows = 5;                      // digits 0 .. 4 are looked at (at least 4 get a pass)
+struct RadixSample {
+  uint32_t clash[kLows][kSamples];  // [low]: pairs of different keys that share the digits from low on
+  uint32_t varying[kSamples];   // bit p: digit p varies
+  uint32_t most[kSamples];      // how often the most frequent key is there
+  uint32_t hots[kSamples];      // keys that are there at least 4 times (kHots at most),
+  uint32_t heavy[kSamples];     // and first those that are there 16 times (all of them counted)
+  uint64_t hot[kSamples][kHots];
+};
+constexpr int kFirstPasses = 7;  // most digits that get a pass before a repair
+// Keys of a sample of n keys (a quarter of them are looked at in 9 us, all in 30),
+// and the pairs that may clash in all samples.
+__device__ inline uint32_t sample_size(uint32_t n) { return n >= 1u << 25 ? kSample : kSample / 4; }
+__device__ inline uint32_t clash_limit(uint32_t n) {
+  const uint32_t size = sample_size(n), pairs = kSamples * (size / 2) * size;
+  return n >= 1u << 29 ? 0u : max(1u, pairs / 4 / n);
+}
+
+// The digit that the passes of n keys start from, or 0, by the rules of (9).
+__device__ inline uint32_t choose_low(uint32_t n, uint32_t varying, bool hot, const uint32_t* clash) {
+  const uint32_t bits = 4 + 32 - (uint32_t)__builtin_clz(n - 1);
+  uint32_t want = (bits + 7) / 8 + (hot ? 1 : 0), low = 8;
+  while (low > 0 && want > 0) want -= varying >> --low & 1u;
+  const uint32_t limit = clash_limit(n);
+  for (; low > 0; --low)
+    if ((varying >> (low - 1) & 1u) && clash[low] <= limit) break;
+  return low;
+}
+
+// The samples' sums (all threads of the block call; s_sum: kLows + 2 words).
+__device__ inline void sum_samples(const RadixSample* __restrict__ sample, uint32_t* s_sum) {
+  const uint32_t tid = threadIdx.x;
+  if (tid < kLows + 2) s_sum[tid] = 0;
+  __syncthreads();
+  if (tid < kLows * kSamples) atomicAdd(&s_sum[tid / kSamples], (&sample->clash[0][0])[tid]);
+  if (tid < kSamples) {
+    atomicOr(&s_sum[kLows], sample->varying[tid]);
+    atomicMax(&s_sum[kLows + 1], sample->most[tid]);
+  }
+  __syncthreads();
+}
+__device__ inline uint32_t sampled_low(uint32_t n, const uint32_t* s_sum) {
+  return choose_low(n, s_sum[kLows], s_sum[kLows + 1] > sample_size(n) / 64, s_sum);
+}
+
+// The samples' hot keys in LDS, two to a bucket of the digits that the passes
+// may start from. Returns 8 times that digit, or 0 when there is nothing to look
+// at; *lost: a heavy key has no room (others are just not looked at). An empty
+// place holds the first hot key: what shares its digits is near a hot key in any
+// case.
+constexpr uint32_t kHotBuckets = 256;  // (with 512 a CU holds three blocks of the histogram, not four)
+__device__ inline uint32_t hot_bucket(uint64_t word, uint32_t shift) {  // shift in 8 .. 32
+  const uint32_t high = (uint32_t)(word >> 32), rest = shift < 32 ? (uint32_t)word >> (shift & 31u) : 0u;
+  return ((high ^ rest ^ (rest << 13)) * 2654435761u) >> 24;
+}
+template <int BLOCK>
+__device__ inline uint32_t hot_table(const RadixSample* __restrict__ sample, uint32_t n, uint64_t* s_hot,
+                                     bool* lost) {
+  constexpr int PER = (int)(kSamples * kHots / BLOCK);
+  static_assert(BLOCK % kHots == 0 && PER > 0, "a thread's keys are of one place in their samples");
+  __shared__ uint32_t s_sum[kLows + 2], s_hots[kSamples], s_heavy[kSamples], s_first;
+  const uint32_t at = threadIdx.x % kHots, sub = threadIdx.x / kHots;
+  uint64_t word[PER];  // (those past a sample's hot keys are not used)
+#pragma unroll
+  for (int j = 0; j < PER; ++j) word[j] = sample->hot[sub + j * (BLOCK / kHots)][at];
+  if (threadIdx.x < kSamples) {
+    s_hots[threadIdx.x] = sample->hots[threadIdx.x];
+    s_heavy[threadIdx.x] = sample->heavy[threadIdx.x];
+  }
+  if (threadIdx.x == 0) s_first = kSamples;
+  sum_samples(sample, s_sum);
+  if (threadIdx.x < kSamples && s_hots[threadIdx.x] > 0) atomicMin(&s_first, threadIdx.x);
+  __syncthreads();
+  const uint32_t shift = 8 * sampled_low(n, s_sum), first = s_first;
+  *lost = false;
+  if (shift == 0 || first == kSamples) return 0;
+  const uint64_t empty = sample->hot[first][0];
+  for (uint32_t i = threadIdx.x; i < 2 * kHotBuckets; i += BLOCK) s_hot[i] = empty;
+  __syncthreads();
+  for (int light = 0; light < 2; ++light) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t s = sub + j * (BLOCK / kHots);
+      *lost = *lost || s_heavy[s] > kHots;
+      if (at >= s_hots[s] || (at >= s_heavy[s]) != (light == 1)) continue;
+      const uint64_t w = word[j];
+      unsigned long long* to = (unsigned long long*)&s_hot[2 * hot_bucket(w, shift)];
+      uint64_t was = atomicCAS(to, (unsigned long long)empty, (unsigned long long)w);
+      if (was != empty && was != w) was = atomicCAS(to + 1, (unsigned long long)empty, (unsigned long long)w);
+      *lost = *lost || (was != empty && was != w && light == 0);
+    }
+    __syncthreads();
+  }
+  return shift;
+}
+
 // 5. Global digit histograms of every digit position in one read of the keys:
 //    hist[p * 256 + d] = number of keys whose digit p is d. Each thread reads
 //    16 keys per step with 16-byte loads (all in flight before the first is
@@ -421,9 +526,13 @@ __global__ __launch_bounds__(BLOCK) void radix_downsweep_kernel(
 //    positions take one LDS add per key and no per-key test (per key and
 //    position, a uniformity test had cost more instructions than the add).
 //    (Its last block making the plan, to save that launch, gained 0-2 us.)
-template <typename K, int MODE, int BLOCK>
+//    SAMPLE: a long sort of 8-byte keys (9), whose hot keys every key is
+//    compared with on the way.
+template <typename K, int MODE, int BLOCK, bool SAMPLE = false>
 __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__ keys, uint32_t n,
-                                                          uint32_t* __restrict__ hist) {
+                                                          uint32_t* __restrict__ hist,
+                                                          const RadixSample* __restrict__ sample,
+                                                          RadixRepair* __restrict__ rep) {
   using U = typename Bits<K>::U;
   constexpr int P = sizeof(K);
   constexpr int KPT = 16;                   // keys per thread per step
@@ -434,6 +543,25 @@ __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__
   uint32_t* s_h = s_hw[tid / kWave];
   for (uint32_t i = tid; i < (uint32_t)(NW * P * kRadixBins); i += BLOCK) (&s_hw[0][0])[i] = 0;
   __syncthreads();
+  uint32_t shift = 0, near = 0;  // shift 0: no hot keys to compare with
+  __shared__ __align__(16) uint64_t s_hot[SAMPLE ? 2 * kHotBuckets : 2];
+  if constexpr (SAMPLE) {
+    bool lost;
+    shift = hot_table<BLOCK>(sample, n, s_hot, &lost);
+    if (lost) near = 8;
+  }
+  auto compare = [&](U word) {
+    if constexpr (SAMPLE) {
+      const uint32_t b = hot_bucket((uint64_t)word, shift);
+      const uint4 hot = *reinterpret_cast<const uint4*>(s_hot + 2 * b);
+      const uint32_t low_word = (uint32_t)word, high = (uint32_t)((uint64_t)word >> 32);
+      // The same digits from shift (8 .. 32) on, but not the same key: the
+      // difference is in [1, 2^shift).
+      const uint32_t x0 = low_word ^ hot.x, x1 = low_word ^ hot.z, span = 0xffffffffu >> (32 - shift);
+      if (high == hot.y && x0 - 1 < span) near = max(near, (32 + (uint32_t)__builtin_clz(x0)) / 8 + 1);
+      if (high == hot.w && x1 - 1 < span) near = max(near, (32 + (uint32_t)__builtin_clz(x1)) / 8 + 1);
+    }
+  };
   const bool aligned = ((uintptr_t)keys & 15u) == 0;
   const size_t step = (size_t)gridDim.x * BLOCK * KPT;
   for (size_t b0 = (size_t)blockIdx.x * BLOCK * KPT; b0 < n; b0 += step) {
@@ -452,6 +580,10 @@ __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__
           else key = bit_cast<K>(((uint64_t)qq[2 * k + 1] << 32) | qq[2 * k]);
           w[r * V + k] = order_bits<K, MODE>(key);
         }
+      }
+      if (SAMPLE && shift != 0) {
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) compare(w[j]);
       }
       // Bytes in which some key of the wave's step differs from its first key.
       uint32_t lo0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)w[0]);
@@ -496,6 +628,7 @@ __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__
     }
 #pragma unroll
     for (int j = 0; j < KPT; ++j) {
+      if (SAMPLE && shift != 0 && ok[j]) compare(w[j]);
       const uint64_t valid = ballot(ok[j]);
 #pragma unroll
       for (int p = 0; p < P; ++p) {
@@ -516,6 +649,10 @@ __global__ __launch_bounds__(BLOCK) void radix_hist_kernel(const K* __restrict__
     for (int w = 0; w < NW; ++w) c += s_hw[w][i];
     if (c) atomicAdd(&hist[i], c);
   }
+  if constexpr (SAMPLE) {
+    near = wave_reduce<uint32_t, OP_MAX>(near);
+    if (near && (tid & 63u) == 0) atomicMax(&rep->near, near);
+  }
 }
 
 // What the local sort (8) does after the first pass: sorts every run of equal
@@ -524,12 +661,6 @@ struct RadixLocal {
   uint32_t on;
   uint32_t top;
   RadixPass pass;  // its source and destination
-};
-
-// How a long sort of 8-byte keys goes (9).
-struct RadixRepair {
-  uint32_t low;   // passes run from this digit; 0: all of them do
-  uint32_t redo;  // the repair gave up: every digit's pass runs
 };
 
 // 6. Onesweep plan (one block of 256 threads): the exclusive scan of every
@@ -541,17 +672,24 @@ struct RadixRepair {
 //    local_max > 0: when at least three positions need a pass and no digit of
 //    the highest holds more than local_max keys, only that position gets a
 //    pass, and `local` the rest.
+//    sample: the passes may start at a higher digit (9), chosen here into rep; a
+//    second table then has the passes over every digit, for when the repair
+//    gives up. These read what the first passes left in the output (equal keys
+//    still in input order): the caller's arrays may have been written by then,
+//    when a job sorts its keys or its values in place. (At least four digits are
+//    passed over before a repair, so they are five or more.)
 //    vofs = 0: the intermediate buffers hold interleaved elements; else each
 //    holds the keys and, vofs bytes in, the values (the two-phase passes).
 struct RadixPlan {
   const uint32_t* hist;     // [P][256]
-  RadixPass* table;         // [P]
+  RadixPass* table;         // [P], or [2 P] with a sample
   uint32_t* gbase;          // [P][256]
-  uint32_t* tile_counters;  // [P]
+  uint32_t* tile_counters;  // one to a launch of the passes, `launches` of them
+  uint32_t launches;
   RadixLocal* local;
   uint32_t local_max;
-  const RadixRepair* rep;   // where the passes start (null: at digit 0)
-  bool redo;                // the second plan, after a repair
+  const RadixSample* sample;  // null: the passes start at digit 0
+  RadixRepair* rep;
   const void *in_k, *in_v;
   void *out_k, *out_v, *aos0, *aos1;
   size_t vofs;
@@ -559,66 +697,75 @@ struct RadixPlan {
 
 template <int P>
 __global__ __launch_bounds__(kRadixBins) void radix_onesweep_plan_kernel(RadixPlan q, uint32_t n) {
-  __shared__ uint32_t s_trivial[P], s_most[P];
-  __shared__ uint32_t s_wsum[kRadixBins / kWave];
+  __shared__ uint32_t s_most[P], s_sum[kLows + 2];
+  __shared__ uint32_t s_wsum[P][kRadixBins / kWave];
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
-  if (t < (uint32_t)P) {
-    s_trivial[t] = s_most[t] = 0;
-    q.tile_counters[t] = 0;
+  if (t < (uint32_t)P) s_most[t] = 0;
+  if (t < q.launches) q.tile_counters[t] = 0;
+  if (P == 8 && q.sample) sum_samples(q.sample, s_sum);
+  uint32_t c[P], incl[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) c[p] = q.hist[p * kRadixBins + t];
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const uint32_t most = wave_reduce<uint32_t, OP_MAX>(c[p]);
+    if (lane == 0) atomicMax(&s_most[p], most);
+    incl[p] = wave_inclusive_scan<uint32_t, OP_ADD>(c[p]);
+    if (lane == 63) s_wsum[p][wid] = incl[p];
   }
   __syncthreads();
+#pragma unroll
   for (int p = 0; p < P; ++p) {
-    const uint32_t c = q.hist[p * kRadixBins + t];
-    if (c == n) s_trivial[p] = 1;
-    const uint32_t most = wave_reduce<uint32_t, OP_MAX>(c);
-    if (lane == 0) atomicMax(&s_most[p], most);
-    const uint32_t incl = wave_inclusive_scan<uint32_t, OP_ADD>(c);
-    if (lane == 63) s_wsum[wid] = incl;
-    __syncthreads();
     uint32_t woff = 0;
-    for (uint32_t k = 0; k < wid; ++k) woff += s_wsum[k];
-    q.gbase[p * kRadixBins + t] = woff + incl - c;
-    __syncthreads();
+    for (uint32_t k = 0; k < wid; ++k) woff += s_wsum[p][k];
+    q.gbase[p * kRadixBins + t] = woff + incl[p] - c[p];
   }
-  if (t != 0) return;
-  int active = 0, top = 0;
-  const int low = q.rep && !q.redo ? (int)q.rep->low : 0;
-  if (q.redo && q.rep->redo == 0) {
-    for (int p = 0; p < P; ++p) q.table[p].active = 0;
+  // The first P threads write an entry of the table each, the next P of the second.
+  if (t >= 2 * P) return;
+  uint32_t varying = 0, hot = n, low = 0;
+  for (int p = 0; p < P; ++p) {
+    varying |= (s_most[p] < n ? 1u : 0u) << p;
+    hot = min(hot, s_most[p]);
+  }
+  if (P == 8 && q.sample) {
+    low = min(choose_low(n, varying, hot > n / 64, s_sum), sampled_low(n, s_sum));
+    low = min(low, 8 - q.rep->near);
+    const int passes = __builtin_popcount(varying >> low);
+    if ((varying & ((1u << low) - 1)) == 0 || passes < 4 || passes > kFirstPasses) low = 0;
+    if (t == 0) q.rep->low = low;
+  } else if (t >= P) {
     return;
   }
-  for (int p = low; p < P; ++p) {
-    if (s_trivial[p]) continue;
-    ++active;
-    top = p;
-  }
-  const bool split = q.vofs != 0;
+  const bool split = q.vofs != 0, again = t >= P;
+  const int active = __builtin_popcount(varying >> low), top = 31 - __builtin_clz(varying | 1u);
   const bool use_local = q.local_max > 0 && active >= 3 && s_most[top] <= q.local_max;
-  q.local->on = use_local ? 1u : 0u;
-  q.local->top = (uint32_t)top;
-  q.local->pass = RadixPass{1u, 0u, split ? 0u : 1u, 0u,
-                            q.aos0, split ? (char*)q.aos0 + q.vofs : nullptr, q.out_k, q.out_v};
-  // All digits constant (all keys equal): one pass still moves the data.
-  const bool force_last = active == 0;
-  const int passes = use_local || force_last ? 1 : active;
-  int j = 0;
-  for (int p = 0; p < P; ++p) {
-    if (use_local ? p != top : (force_last ? p != P - 1 : p < low || s_trivial[p] != 0)) continue;
-    const bool to_out = j == passes - 1 && !use_local;
-    char* src = (char*)(((j - 1) & 1) ? q.aos1 : q.aos0);
-    char* dst = (char*)((j & 1) ? q.aos1 : q.aos0);
-    RadixPass rp;
-    rp.active = 1;
-    rp.shift = 8u * (uint32_t)p;
-    rp.in_aos = j > 0 && !split;
-    rp.out_aos = !to_out && !split;
-    rp.src_k = j == 0 ? q.in_k : src;
-    rp.src_v = j == 0 ? q.in_v : (split ? src + q.vofs : nullptr);
-    rp.dst_k = to_out ? q.out_k : dst;
-    rp.dst_v = to_out ? q.out_v : (split ? dst + q.vofs : nullptr);
-    q.table[j++] = rp;
+  if (t == 0) {
+    q.local->on = use_local ? 1u : 0u;
+    q.local->top = (uint32_t)top;
+    q.local->pass = RadixPass{1u, 0u, split ? 0u : 1u, 0u,
+                              q.aos0, split ? (char*)q.aos0 + q.vofs : nullptr, q.out_k, q.out_v};
   }
-  for (; j < P; ++j) q.table[j].active = 0;
+  uint32_t digits = again ? varying : (use_local ? 1u << top : (varying >> low << low));
+  if (digits == 0) digits = 1u << (P - 1);  // all keys equal: one pass still moves the data
+  const int passes = __builtin_popcount(digits), p = (int)(t % P);
+  RadixPass* table = q.table + (again ? P : 0);
+  if (p >= passes) table[p].active = 0;
+  if (!(digits >> p & 1u)) return;
+  const int j = __builtin_popcount(digits & ((1u << p) - 1));
+  const bool to_out = j == passes - 1 && !use_local;
+  char* src = (char*)(((j - 1) & 1) ? q.aos1 : q.aos0);
+  char* dst = (char*)((j & 1) ? q.aos1 : q.aos0);
+  RadixPass rp;
+  rp.active = 1;
+  rp.shift = 8u * (uint32_t)p;
+  rp.in_aos = j > 0 && !split;
+  rp.out_aos = !to_out && !split;
+  rp.src_k = j == 0 ? (again ? q.out_k : q.in_k) : src;
+  rp.src_v = j == 0 ? (again ? q.out_v : q.in_v) : (split ? src + q.vofs : nullptr);
+  rp.dst_k = to_out ? q.out_k : dst;
+  rp.dst_v = to_out ? q.out_v : (split ? dst + q.vofs : nullptr);
+  table[j] = rp;
 }
 
 // Whether a onesweep pass over EW-word elements reorders keys and values in
@@ -650,9 +797,9 @@ constexpr bool radix_split(int EW) { return EW >= 3; }
 //    tiles): 1.35.
 template <typename K, int MODE, int EW, int BLOCK, int IPT = kRadixIpt>
 __global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
-    const RadixPass* __restrict__ table, int pass, const uint32_t* __restrict__ gbase,
-    uint32_t* __restrict__ tile_counters, uint64_t* __restrict__ status, uint32_t gen,
-    uint32_t n) {
+    const RadixPass* __restrict__ table, int pass, int again, const RadixRepair* __restrict__ rep,
+    const uint32_t* __restrict__ gbase, uint32_t* __restrict__ tile_counter,
+    uint64_t* __restrict__ status, uint32_t gen, uint32_t n) {
   constexpr int NW = BLOCK / kWave;
   constexpr uint32_t TILE = (uint32_t)BLOCK * IPT;
   constexpr int KW = (int)sizeof(K) / 4, VW = EW - KW;
@@ -668,6 +815,9 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
   __shared__ uint32_t s_cnt[kRadixBins];          // the tile's digit counts (early)
   __shared__ uint32_t s_tile;
 
+  // After a repair (rep): pass `again` when it gave up, else `pass`, if any.
+  if (rep && rep->redo) pass = again;
+  if (pass < 0) return;
   const RadixPass rp = table[pass];
   if (!rp.active) return;
 
@@ -676,7 +826,7 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_onesweep_kernel(
   for (uint32_t i = tid; i < NW * kRadixBins / 2; i += BLOCK)
     reinterpret_cast<uint32_t*>(&s_hist[0][0])[i] = 0;
   if (digit_thread) s_cnt[tid] = 0;
-  if (tid == 0) s_tile = atomicAdd(tile_counters + pass, 1u);
+  if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
   __syncthreads();
   const uint32_t tile = s_tile;
   const size_t base = (size_t)tile * TILE + (size_t)wid * (kWave * IPT);
@@ -1058,92 +1208,140 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_local_kernel(
 //    their highest varying bits, so the passes stop at digit `low` and a repair
 //    orders what they left equal: a pass moves every element once (24 bytes of
 //    traffic for u64 + u32), the look of the repair reads 8 of them.
-//     * radix_sample_kernel (one block) chooses low: at least log2(n) + 4 bits
-//       of varying digits (then n / 32 pairs of random keys agree above it, half
-//       of them in the wrong order), one digit more when some key may hold over
-//       1/64 of the input (its run would be long to repair), and lower while
-//       two different keys of a sample of kSample agree above it.
+//     * radix_begin_kernel looks at some samples of kSample keys: for every
+//       digit, how many pairs of different keys share the digits from there on.
+//     * low: at least log2(n) + 4 bits of varying digits, one digit more when some
+//       key may hold over 1/64 of the input, and lower until the samples' pairs
+//       say that at most a quarter of the keys share these digits with another
+//       one (n / 16 runs to repair: 2^27 keys of 100 values to a digit have n / 3,
+//       which took 2.4 ms, more than two passes; 16 samples hold 2^29 pairs, so one
+//       may clash at 2^27).
+//       16 keys of a sample with the same digits that are not all equal are a long
+//       run, which counts as any number of pairs.
+//     * Keys that a sample has 4 times (a share of 2^-12 is found nearly always)
+//       are hot: their runs are too long to repair when any other key shares
+//       their digits, however rare. radix_hist_kernel compares every key with
+//       them, and low goes down to the highest digit that tells all apart.
 //     * radix_repair_find_kernel lists the runs of equal digits that have an
 //       element below its predecessor, radix_repair_kernel orders them.
-//     * When that is too much (many runs, or long ones: a run that holds a good
-//       part of the input and few keys that differ), the passes start over with
-//       every digit. Any input is sorted; the choice only decides how soon.
-//    2^27 u64 + u32, eight passes -> now: uniform 7.0 -> 4.42 ms (four passes),
-//    zipf with hot keys 7.2 -> 5.09 ms (five); the look 0.23 ms (4.7 TB/s; with
-//    64 consecutive bytes per thread 0.46), ordering the runs 5 us, the sample
-//    26 us, the passes left out 14 us each. 2^25 with half the keys equal and
-//    1e-5 of them off in the low digits, which starts over: 2.3 -> 3.5 ms.
-constexpr uint32_t kRepairMin = 1u << 21;   // keys: 2^21 + 1 uniform u64 + u32 214 -> 184 us, 2^23 522 -> 379
-constexpr uint32_t kRepairRun = 32;         // elements one thread orders
+//     * When that is too much (many long runs), the passes start over with every
+//       digit. Any input is sorted; the choice only decides how soon.
+//    2^27 u64 + u32, eight passes -> now: uniform 7.0 -> 4.50 ms (four passes),
+//    zipf with hot keys 7.2 -> 5.12 (five); the samples 34 us, the comparison with
+//    hot keys 50 us, the look 0.22 ms (4.7 TB/s; with 64 consecutive bytes per
+//    thread 0.46), ordering the runs 5 us, passes left out 14 us each. Digits of
+//    100 values 4.6, of 32 values 5.6, groups of two keys that differ in the lowest
+//    bytes 6.7 (10.2, 10.4 and 11.4 when digits counted 8 bits each and the passes
+//    then started over). 2^25 with half the keys equal and 1e-5 of them off in the
+//    low digits 2.3 (3.5 when only a sample looked).
+// Keys: 2^21 + 100000 uniform u64 + u32 223 -> 171 us. What the samples and the
+// launches that find nothing to do cost shows where few digits vary: two digits 81
+// -> 111 us there, 183 -> 219 at 8 million, 299 -> 344 at 16 million.
+constexpr uint32_t kRepairMin = 1u << 21;
+constexpr uint32_t kRepairRun = 32;         // Elements one thread orders,
 constexpr uint32_t kRepairLong = 1u << 15;  // elements of a run that a block orders,
 constexpr uint32_t kRepairSum = 1u << 16;   // and of all that one block does,
 constexpr uint32_t kRepairLongs = 64;       // and how many
-constexpr uint32_t kSample = 8192;
 
+// The first kLows blocks to a sample look at it: block b at sample b / kLows, from
+// digit b % kLows on (0: whole keys). The others zero words.
 template <typename K, int MODE>
-__global__ __launch_bounds__(1024) void radix_sample_kernel(const K* __restrict__ keys, uint32_t n,
-                                                            const uint32_t* __restrict__ hist,
-                                                            RadixRepair* __restrict__ rep) {
-  constexpr int P = (int)sizeof(K);
-  constexpr uint32_t SLOTS = 2 * kSample;
+__global__ __launch_bounds__(1024) void radix_begin_kernel(const K* __restrict__ keys, uint32_t n,
+                                                           RadixSample* __restrict__ sample,
+                                                           uint32_t* __restrict__ zero, uint32_t words) {
+  // A slot: the number of its first key, from 1; whether another one differs; how
+  // many more share its digits.
+  constexpr uint32_t kFirst = 0x3fffu, kDiffers = 0x8000u, kMore = 0x10000u;
+  constexpr uint32_t kLongRun = 16, kAny = 1u << 20;
   __shared__ uint64_t s_word[kSample];
-  __shared__ uint32_t s_slot[SLOTS];
-  __shared__ uint32_t s_most[P], s_clash;
+  __shared__ uint32_t s_slot[2 * kSample];
+  __shared__ uint32_t s_sum, s_most, s_heavy;
+  __shared__ unsigned long long s_xor;
+  constexpr int PER = (int)(kSample / 1024);  // most keys of a thread
+  constexpr uint32_t looks = kSamples * kLows;
   const uint32_t tid = threadIdx.x;
-  if (tid < (uint32_t)P) s_most[tid] = 0;
-  __syncthreads();
-  for (uint32_t i = tid; i < (uint32_t)P * kRadixBins; i += 1024) atomicMax(&s_most[i / kRadixBins], hist[i]);
-  // Positions spread by an odd multiplier.
-  for (uint32_t i = tid; i < kSample; i += 1024)
-    s_word[i] = (uint64_t)order_bits<K, MODE>(keys[(uint64_t)(i * 2654435761u) * n >> 32]);
-  __syncthreads();
-  uint32_t bits = 4, hot = n;
-  while ((1ull << (bits - 4)) < n) ++bits;
-  int want = (int)(bits + 7) / 8;
-  for (int p = 0; p < P; ++p) hot = min(hot, s_most[p]);
-  if (hot > n / 64) ++want;
-  int low = P;
-  for (int p = P; p-- > 0 && want > 0;) {
-    low = p;
-    want -= s_most[p] < n ? 1 : 0;
+  if (blockIdx.x >= looks) {
+    const uint32_t step = (gridDim.x - looks) * 1024u;
+    for (size_t i = (blockIdx.x - looks) * 1024u + tid; i < words; i += step) zero[i] = 0;
+    return;
   }
-  for (; low > 0; --low) {
-    if (s_most[low - 1] == n) continue;  // a constant digit needs no look
-    for (uint32_t i = tid; i < SLOTS; i += 1024) s_slot[i] = 0;
-    if (tid == 0) s_clash = 0;
-    __syncthreads();
-    for (uint32_t i = tid; i < kSample; i += 1024) {
-      const uint64_t prefix = s_word[i] >> (8 * low);
-      uint32_t h = (uint32_t)((prefix * 0x9E3779B97F4A7C15ull) >> 40) % SLOTS;
-      for (;;) {
-        const uint32_t other = atomicCAS(&s_slot[h], 0u, i + 1);
-        if (other == 0) break;
-        const uint64_t w = s_word[other - 1];
-        if (w >> (8 * low) == prefix) {
-          if (w != s_word[i]) s_clash = 1;
-          break;
-        }
-        h = (h + 1) % SLOTS;
+  const uint32_t low = blockIdx.x % kLows, sub = blockIdx.x / kLows;
+  const uint32_t size = sample_size(n), slots = 2 * size;
+  // Positions spread by an odd multiplier.
+  uint64_t word[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const uint32_t i = sub * size + j * 1024 + tid;
+    if (j * 1024u < size) word[j] = (uint64_t)order_bits<K, MODE>(keys[(uint64_t)(i * 2654435761u) * n >> 32]);
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (j * 1024u < size) s_word[j * 1024 + tid] = word[j];
+  for (uint32_t i = tid; i < slots; i += 1024) s_slot[i] = 0;
+  if (tid == 0) {
+    s_sum = s_most = s_heavy = 0;
+    s_xor = 0;
+  }
+  __syncthreads();
+  uint64_t x = 0;
+#pragma unroll 1
+  for (uint32_t j = 0; j < size / 1024; ++j) {
+    const uint32_t i = j * 1024 + tid;
+    const uint64_t mine = s_word[i], prefix = mine >> (8 * low);
+    x |= mine ^ s_word[0];
+    uint32_t h = (uint32_t)((prefix * 0x9E3779B97F4A7C15ull) >> 40) % slots;
+    for (;;) {
+      uint32_t other = s_slot[h];  // (a hot key: one read for all)
+      if (other == 0) other = atomicCAS(&s_slot[h], 0u, i + 1);
+      if (other == 0) break;
+      const uint64_t w = s_word[(other & kFirst) - 1];
+      if (w >> (8 * low) == prefix) {
+        const uint64_t same = ballot(true);  // the lanes that are here at once
+        if (ballot(h != (uint32_t)__builtin_amdgcn_readfirstlane((int)h)) != 0) atomicAdd(&s_slot[h], kMore);
+        else if (__builtin_ctzll(same) == (int)(tid & 63u)) atomicAdd(&s_slot[h], kMore * (uint32_t)__builtin_popcountll(same));
+        if (w != mine && !(other & kDiffers)) atomicOr(&s_slot[h], kDiffers);
+        break;
       }
+      h = (h + 1) % slots;
+    }
+  }
+#pragma unroll
+  for (int m = 1; m < kWave; m <<= 1) x |= __shfl_xor(x, m);
+  if (x && (tid & 63u) == 0) atomicOr(&s_xor, (unsigned long long)x);
+  __syncthreads();
+  if (low > 0) {
+    uint32_t pairs = 0;
+    for (uint32_t i = tid; i < slots; i += 1024) {
+      const uint32_t more = s_slot[i] / kMore;
+      if (s_slot[i] & kDiffers) pairs += more + 1 >= kLongRun ? kAny : more;
+    }
+    if (pairs) atomicAdd(&s_sum, min(pairs, kAny));
+    __syncthreads();
+    if (tid == 0) sample->clash[low][sub] = min(s_sum, kAny);
+    return;
+  }
+  // The hot keys, the most frequent ones first.
+  for (uint32_t least : {16u, 4u}) {
+    for (uint32_t i = tid; i < slots; i += 1024) {
+      const uint32_t count = s_slot[i] / kMore + 1;
+      if (count < least || (least == 4 && count >= 16)) continue;
+      atomicMax(&s_most, count);
+      const uint32_t k = atomicAdd(&s_sum, 1u);
+      if (k < kHots) sample->hot[sub][k] = s_word[(s_slot[i] & kFirst) - 1];
     }
     __syncthreads();
-    const bool clash = s_clash != 0;
+    if (least == 16 && tid == 0) s_heavy = s_sum;
     __syncthreads();
-    if (!clash) break;
   }
   if (tid == 0) {
-    bool below = false;
-    for (int p = 0; p < low; ++p) below = below || s_most[p] < n;
-    rep->low = below ? (uint32_t)low : 0u;
-    rep->redo = 0;
+    uint32_t varying = 0;
+    for (int p = 0; p < 8; ++p) varying |= (s_xor >> (8 * p) & 0xffu ? 1u : 0u) << p;
+    sample->clash[0][sub] = 0;
+    sample->varying[sub] = varying;
+    sample->most[sub] = s_most;
+    sample->hots[sub] = min(s_sum, kHots);
+    sample->heavy[sub] = s_heavy;
   }
-}
-
-// Zeroes the marks (a bit per element).
-static __global__ void radix_repair_clear_kernel(const RadixRepair* __restrict__ rep,
-                                                 uint32_t* __restrict__ marks, uint32_t words) {
-  if (rep->low == 0) return;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) marks[i] = 0;
 }
 
 // The end of the run of equal words >> shift that i is in (the first index
@@ -1277,10 +1475,6 @@ __global__ __launch_bounds__(1024) void radix_repair_kernel(K* keys, uint32_t* v
   if (low == 0) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid / 64u, shift = 8 * low;
   const uint32_t runs = counts[blockIdx.x];
-  if (runs > chunk / 8) {
-    if (tid == 0) rep->redo = 1;
-    return;
-  }
   list += (size_t)blockIdx.x * (chunk / 2 + 1);
   if (tid == 0) s_longs = s_sum = 0;
   __syncthreads();

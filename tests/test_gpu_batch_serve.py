@@ -147,13 +147,13 @@ def test_run_jobs_mixed_batch(exec_):
 @pytest.mark.parametrize("in_place", ["keys", "values", "both"])
 def test_run_jobs_long_sort_in_place(exec_, in_place):
     """A device-wide sort whose keys or values are written over its input, with
-    half the keys equal and a few of them off in the low digits (which the
-    sort's first passes leave out and then have to order after all)."""
+    150 runs of 34 keys beside each other that differ in their low digits only: too
+    many for one block of the repair after the first passes, which start over."""
     n = (1 << 23) + 11
     rng = np.random.default_rng(9)
     k = rng.integers(0, 2**62, n, dtype=np.uint64)
-    k[rng.random(n) < 0.5] = 5 << 40 | 7
-    k[np.flatnonzero(k == (5 << 40 | 7))[777::50_000]] -= np.uint64(1)
+    runs = (np.uint64(1 << 29) + np.arange(150, dtype=np.uint64).repeat(34)) << np.uint64(32)
+    k[rng.choice(n, runs.size, replace=False)] = runs | rng.integers(0, 2**32, runs.size, dtype=np.uint64)
     order = np.argsort(k, kind="stable")
     dk, dv = exec_.to_device(k), exec_.to_device(np.arange(n, dtype=np.uint32))
     ok = exec_.alloc(np.uint64, n) if in_place == "values" else dk

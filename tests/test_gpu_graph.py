@@ -86,6 +86,30 @@ def test_graph_replays_long_sort_of_wide_keys(exec_):
     cap.graph.close()
 
 
+def test_graph_replays_sort_that_starts_over(exec_):
+    """Between replays that need no repair, one whose repair gives up (many runs of 34
+    keys beside each other)."""
+    n = (1 << 23) + 11
+    rng = np.random.default_rng(9)
+    plain = rng.integers(0, 2**62, n, dtype=np.uint64)
+    runs = (np.uint64(1 << 29) + np.arange(150, dtype=np.uint64).repeat(34)) << np.uint64(32)
+    many = plain.copy()
+    many[rng.choice(n, runs.size, replace=False)] = runs | rng.integers(0, 2**32, runs.size, dtype=np.uint64)
+    k, v = exec_.alloc(np.uint64, n), exec_.to_device(np.arange(n, dtype=np.uint32))
+    exec_.sync()
+    with exec_.capture() as cap:
+        out, srt = m.vector.radix_sort_by_key(exec_, k, v, return_keys=True)
+    for rep, h in enumerate((plain, many, plain, many)):
+        m.vector.scatter(exec_, exec_.to_device(h), v, k)
+        exec_.sync()
+        cap.graph.launch()
+        exec_.sync()
+        order = np.argsort(h, kind="stable")
+        assert np.array_equal(exec_.to_host(out), order.astype(np.uint32)), rep
+        assert np.array_equal(exec_.to_host(srt), h[order]), rep
+    cap.graph.close()
+
+
 @pytest.mark.parametrize("beside", ["scans", "device-wide"])
 def test_graph_replays_forked_jobs(exec_, beside):
     """A captured batch whose long sort runs on the second stream, beside scans of

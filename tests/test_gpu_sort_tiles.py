@@ -94,10 +94,14 @@ def test_sort_few_values_in_high_digits(exec_, dtype, value, values):
 
 
 @pytest.mark.parametrize("dtype,value", [(np.uint64, np.uint32), (np.int64, None), (np.float64, np.uint64)])
-@pytest.mark.parametrize("spread", ["uniform", "sorted", "pairs", "runs", "half", "one digit"])
+@pytest.mark.parametrize("spread", ["uniform", "sorted", "pairs", "runs", "half", "one digit", "many runs",
+                                    "few values", "six digits", "seven digits"])
 def test_sort_high_digits_and_repair(exec_, dtype, value, spread):
     """Long sorts of 8-byte keys: nothing, pairs, runs of some hundred elements and a
-    run of half the keys that differ only in the digits the first passes leave out."""
+    run of half the keys that differ only in digits the first passes could leave
+    out; many runs of 34 beside each other, which the repair gives up on, so that
+    the passes start over; digits of ten values each; and seven digits or all of
+    them before the keys differ."""
     n = (1 << 23) + 4099
     rng = np.random.default_rng(41)
     few = rng.random(n) < (1e-4 if spread == "runs" else 1e-5)
@@ -112,6 +116,16 @@ def test_sort_high_digits_and_repair(exec_, dtype, value, spread):
         k = rng.integers(0, 2**62, n, dtype=np.uint64)
         hot = rng.random(n) < 0.5
         k[hot] = np.uint64(5 << 40) | np.where(few, low, np.uint64(7))[hot]
+    elif spread == "many runs":
+        k = rng.integers(0, 2**62, n, dtype=np.uint64)
+        runs = (np.uint64(1 << 29) + np.arange(150, dtype=np.uint64).repeat(34)) << np.uint64(32)
+        k[rng.choice(n, runs.size, replace=False)] = runs | rng.integers(0, 2**32, runs.size, dtype=np.uint64)
+    elif spread == "few values":
+        k = rng.integers(0, 10, (n, 8), dtype=np.uint8).view(np.uint64).reshape(-1)
+    elif spread == "six digits":  # groups of 512 keys that differ in the lowest two
+        k = rng.choice(rng.integers(0, 2**46, n >> 9, dtype=np.uint64), n) << np.uint64(16) | low
+    elif spread == "seven digits":  # groups of 16
+        k = rng.choice(rng.integers(0, 2**46, n >> 4, dtype=np.uint64), n) << np.uint64(16) | low
     elif spread == "one digit":
         k = rng.integers(0, 256, n, dtype=np.uint64) << np.uint64(48)
     else:
