@@ -93,8 +93,8 @@ def test_twelve_columns_one_pass(exec_):
     """12 columns of mixed widths (u32, i32, f32, u64, i64, f64), read through
     views that start one element in (unaligned rows), against numpy and the
     single-column calls: gather with out-of-range indices (0), scatter with
-    out-of-range indices (dropped) into small and into 2^24-element outputs
-    (the latter column by column in the binned form), copy_where /
+    out-of-range indices (dropped) into small and into 2^24-element outputs,
+    copy_where /
     remove_where and a predicate on a separate stencil column."""
     dts = [np.uint32, np.int32, np.float32, np.uint64, np.int64, np.float64] * 2
     for n in (5, 8193, 70001):
@@ -132,6 +132,25 @@ def test_twelve_columns_one_pass(exec_):
             keep = perm < olen  # destinations are distinct: check the written ones
             for o, c in zip(_host(exec_, outs), host[:3]):
                 assert o[perm[keep]].tobytes() == c[keep].tobytes(), (n, olen)
+
+
+def test_zipped_scatter_column_by_column(exec_):
+    """Outputs too large for the caches: every column takes the binned form by itself
+    (from 2^23 indices on), here from views that start one element in, with dropped
+    indices and places that no index names."""
+    n, size = (1 << 23) + 4099, (1 << 23) + 70_001
+    cols = [RNG.integers(0, 2**31, n + 1).astype(dt) for dt in (np.uint32, np.int64, np.float32, np.float64)]
+    idx = RNG.permutation(size)[:n].astype(np.uint32)
+    idx[::97] = size + 3
+    outs = tuple(exec_.to_device(np.full(size + 1, 7, c.dtype)) for c in cols)
+    di = exec_.to_device(np.concatenate([[0], idx]).astype(np.uint32)).slice(1, n + 1)
+    m.vector.scatter(exec_, tuple(d.slice(1, n + 1) for d in _dev(exec_, cols)), di,
+                     tuple(o.slice(1, size + 1) for o in outs))
+    keep = idx < size
+    for o, c in zip(_host(exec_, outs), cols):
+        want = np.full(size + 1, 7, c.dtype)
+        want[1:][idx[keep]] = c[1:][keep]
+        assert o.tobytes() == want.tobytes(), c.dtype
 
 
 def test_zipped_sort_and_merge_by_key(exec_):
