@@ -18,7 +18,11 @@
  * Threading: one executor owns one HIP stream; calls on one executor must be
  * externally serialised. Work is enqueued asynchronously; functions that
  * return a host value (msv_reduce, msv_to_host, msv_vec_len of a vector with
- * a device-resident length, segmentation constructors) synchronise.
+ * a device-resident length, segmentation constructors) wait for it: the work
+ * enqueued on the executor before the call has then finished and its results
+ * are visible to every stream and, in host memory, to the host. The kernel
+ * that hands over a reduce's value, a length or a count may still be ending,
+ * so hipStreamQuery on the executor's stream may say "not ready" for a moment.
  */
 #ifndef MSV_H
 #define MSV_H
@@ -226,7 +230,7 @@ msv_status msv_wrap_device(msv_executor* ex, msv_dtype dtype, void* device_ptr, 
 /* Shallow Clone (runtime.rs:275-285): shares the allocation. */
 msv_status msv_vec_retain(msv_vec* v);
 msv_status msv_vec_release(msv_vec* v);
-/* Logical length; synchronises only if the length is device-resident. */
+/* Logical length; waits for it only if the length is device-resident. */
 msv_status msv_vec_len(msv_executor* ex, msv_vec* v, uint32_t* out_len);
 uint32_t msv_vec_capacity(const msv_vec* v);
 int32_t msv_vec_dtype(const msv_vec* v);
@@ -255,7 +259,7 @@ msv_status msv_inclusive_scan_noalloc(msv_executor* ex, msv_slice input, msv_op 
 msv_status msv_exclusive_scan(msv_executor* ex, msv_slice input, const void* init, msv_op op,
                               msv_vec** out);
 /* vector::reduce (api/algorithm/reduce.rs:32-50): result = op(init, fold(x)),
- * written to the host element `out_host`. Synchronises. */
+ * written to the host element `out_host`. Waits for it (see Threading). */
 msv_status msv_reduce(msv_executor* ex, msv_slice input, const void* init, msv_op op,
                       void* out_host);
 
@@ -559,8 +563,11 @@ msv_status msv_unique_by_key(msv_executor* ex, msv_slice keys, msv_slice values,
  * device memory. Jobs small enough for one workgroup (scan / reduce /
  * copy_where up to 2^17 elements, sort_by_key up to 2^15) run as one
  * persistent launch per job family; larger jobs run with the device-wide
- * kernels. All work is enqueued on the executor's stream (no host sync). A
- * job's result does not depend on which other jobs share the call. */
+ * kernels. All work is enqueued on the executor's stream (no host sync), but
+ * for the longest one-workgroup sorts, which may run on a second stream beside
+ * the rest and which the executor's stream waits for before anything enqueued
+ * later. Jobs of one call must be independent of each other; a job's result
+ * does not depend on which other jobs share the call. */
 typedef enum msv_job_kind {
   MSV_JOB_INCLUSIVE_SCAN = 1, /* out[n] = inclusive_scan(in, op) */
   MSV_JOB_EXCLUSIVE_SCAN = 2, /* out[n] = exclusive_scan(in, init, op) */

@@ -9,8 +9,9 @@
 //  * gather: gather_look_kernel looks at some tiles, and the whole call goes
 //    directly or this way. gather_window_kernel walks the table window by window
 //    while it stays in one L2, and unbin_tiles_kernel undoes the sort through
-//    LDS with the 16-bit source positions the sort kept (2^28 u32: 0.58 + 2.07 +
-//    0.43 ms, from 5.56 directly; the L2s serve about 130 G random reads/s).
+//    LDS with the 16-bit source positions the sort kept (2^28 u32: 0.65 + 2.07 +
+//    0.43 ms and 0.03 for the look and the direct kernel, which ends at once; 5.56
+//    directly; the L2s serve about 130 G random reads/s).
 //  * scatter: an L2 takes random 4-byte stores at about the same rate and lets
 //    them go as partial lines, so it ends in LDS instead. bin_leaves_kernel
 //    takes a window's runs from a group of tiles (a chunk of at most kBinChunk
@@ -47,9 +48,11 @@ struct BinPlan {
 
 // What bin_leaves_kernel hands to leaf_scatter_kernel. Chunk c of window w has row
 // w * cap + c of leaf starts. Elements are placed as blocks come, in one of
-// kShards parts of the memory (one counter for all blocks cost 8 us when 512
-// blocks begin at once).
-constexpr uint32_t kShards = 8, kShardStep = 16;
+// kShards parts of the memory, a part to neighbouring windows (one counter for
+// all blocks cost 8 us when 512 blocks begin at once, and chunks of a window all
+// over the memory 5% of the collecting step); windows with more than their share
+// go on in other parts.
+constexpr uint32_t kShards = 64, kShardStep = 16;
 struct BinChunks {
   uint32_t* used;    // elements / 8 of each part, kShardStep words apart
   uint32_t* counts;  // chunks of each window
@@ -59,18 +62,23 @@ struct BinChunks {
 
 // Room for cnt elements (their first / 8), in two steps: the first only asks, so
 // that the answer can come while the block does other work. A part that has run
-// out leaves less than a chunk unused, which the parts' size allows for.
-__device__ inline uint32_t ask_room(const BinChunks& c, uint32_t cnt) {
-  return atomicAdd(&c.used[blockIdx.x % kShards * kShardStep], (cnt + 7) / 8);
+// out leaves less than a chunk unused, which the parts' size allows for, so one
+// of them has room. (A part that is seen to have none is not asked: its counter
+// stays far from 2^32.)
+__device__ inline uint32_t ask_room(const BinChunks& c, uint32_t part, uint32_t cnt) {
+  return atomicAdd(&c.used[part * kShardStep], (cnt + 7) / 8);
 }
-__device__ inline uint32_t take_room(const BinChunks& c, uint32_t cnt, uint32_t asked) {
+// `other`: where this block found room the last time that a window's own part had none.
+__device__ inline uint32_t take_room(const BinChunks& c, uint32_t part, uint32_t cnt, uint32_t asked,
+                                     uint32_t& other) {
   const uint32_t units = (cnt + 7) / 8;
-  uint32_t s = blockIdx.x % kShards;
   while (asked + units > c.shard) {
-    s = (s + 1) % kShards;
-    asked = atomicAdd(&c.used[s * kShardStep], units);
+    part = other;
+    asked = __hip_atomic_load(&c.used[part * kShardStep], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (asked + units <= c.shard) asked = ask_room(c, part, cnt);
+    if (asked + units > c.shard) other = (other * 13 + 11) % kShards;  // (goes through all of them)
   }
-  return s * c.shard + asked;
+  return part * c.shard + asked;
 }
 
 // Exclusive scan of s_cnt[0, kBinMost) into s_start, by the first kBinMost
@@ -527,8 +535,9 @@ __global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_
   const uint32_t tid = threadIdx.x;
   uint32_t* s_idx = reinterpret_cast<uint32_t*>(s_val);
   uint16_t* s_16 = reinterpret_cast<uint16_t*>(s_val);
+  uint32_t other = (kShards - 1 - blockIdx.x) % kShards;
   for (uint32_t q = blockIdx.x; q < p.windows * p.groups; q += gridDim.x) {
-    const uint32_t w = q % p.windows, g = q / p.windows;
+    const uint32_t w = q % p.windows, g = q / p.windows, part = w * kShards / p.windows;
     // The window's runs in the group's tiles: where each begins, and its place
     // among them.
     const uint32_t t0 = g * p.group, runs = min(p.group, p.tiles - t0);
@@ -555,7 +564,7 @@ __global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_
       uint32_t place = 0, asked = 0;
       if (tid == kBinBlock - 1) {
         place = atomicAdd(&chunks.counts[w], 1u);
-        asked = ask_room(chunks, cnt);
+        asked = ask_room(chunks, part, cnt);
       }
       uint32_t ix[kChunkIpt], at[kChunkIpt];
 #pragma unroll
@@ -577,7 +586,7 @@ __global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_
       }
       if (tid == kBinBlock - 1) {
         s_place = w * p.cap + place;
-        s_at = take_room(chunks, cnt, asked);
+        s_at = take_room(chunks, part, cnt, asked, other);
         chunks.at[s_place] = s_at;
       }
       __syncthreads();

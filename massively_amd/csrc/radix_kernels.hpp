@@ -1227,9 +1227,10 @@ __global__ __launch_bounds__(BLOCK, 8) void radix_local_kernel(
 //     * When that is too much (many long runs), the passes start over with every
 //       digit. Any input is sorted; the choice only decides how soon.
 //    2^27 u64 + u32, eight passes -> now: uniform 7.0 -> 4.50 ms (four passes),
-//    zipf with hot keys 7.2 -> 5.12 (five); the samples 34 us, the comparison with
-//    hot keys 50 us, the look 0.22 ms (4.7 TB/s; with 64 consecutive bytes per
-//    thread 0.46), ordering the runs 5 us, passes left out 14 us each. Digits of
+//    zipf with hot keys 7.2 -> 5.12 (five); the samples 34 us (uniform 47), the
+//    comparison with hot keys 50 us, the look 0.22 ms (4.7 TB/s; with 64 consecutive
+//    bytes per thread 0.46; uniform, with 2 million runs to list, 0.34), ordering the
+//    runs 5 us (uniform 0.27 ms), passes left out 14 us each. Digits of
 //    100 values 4.6, of 32 values 5.6, groups of two keys that differ in the lowest
 //    bytes 6.7 (10.2, 10.4 and 11.4 when digits counted 8 bits each and the passes
 //    then started over). 2^25 with half the keys equal and 1e-5 of them off in the
