@@ -17,7 +17,7 @@
 //    takes a window's runs from a group of tiles (a chunk of at most kBinChunk
 //    elements; more of them where the window has more) and sorts them by leaf
 //    (64 KiB of the table), chunk-local; leaf_scatter_kernel collects a leaf in
-//    LDS and writes whole lines (2^28 u32: 0.76 + 0.94 + 0.57 ms, from 6.0 with one look-back
+//    LDS and writes whole lines (2^28 u32: 0.76 + 0.93 + 0.52 ms, from 6.0 with one look-back
 //    partition into 256 windows and random stores from L2).
 // Each tile decides for itself as well: one whose indices stay near each other
 // (sorted, reversed, clustered, rows of elements) is gathered or scattered
@@ -521,7 +521,7 @@ __device__ inline void load_runs(const E* __restrict__ from, const uint32_t* s_s
 // windows of one group of tiles, so the runs they read are neighbours (a
 // window at a time over all tiles was 8% slower: 1 KiB pieces of 1 GiB).
 // 64 registers and 64 KiB of LDS: two blocks a CU (one: 1.12 ms at 2^28 u32, two
-// then 0.86, and 0.94 with the chunks' places asked for).
+// then 0.86, and 0.93 with the chunks' places asked for).
 template <typename T, uint32_t TILE>
 __global__ __launch_bounds__(kBinBlock, sizeof(T) == 4 ? 8 : 4) void bin_leaves_kernel(
     BinPlan p, const uint32_t* __restrict__ pidx, const T* __restrict__ pval,
