@@ -63,7 +63,7 @@ def test_graph_replays_scan_seg_sort_and_jobs(exec_):
 
 
 def test_graph_replays_long_sort_of_wide_keys(exec_):
-    """The digits that get a pass, and whether the passes start over, are chosen on every replay."""
+    """The digits that get a pass are chosen on every replay (starting over: below)."""
     n = (1 << 21) + 77
     k, v = exec_.alloc(np.uint64, n), exec_.to_device(np.arange(n, dtype=np.uint32))
     mr.uniform_u64(exec_, 0, 9, 1, k)
